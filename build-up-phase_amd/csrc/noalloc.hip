@@ -21,13 +21,14 @@ namespace rtx {
 
 namespace {
 
-// 48 MiB: a DeviceState and the stack spill of 262,144 lanes (4 blocks of 256 on 256 CUs) x 24 entries of 8 B,
-// i.e. TLAS + BLAS depth up to 16 BVH8 levels with 12 stack entries per lane in LDS.
+// 48 MiB: 256 bytes that every launch counts for its state and the stack spill of 262,144 lanes (4 blocks of 256 on
+// 256 CUs) x 24 entries of 8 B, i.e. TLAS + BLAS depth up to 16 BVH8 levels with 12 stack entries per lane in LDS.
 constexpr uint64_t kScratchBytes = 48ull << 20;
 constexpr uint64_t kStateBytes = 256;
-static_assert(sizeof(DeviceState) <= kStateBytes, "device state fits its slot");
 
-static __device__ __align__(256) uint8_t scratch[kScratchBytes];
+// the DeviceState (in its own slot, so that its size takes nothing from the spill), then the spill
+constexpr uint64_t kStateSlot = (sizeof(DeviceState) + 255) / 256 * 256;
+static __device__ __align__(256) uint8_t scratch[kStateSlot + kScratchBytes];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;
@@ -49,7 +50,7 @@ hipError_t noalloc_setup(int device, hipStream_t stream) {
     hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
     if (e != hipSuccess) return e;
     // the device state starts at zero (ray counter, error flags, statistics)
-    clear_state_kernel<<<1, 64, 0, stream>>>((uint32_t*)p, (uint32_t)(kStateBytes / 4));
+    clear_state_kernel<<<1, 64, 0, stream>>>((uint32_t*)p, (uint32_t)(kStateSlot / 4));
     if ((e = hipGetLastError()) || (e = hipStreamSynchronize(stream))) return e;
     g_ptr[device] = (uint8_t*)p;
     return hipSuccess;
@@ -72,7 +73,7 @@ hipError_t noalloc_trace(int device, TraceRequest q, const TraceLaunch& L, hipSt
     *need_bytes = need;
     if (need > kScratchBytes) return hipErrorOutOfMemory;
     q.state = (DeviceState*)base;
-    q.gstack = (uint2*)(base + kStateBytes);
+    q.gstack = (uint2*)(base + kStateSlot);
     return trace_rays_launch(q, L, stream);
 }
 

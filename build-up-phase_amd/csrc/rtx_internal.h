@@ -140,11 +140,18 @@ struct PathHit {
 };
 static_assert(sizeof(PathHit) == 48, "PathHit must be 48 B");
 
+// A queue of ray chunks: one counter on a 128-B line of its own.
+struct RayQueue {
+    uint32_t next;
+    uint32_t pad[31];
+};
+constexpr uint32_t kRayQueues = 32;
+
 // Context-owned device state.
 struct DeviceState {
-    uint32_t ray_counter;
+    RayQueue queue[kRayQueues];
     uint32_t error_flags;  // bit 0: stack overflow, bit 1: sort look-back timeout, bit 2: bad AS
-    uint32_t pad[2];
+    uint32_t pad[3];
     unsigned long long stat_nodes;
     unsigned long long stat_tris;
     unsigned long long stat_insts;

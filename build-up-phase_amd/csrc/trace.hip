@@ -3,7 +3,7 @@
 // Replaces the driver traversal behind traceRayEXT (call site main.cpp:1047-1052) and the raygen / miss /
 // closest-hit programs (main.cpp:1033-1091).
 //
-// Per lane (wave64; one persistent grid; a wave takes ray ids from an atomic counter in chunks and refills its
+// Per lane (wave64; one persistent grid; a wave takes ray ids from atomic counters in chunks and refills its
 // idle lanes once fewer than refill_lanes of 64 are busy, checked every refill_interval steps):
 //   * world ray (FP32) -> TLAS: nodes are tested with a conservative quantised slab test, instance leaves
 //     enter their BLAS;
@@ -23,6 +23,7 @@
 //     (result writes and their FP64 refinement run with many lanes instead of one or two); in the whole-path
 //     modes (training paths, pixel paths) finishing means shading the vertex and continuing the lane's path
 //     with its next ray, so one launch traces whole paths.
+#include <algorithm>
 #include <cmath>
 
 #include "pt_shade.h"
@@ -250,6 +251,8 @@ struct TraceArgs {
     uint32_t lds_depth;
     uint32_t gdepth;
     uint32_t ray_chunk;        // ray ids per queue fetch (< 64: automatic)
+    uint32_t guard;            // 1 / 2: the launch traces only if guard_passes
+    uint32_t first_chunks;     // 1: every wave's first chunk is its own, 0: all chunks come from the queues
     uint32_t refill_lanes;     // refill a wave once fewer lanes than this are busy
     uint32_t refill_interval;  // steps between refill checks
     uint32_t leaf_lanes;       // pending leaf groups needed before a leaf step runs
@@ -485,6 +488,20 @@ __device__ __forceinline__ bool candidate_accepted(const TraceArgs& args, uint32
     return any_hit_accepts(args, table + (cur_inst & kInstIdMask), geom, u, v);
 }
 
+// Ray ids per chunk of a launch of n rays on `waves` waves.  Automatic: at most one ray per lane is spread over all
+// waves (a wave of few rays diverges less, and the launch lasts as long as its slowest wave) where they all run at
+// once; otherwise 64, or for single rays 256 when every wave gets at least 8 chunks (neighbouring rays in one wave:
+// 16.7M camera rays 1.72 ms, 1.81 ms with 64; whole paths are too uneven for that: 4 samples of the 1080p Cornell
+// box 19.6 ms with 256, 18.8 ms with 64).
+__host__ __device__ __forceinline__ uint32_t rays_per_chunk(uint32_t configured, uint32_t n, uint32_t waves,
+                                                            uint32_t first_chunks, bool paths) {
+    if (configured >= 64u) return configured;
+    if (first_chunks && (uint64_t)n <= (uint64_t)waves * 64u) return n ? (n + waves - 1u) / waves : 1u;
+    return !paths && (uint64_t)n >= (uint64_t)waves * 64u * 8u ? 256u : 64u;
+}
+// Queues that a wave tries before it takes no more chunks.
+constexpr uint32_t kQueueHops = 3u;
+
 template <int MODE, bool STATS, bool FLAGS>
 __device__ __forceinline__ void trace_body(const TraceArgs& args) {
     const uint32_t ray_flags = FLAGS ? args.ray_flags : 0u;  // the default variant compiles the flags out
@@ -514,12 +531,13 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
     const bool cull_all = ((ray_flags & kRaySkipTriangles) && (ray_flags & kRaySkipAabbs)) ||
                           ((ray_flags & kRayCullOpaque) && (ray_flags & (kRayOpaque | kRayCullNoOpaque))) ||
                           ((ray_flags & kRayCullNoOpaque) && (ray_flags & kRayNoOpaque));
+    if (args.guard && !guard_passes(args.tlas, args.ray_flags, args.guard)) return;  // the other launch takes the rays
     const uint32_t nA = args.n_ptr ? *args.n_ptr : args.n;
     const uint32_t nrays = MODE == kModeFused ? nA + *args.n2_ptr : nA;
 
     uint64_t st_nodes = 0, st_tris = 0, st_insts = 0, st_rays = 0;
 
-    bool active = false, exhausted = false, finished = false;
+    bool active = false, finished = false;
     uint32_t ray_id = 0;
     float wo[3], wd[3], wtmin = 0.0f, tc = 0.0f;
     Space s;
@@ -587,13 +605,30 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
         tc = r.tmax;
     };
 
-    // Wave-uniform pool of ray ids [pool_next, pool_end): one atomic fetches `chunk` consecutive ids (256 when the
-    // launch has at least 8 rounds of work for every wave, else 64 so that small launches still spread over all
-    // waves).
-    const uint32_t waves_total = gridDim.x * (blockDim.x >> 6);
-    const uint32_t chunk = args.ray_chunk >= 64u ? args.ray_chunk
-                           : ((uint64_t)nrays >= (uint64_t)waves_total * 64u * 8u ? 256u : 64u);
+    // Wave-uniform pool of ray ids [pool_next, pool_end).  Chunk w of the launch is wave w's first pool (not where
+    // the grid's later blocks start only as another launch's blocks retire: first_chunks = 0); the chunks after those
+    // come from kRayQueues counters, each shared by the blocks of one residue: queue q's c-th chunk is one
+    // of the c-th group of nq chunks, at a place rotated by a hash of c (with a fixed place, a film whose rows hold a
+    // multiple of nq / 2 chunks gives every queue its own columns: 20% slower).  An atomic on one word shared by all waves costs 10-20 ns in turn, so one counter
+    // bounded short launches by its 4,096 waves' fetches alone: 777 rays 96 us, the 1200x800 reference film 224 us.
+    const uint32_t waves_block = blockDim.x >> 6;
+    const uint32_t waves_total = gridDim.x * waves_block;
+    const uint32_t wave =
+        (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * waves_block + (threadIdx.x >> 6)));
+    const uint32_t chunk = rays_per_chunk(args.ray_chunk, nrays, waves_total, args.first_chunks, kTrain);
+    const uint32_t nqueues = gridDim.x < kRayQueues ? gridDim.x : kRayQueues;
+    uint32_t queue = blockIdx.x % nqueues;
+    uint32_t hops = 0;  // queues this wave has found empty
+    const uint32_t own_chunks = args.first_chunks ? waves_total : 0u;
+    bool more = (uint64_t)chunk * own_chunks < nrays;
     uint32_t pool_next = 0, pool_end = 0;
+    if (own_chunks) {
+        const uint64_t first = (uint64_t)wave * chunk;
+        if (first < nrays) {
+            pool_next = (uint32_t)first;
+            pool_end = (uint32_t)(first + chunk < nrays ? first + chunk : nrays);
+        }
+    }
     for (;;) {
         if (kTrain && finished) {
             // continue the lane's path: gather a shadow ray's contribution, or shade the vertex the continuation
@@ -811,7 +846,7 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
             }
             finished = false;
         }
-        const uint64_t need = __ballot(!active && !exhausted);
+        const uint64_t need = more || pool_next < pool_end ? __ballot(!active) : 0ull;
         if (need) {
             const uint32_t want = (uint32_t)__popcll(need);
             const uint32_t rank = (uint32_t)__popcll(need & lt_mask);
@@ -819,16 +854,30 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
             const uint32_t served = avail < want ? avail : want;
             uint32_t id = rank < served ? pool_next + rank : 0xFFFFFFFFu;
             pool_next += served;
-            if (served < want && pool_end < nrays) {
-                uint32_t base = 0;
-                if (lane == 0) base = atomicAdd(&args.state->ray_counter, chunk);
-                base = __shfl(base, 0);
-                pool_next = base;
-                pool_end = base + chunk;
-                if (rank >= served) id = pool_next + (rank - served);
-                pool_next += want - served;
+            if (served < want && more) {
+                uint64_t base;
+                for (;;) {
+                    uint32_t c = 0;
+                    if (lane == 0) c = atomicAdd(&args.state->queue[queue].next, 1u);
+                    c = (uint32_t)__builtin_amdgcn_readfirstlane((int)c);
+                    const uint32_t place = (queue + ((c * 0x9E3779B1u) >> 16)) % nqueues;
+                    base = ((uint64_t)own_chunks + (uint64_t)c * nqueues + place) * chunk;
+                    if (base < nrays || ++hops >= kQueueHops) break;
+                    queue = queue + 1u < nqueues ? queue + 1u : 0u;
+                }
+                if (base < nrays) {
+                    const uint32_t left = nrays - (uint32_t)base;
+                    pool_next = (uint32_t)base;
+                    pool_end = pool_next + (left < chunk ? left : chunk);
+                    const uint32_t rest = want - served;
+                    const uint32_t take = pool_end - pool_next < rest ? pool_end - pool_next : rest;
+                    if (rank >= served && rank - served < take) id = pool_next + (rank - served);
+                    pool_next += take;
+                } else {
+                    more = false;
+                }
             }
-            if (!active && !exhausted) {
+            if (!active) {
                 if (id < nrays) {
                     ray_id = id;
                     active = true;
@@ -872,13 +921,11 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
                         tc = r1.w;
                     }
                     begin_ray();
-                } else {
-                    exhausted = true;
                 }
             }
         }
         if (!__any(active)) break;
-        const bool wave_exhausted = __any(exhausted);
+        const bool wave_exhausted = !more && pool_next >= pool_end;
         // kModeTrain: back to the refill point (where ended rays continue their paths) once a quarter of the lanes
         // that start this round (64 - refill_lanes of 64) have ended their rays, at least one
         uint32_t train_floor = 0;
@@ -1204,8 +1251,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void t
 }
 
 __global__ void reset_counter_kernel(DeviceState* st, int clear_stats) {
+    if (blockIdx.x == 0 && threadIdx.x < kRayQueues) st->queue[threadIdx.x].next = 0;
     if (threadIdx.x == 0 && blockIdx.x == 0) {
-        st->ray_counter = 0;
         if (clear_stats) {
             st->stat_nodes = 0;
             st->stat_tris = 0;
@@ -1249,15 +1296,6 @@ hipError_t launch(const TraceArgs& a, const TraceLaunch& L, uint32_t content, hi
 // every primitive as an opaque triangle.
 static_assert(kFlagsVariantRayFlags == kActiveRayFlags, "one set of ray flags selects the FLAGS variant");
 bool trace_needs_flags(uint32_t ray_flags, uint32_t content) { return needs_flags_variant(ray_flags, content); }
-
-namespace {
-// A guarded launch that the device does not choose takes no ray: its rays come from the ray counter, which is set
-// past every ray id (no wrap-around: fetches add at most a few chunks per wave).
-constexpr uint32_t kGuardSkip = 0xC0000000u;
-__global__ void guard_counter_kernel(const void* tlas, uint32_t ray_flags, uint32_t guard, DeviceState* st) {
-    if (threadIdx.x == 0 && blockIdx.x == 0 && !guard_passes(tlas, ray_flags, guard)) st->ray_counter = kGuardSkip;
-}
-}  // namespace
 
 hipError_t trace_rays_launch(const TraceRequest& r, const TraceLaunch& L, hipStream_t s) {
     TraceArgs a{};
@@ -1306,39 +1344,37 @@ hipError_t trace_rays_launch(const TraceRequest& r, const TraceLaunch& L, hipStr
         reset_counter_kernel<<<1, 64, 0, s>>>(r.state, r.stats ? 1 : 0);
         return hipGetLastError();
     }
-    if (r.guard == 3u && r.mode <= 2 && !(r.ray_flags & kActiveRayFlags)) {
-        // both variants, each guarded by the TLAS content the device reads: one of them takes every ray
+    // A host-known ray count: no more waves than rays, and no queue to clear where the first chunks cover the rays.
+    TraceLaunch G = L;
+    bool queues = true;
+    a.first_chunks = r.mode != 5;  // training paths run beside the pixel paths, on blocks that start one by one
+    if (!r.n_ptr && a.first_chunks) {
+        const uint32_t waves_block = L.block_size / 64u;
+        if (L.ray_chunk < 64u) G.grid = std::min(L.grid, (r.n - 1u) / waves_block + 1u);
+        const uint32_t waves = G.grid * waves_block;
+        queues = (uint64_t)rays_per_chunk(L.ray_chunk, r.n, waves, 1u, r.mode >= 5) * waves < r.n;
+    }
+    // guard 3: both variants, each guarded by the TLAS content the device reads, so that one of them takes the rays
+    const bool both = r.guard == 3u && r.mode <= 2 && !(r.ray_flags & kActiveRayFlags);
+    for (uint32_t g = 1; g <= (both ? 2u : 1u); ++g) {
+        const bool clear = r.stats && g == 1;
+        if (queues || clear) reset_counter_kernel<<<1, 64, 0, s>>>(r.state, clear ? 1 : 0);
+        a.guard = both ? g : (r.guard == 1u || r.guard == 2u ? r.guard : 0u);
+        const uint32_t c = !both ? r.content : (g == 1 ? 0u : (kContentAabb | kContentNonOpaque));
         hipError_t e;
-        for (uint32_t g = 1; g <= 2; ++g) {
-            reset_counter_kernel<<<1, 64, 0, s>>>(r.state, r.stats && g == 1 ? 1 : 0);
-            guard_counter_kernel<<<1, 64, 0, s>>>(r.tlas, r.ray_flags, g, r.state);
-            const uint32_t c = g == 1 ? 0u : (kContentAabb | kContentNonOpaque);
-            switch (r.mode) {
-                case 0:
-                    e = r.stats ? launch<kModeClosest, true>(a, L, c, s) : launch<kModeClosest, false>(a, L, c, s);
-                    break;
-                case 1: e = r.stats ? launch<kModeAny, true>(a, L, c, s) : launch<kModeAny, false>(a, L, c, s); break;
-                default:
-                    e = r.stats ? launch<kModeRaygen, true>(a, L, c, s) : launch<kModeRaygen, false>(a, L, c, s);
-            }
-            if (e) return e;
+        switch (r.mode) {
+            case 0: e = r.stats ? launch<kModeClosest, true>(a, G, c, s) : launch<kModeClosest, false>(a, G, c, s); break;
+            case 1: e = r.stats ? launch<kModeAny, true>(a, G, c, s) : launch<kModeAny, false>(a, G, c, s); break;
+            case 3: e = launch<kModePath, false>(a, G, c, s); break;
+            case 4: e = launch<kModeFused, false>(a, G, c, s); break;
+            case 5: e = launch_variant<kModeTrain, false, false>(a, G, s); break;
+            case 6: e = launch_variant<kModePixelPaths, false, false>(a, G, s); break;
+            case 7: e = launch_variant<kModePixelCache, false, false>(a, G, s); break;
+            default: e = r.stats ? launch<kModeRaygen, true>(a, G, c, s) : launch<kModeRaygen, false>(a, G, c, s);
         }
-        return hipSuccess;
+        if (e) return e;
     }
-    reset_counter_kernel<<<1, 64, 0, s>>>(r.state, r.stats ? 1 : 0);
-    if (r.guard == 1u || r.guard == 2u) guard_counter_kernel<<<1, 64, 0, s>>>(r.tlas, r.ray_flags, r.guard, r.state);
-    switch (r.mode) {
-        case 0:
-            return r.stats ? launch<kModeClosest, true>(a, L, r.content, s) : launch<kModeClosest, false>(a, L, r.content, s);
-        case 1: return r.stats ? launch<kModeAny, true>(a, L, r.content, s) : launch<kModeAny, false>(a, L, r.content, s);
-        case 3: return launch<kModePath, false>(a, L, r.content, s);
-        case 4: return launch<kModeFused, false>(a, L, r.content, s);
-        case 5: return launch_variant<kModeTrain, false, false>(a, L, s);
-        case 6: return launch_variant<kModePixelPaths, false, false>(a, L, s);
-        case 7: return launch_variant<kModePixelCache, false, false>(a, L, s);
-        default:
-            return r.stats ? launch<kModeRaygen, true>(a, L, r.content, s) : launch<kModeRaygen, false>(a, L, r.content, s);
-    }
+    return hipSuccess;
 }
 
 }  // namespace rtx

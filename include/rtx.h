@@ -409,8 +409,9 @@ typedef struct rtx_trace_config {
     uint32_t blocks_per_cu;   /* persistent blocks per compute unit (1..32) */
     uint32_t lds_stack_depth; /* stack entries held in LDS per lane before spilling to global memory; with the
                                  lane's world ray (24 B) at most 64 KiB of LDS per block: (8 depth + 24) block */
-    uint32_t ray_chunk;       /* ray ids a wave takes from the global queue per fetch: a multiple of 64 up to
-                                 4096, or RTX_TRACE_RAY_CHUNK_AUTO (64, or 256 when every wave gets >= 8 chunks) */
+    uint32_t ray_chunk;       /* ray ids a wave takes from a queue per fetch: a multiple of 64 up to
+                                 4096, or RTX_TRACE_RAY_CHUNK_AUTO (up to 64, or 256 for single
+                                 rays when every wave gets >= 8 chunks) */
     uint32_t refill_lanes;    /* a wave fetches new rays once fewer than this many of its 64 lanes are busy */
     uint32_t refill_interval; /* traversal steps between two refill checks (1..64) */
     uint32_t leaf_lanes;      /* postponed leaves: a wave runs its leaf step (BLAS entry, triangle tests) once this

@@ -8,7 +8,8 @@
 //   morton    30-bit (uint32) or 63-bit (uint64) Morton code of each box centroid
 //   sort      stable onesweep radix sort of (code, primitive index)                         [sort.hip]
 //   karras    binary radix tree over the sorted codes (Karras 2012), one thread per internal node
-//   refit     bottom-up boxes: the second thread to reach a node merges its children (atomic arrival count)
+//   refit     bottom-up boxes and treelet refinement: subtrees of up to kSubtree primitives a wave each in LDS, then the
+//             nodes above them, the second thread to reach a node merging its children (atomic arrival count)
 //   collapse  level-synchronous top-down conversion to 8-wide nodes: each node adopts up to 8 children by
 //             repeatedly opening the child with the largest surface area, places them by octant, quantises
 //             their boxes to 8 bits per plane and allocates their slots with one atomic add.
@@ -446,10 +447,12 @@ __device__ __forceinline__ int karras_delta(const K* keys, int64_t n, int64_t i,
     return __clz((uint32_t)(a ^ b));
 }
 
-// node_blas != nullptr (batched builds): the BLAS that owns all primitives of internal node i, or kMixedBlas.
+// cnt: primitives below each internal node.  node_blas != nullptr (batched builds): the BLAS that owns all primitives
+// of internal node i, or kMixedBlas.
 template <typename K>
 __global__ __launch_bounds__(256) void karras_kernel(const K* __restrict__ keys, uint32_t n, int32_t* __restrict__ left,
                                                      int32_t* __restrict__ right, int32_t* __restrict__ parent,
+                                                     uint32_t* __restrict__ cnt,
                                                      uint32_t* __restrict__ node_blas = nullptr) {
     int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (i == 0) parent[0] = -1;
@@ -476,6 +479,7 @@ __global__ __launch_bounds__(256) void karras_kernel(const K* __restrict__ keys,
     int32_t rc = (hi == gamma + 1) ? (int32_t)(-1 - (gamma + 1)) : (int32_t)(gamma + 1);
     left[i] = lc;
     right[i] = rc;
+    cnt[i] = (uint32_t)(hi - lo + 1);
     parent[lc >= 0 ? lc : (N - 1) + (-1 - lc)] = (int32_t)i;
     parent[rc >= 0 ? rc : (N - 1) + (-1 - rc)] = (int32_t)i;
     if (node_blas) {
@@ -532,9 +536,8 @@ __device__ __forceinline__ void store_coherent_i32(int32_t* p, int32_t v) { stor
 // (sum of internal-node surface areas, the only term a restructuring can change), the primitive count and the
 // height (leaves: cost 0, count 1, height 0).  The node cost is area + (cost(left) + cost(right)).
 //
-// The second thread to reach a node (atomic arrival count) merges its children.  When a node with at least
-// min_prims primitives is complete, the whole wave restructures the treelet below it (Karras & Aila 2013,
-// "Fast Parallel Construction of High-Quality Bounding Volume Hierarchies"):
+// When a node with at least min_prims primitives is complete, a whole wave restructures the treelet below it (Karras &
+// Aila 2013, "Fast Parallel Construction of High-Quality Bounding Volume Hierarchies"):
 //   formation  start from the node's two children and open the internal treelet leaf with the largest surface
 //              area (lowest slot on ties) until there are 7 leaves; the node and the 5 opened nodes are the
 //              treelet's 6 internal nodes
@@ -544,36 +547,235 @@ __device__ __forceinline__ void store_coherent_i32(int32_t* p, int32_t v) { stor
 //              keeps the depth bound the collapse relies on): breadth-first from S = all leaves, internal
 //              nodes reused in formation order.
 // A treelet covers only nodes of its root's finished subtree and is processed after that subtree is final, so
-// the result does not depend on the order in which waves finish.  Cross-wave hand-off uses agent-scope atomic
-// loads and stores (coherent across XCDs without L2 write-back fences): a wave waits for its stores to
-// complete (s_waitcnt) before it bumps a parent's arrival count.
+// the result does not depend on the order in which waves finish.
+//
+// A pass has two launches.  subtree_refine_kernel: a wave takes a maximal subtree of at most kSubtree primitives into
+// LDS and works through it level by level, deepest first.  refit_refine_kernel: the nodes above, a thread per subtree
+// climbing from its root; the second thread to reach a node (atomic arrival count) merges its children.  There the
+// cross-wave hand-off uses agent-scope atomic loads and stores (coherent across XCDs without L2 write-back fences): a
+// wave waits for its stores to complete (s_waitcnt) before it bumps a parent's arrival count.
 constexpr int kTreeletLeaves = 7;
-constexpr int kTreeletSubsets = 127;
+constexpr uint32_t kTreeletNodes = kTreeletLeaves - 1;
 
-// Subsets of the 7 treelet leaves ordered by size, then value (size k starts at entry 0, 7, 28, 63, 98, 119, 126
-// for k = 1..7).
-__constant__ uint8_t kSubsetsBySize[127] = {
-    1, 2, 4, 8, 16, 32, 64, 3, 5, 6, 9, 10, 12, 17, 18, 20, 24, 33, 34, 36, 40, 48, 65, 66, 68, 72, 80, 96, 7, 11,
-    13, 14, 19, 21, 22, 25, 26, 28, 35, 37, 38, 41, 42, 44, 49, 50, 52, 56, 67, 69, 70, 73, 74, 76, 81, 82, 84, 88,
-    97, 98, 100, 104, 112, 15, 23, 27, 29, 30, 39, 43, 45, 46, 51, 53, 54, 57, 58, 60, 71, 75, 77, 78, 83, 85, 86,
-    89, 90, 92, 99, 101, 102, 105, 106, 108, 113, 114, 116, 120, 31, 47, 55, 59, 61, 62, 79, 87, 91, 93, 94, 103,
-    107, 109, 110, 115, 117, 118, 121, 122, 124, 63, 95, 111, 119, 123, 125, 126, 127};
+// The DP's work of one wave, per lane.  A subset S of size K has 2^(K-1) - 1 splits {P, S\P} with P holding S's lowest
+// leaf; kSplitLanes[K] consecutive lanes share a subset (1 for K <= 4, 2 for K = 5, 8 for K = 6) and take its splits
+// in turn, in order of P.  split[t][lane]: the byte offsets of cost[P] (low half) and cost[S\P] (high half) of the
+// lane's split in step t, offsets of cost[0] (infinite) where it has none; steps of size K from kSplitStep[K].
+// subset[w][lane]: byte K - 2 of the two words: the subset whose result the lane writes (0: none).
+constexpr uint32_t kSplitLanes[7] = {0, 0, 1, 1, 1, 2, 8};
+constexpr uint32_t kSplitStep[8] = {0, 0, 0, 1, 4, 11, 19, 23};
+constexpr uint32_t kSplitSteps = 23;
+struct SplitTable {
+    uint32_t split[kSplitSteps][64];
+    uint32_t subset[2][64];
+};
+constexpr uint32_t bits7(uint32_t v) {
+    uint32_t c = 0;
+    for (; v; v &= v - 1u) ++c;
+    return c;
+}
+constexpr SplitTable make_split_table() {
+    SplitTable T{};
+    for (uint32_t K = 2; K <= 6; ++K) {
+        uint32_t sub = 0;
+        for (uint32_t S = 1; S < 128; ++S) {
+            if (bits7(S) != K) continue;
+            const uint32_t low = S & (0u - S), rest = S ^ low;
+            const uint32_t first = sub * kSplitLanes[K];
+            T.subset[(K - 2) / 4][first] |= S << (8 * ((K - 2) & 3));
+            uint32_t q = 0;  // the proper subsets of rest in increasing order
+            for (uint32_t i = 0; i < (1u << (K - 1)) - 1u; ++i) {
+                const uint32_t P = low | q;
+                T.split[kSplitStep[K] + i / kSplitLanes[K]][first + i % kSplitLanes[K]] = (4u * P) | (4u * (S ^ P)) << 16;
+                q = (q - rest) & rest;
+            }
+            ++sub;
+        }
+    }
+    return T;
+}
+__constant__ SplitTable kSplitTable = make_split_table();
 
+// A lane's part of the table, loaded once per wave.
+struct SplitRegs {
+    uint32_t split[kSplitSteps];
+    uint32_t subset[2];
+};
+__device__ __forceinline__ void load_splits(SplitRegs& r) {
+    const uint32_t lane = threadIdx.x;
+#pragma unroll
+    for (uint32_t t = 0; t < kSplitSteps; ++t) r.split[t] = kSplitTable.split[t][lane];
+    r.subset[0] = kSplitTable.subset[0][lane];
+    r.subset[1] = kSplitTable.subset[1][lane];
+}
+
+// One treelet in LDS: its leaves and internal nodes (codes of the caller), the leaves' boxes and values, the DP.
 struct TreeletLds {
-    float area[128];
-    float cost[128];
-    uint32_t part[128];
-    float box[kTreeletLeaves][6];
-    float lcost[kTreeletLeaves];
+    float cost[128];  // of every subset; its surface area until the DP reaches it
+    uint8_t part[128];
+    float box[kTreeletLeaves + 1][6];
     uint32_t lcnt[kTreeletLeaves], lhgt[kTreeletLeaves];
     int32_t leaf[kTreeletLeaves];
-    int32_t pool[kTreeletLeaves - 1];
-    // rebuild list: subset, node, child codes, child list index (-1: treelet leaf), height
-    uint32_t ls[kTreeletLeaves - 1];
-    int32_t lx[kTreeletLeaves - 1], lc[kTreeletLeaves - 1][2], li[kTreeletLeaves - 1][2];
-    uint32_t lh[kTreeletLeaves - 1];
-    uint32_t commit;
+    int32_t pool[kTreeletNodes];
 };
+
+// The restructured treelet (wave-uniform): node i (0 = the root, breadth-first) covers leaf subset (sets >> 8 i) & 255,
+// its children are 4-bit codes in byte i of kids (child 0 low): node index, or 8 + leaf; heights in bytes.
+struct TreeletPlan {
+    uint64_t sets, kids, heights;
+    float total;
+    bool commit;
+};
+
+// DP steps of subset size K.
+template <uint32_t K>
+__device__ __forceinline__ void treelet_dp_size(TreeletLds& T, const SplitRegs& r) {
+    constexpr uint32_t G = kSplitLanes[K];
+    const uint8_t* const cost = (const uint8_t*)T.cost;
+    float best = INFINITY;
+    uint32_t bp = 0;  // offset of the best P; no finite split: 0
+#pragma unroll
+    for (uint32_t t = kSplitStep[K]; t < kSplitStep[K + 1]; ++t) {
+        const uint32_t p = r.split[t] & 0xFFFFu;
+        const float c = *(const float*)(cost + p) + *(const float*)(cost + (r.split[t] >> 16));
+        if (c < best) {
+            best = c;
+            bp = p;
+        }
+    }
+#pragma unroll
+    for (uint32_t off = G / 2; off > 0; off >>= 1) {
+        const float oc = __shfl_xor(best, (int)off);
+        const uint32_t op = (uint32_t)__shfl_xor((int)bp, (int)off);
+        if (oc < best || (oc == best && op < bp)) {
+            best = oc;
+            bp = op;
+        }
+    }
+    const uint32_t S = (r.subset[(K - 2) / 4] >> (8 * ((K - 2) & 3))) & 255u;
+    if (S) {
+        T.cost[S] = T.cost[S] + best;
+        T.part[S] = (uint8_t)(bp >> 2);
+    }
+    __syncthreads();
+}
+
+// Whole-wave solution of the treelet staged in T (boxes, counts, heights, and cost[1 << j] of its leaves).
+__device__ __forceinline__ TreeletPlan treelet_solve(TreeletLds& T, const SplitRegs& r, float old_cost, uint32_t old_h) {
+    const uint32_t lane = threadIdx.x;
+    TreeletPlan plan;
+    plan.sets = plan.kids = plan.heights = 0;
+    plan.total = old_cost;
+    plan.commit = false;
+    // surface areas: lane S for subset S of leaves 0..5, then with leaf 6 for subset 64 + S
+    {
+        float b[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+        for (int j = 0; j < kTreeletLeaves - 1; ++j)
+            if (lane & (1u << j)) {
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    b[a] = fminf(b[a], T.box[j][a]);
+                    b[3 + a] = fmaxf(b[3 + a], T.box[j][3 + a]);
+                }
+            }
+        const float a0 = box_area(b);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            b[a] = fminf(b[a], T.box[kTreeletLeaves - 1][a]);
+            b[3 + a] = fmaxf(b[3 + a], T.box[kTreeletLeaves - 1][3 + a]);
+        }
+        const float a1 = box_area(b);
+        if (lane & (lane - 1u)) T.cost[lane] = a0;
+        if (lane) T.cost[64u + lane] = a1;
+        if (lane == 0) T.cost[0] = INFINITY;
+    }
+    __syncthreads();
+    treelet_dp_size<2>(T, r);
+    treelet_dp_size<3>(T, r);
+    treelet_dp_size<4>(T, r);
+    treelet_dp_size<5>(T, r);
+    treelet_dp_size<6>(T, r);
+    // all 7 leaves: the 63 splits containing leaf 0, one per lane; the lowest lane with the least cost has the smallest P
+    const uint32_t p7 = 1u | (lane << 1);
+    const float c7 = lane < 63u ? T.cost[p7] + T.cost[127u ^ p7] : INFINITY;
+    float m = c7;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) m = fminf(m, __shfl_xor(m, off));
+    const uint64_t at = __ballot(c7 == m && lane < 63u);
+    const float total = T.cost[127] + m;
+    if (!(total < old_cost) || !at) return plan;
+    const uint32_t P7 = 1u | ((uint32_t)__ffsll((unsigned long long)at) - 1u) << 1;
+    // rebuild, breadth-first, on wave-uniform values
+    uint64_t sets = 127u, kids = 0;
+    uint32_t nodes = 1;
+#pragma unroll
+    for (uint32_t i = 0; i < kTreeletNodes; ++i) {
+        const uint32_t S = (uint32_t)(sets >> (8 * i)) & 127u;
+        const uint32_t P =
+            i == 0 ? P7 : (uint32_t)__builtin_amdgcn_readfirstlane((int)T.part[S]);
+        if (i >= nodes || P == 0u || (P & S) != P || P == S) return plan;  // no finite split was found
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t C = h ? S ^ P : P;
+            uint32_t code;
+            if ((C & (C - 1u)) == 0u) {
+                code = 8u + (uint32_t)__ffs((int)C) - 1u;
+            } else {
+                code = nodes;
+                sets |= (uint64_t)C << (8 * nodes);
+                ++nodes;
+            }
+            kids |= (uint64_t)code << (8 * i + 4 * h);
+        }
+    }
+    uint64_t lh = 0, heights = 0;
+#pragma unroll
+    for (int j = 0; j < kTreeletLeaves; ++j)
+        lh |= (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)T.lhgt[j]) << (8 * j);
+#pragma unroll
+    for (int i = (int)kTreeletNodes - 1; i >= 0; --i) {
+        uint32_t hc[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t code = (uint32_t)(kids >> (8 * i + 4 * h)) & 15u;
+            hc[h] = (uint32_t)((code & 8u ? lh : heights) >> (8 * (code & 7u))) & 255u;
+        }
+        heights |= (uint64_t)(1u + (hc[0] > hc[1] ? hc[0] : hc[1])) << (8 * i);
+    }
+    plan.sets = sets;
+    plan.kids = kids;
+    plan.heights = heights;
+    plan.commit = (heights & 255u) <= old_h;
+    if (plan.commit) plan.total = total;
+    return plan;
+}
+
+__device__ __forceinline__ int32_t plan_child(const TreeletLds& T, const TreeletPlan& plan, uint32_t i, int h) {
+    const uint32_t code = (uint32_t)(plan.kids >> (8 * i + 4 * h)) & 15u;
+    return code & 8u ? T.leaf[code & 7u] : T.pool[code];
+}
+
+// Box and primitive count of plan node i.
+__device__ __forceinline__ uint32_t plan_bounds(const TreeletLds& T, uint32_t S, float* b) {
+    uint32_t np = 0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        b[k] = INFINITY;
+        b[3 + k] = -INFINITY;
+    }
+#pragma unroll
+    for (int j = 0; j < kTreeletLeaves; ++j)
+        if (S & (1u << j)) {
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                b[a] = fminf(b[a], T.box[j][a]);
+                b[3 + a] = fmaxf(b[3 + a], T.box[j][3 + a]);
+            }
+            np += T.lcnt[j];
+        }
+    return np;
+}
 
 __device__ __forceinline__ uint64_t node_index(uint32_t n, int32_t c) {
     return c >= 0 ? (uint64_t)c : (uint64_t)n - 1 + (uint64_t)(-1 - c);
@@ -587,44 +789,38 @@ __device__ __forceinline__ float coherent_area(const float* nboxes, uint64_t i) 
 }
 
 // Treelet formation for root R, by one lane: open the largest-area internal treelet leaf until there are 7
-// leaves.  Writes the leaves and the 6 internal nodes (R first, in opening order) to the lane's staging row;
-// false when fewer than 7 primitives lie below R (nothing to restructure).  The lanes of a wave form their
-// treelets at the same time: their roots were completed in the same step of the climb, so none is an ancestor
-// of another and their subtrees - everything a formation reads and a restructuring writes - are disjoint.
+// leaves; false when fewer than 7 primitives lie below R (nothing to restructure).  The lanes of a wave form their
+// treelets at the same time: their roots were completed in the same step, so none is an ancestor of another and their
+// subtrees - everything a formation reads and a restructuring writes - are disjoint.  children(c, l, r, al, ar): node
+// c's children and their areas (-1 for leaves, which have negative codes).
 struct TreeletForm {
     int32_t leaf[kTreeletLeaves];
-    int32_t pool[kTreeletLeaves - 1];
+    int32_t pool[kTreeletNodes];
 };
 
-__device__ bool treelet_form(int32_t R, const int32_t* left, const int32_t* right, const float* nboxes,
-                             TreeletForm& out) {
+template <typename Children>
+__device__ __forceinline__ bool treelet_form(int32_t R, Children children, TreeletForm& out) {
     int32_t lf[kTreeletLeaves];
     float la[kTreeletLeaves];
-    int32_t pool[kTreeletLeaves - 1];
-    lf[0] = load_coherent_i32(left + R);
-    lf[1] = load_coherent_i32(right + R);
-    la[0] = lf[0] >= 0 ? coherent_area(nboxes, (uint64_t)lf[0]) : 0.0f;
-    la[1] = lf[1] >= 0 ? coherent_area(nboxes, (uint64_t)lf[1]) : 0.0f;
-    pool[0] = R;
+    out.pool[0] = R;
+    children(R, lf[0], lf[1], la[0], la[1]);
 #pragma unroll
     for (int k = 2; k < kTreeletLeaves; ++k) {
         int best = -1;
         float ba = -1.0f;
-#pragma unroll
-        for (int j = 0; j < k; ++j)
-            if (lf[j] >= 0 && la[j] > ba) {
-                ba = la[j];
-                best = j;
-            }
-        if (best < 0) return false;
         int32_t c = 0;
 #pragma unroll
         for (int j = 0; j < k; ++j)
-            if (j == best) c = lf[j];
-        pool[k - 1] = c;
-        const int32_t l = load_coherent_i32(left + c), r = load_coherent_i32(right + c);
-        const float al = l >= 0 ? coherent_area(nboxes, (uint64_t)l) : 0.0f;
-        const float ar = r >= 0 ? coherent_area(nboxes, (uint64_t)r) : 0.0f;
+            if (la[j] > ba) {
+                ba = la[j];
+                best = j;
+                c = lf[j];
+            }
+        if (best < 0) return false;
+        out.pool[k - 1] = c;
+        int32_t l, r;
+        float al, ar;
+        children(c, l, r, al, ar);
 #pragma unroll
         for (int j = 0; j < k; ++j)
             if (j == best) {
@@ -636,208 +832,317 @@ __device__ bool treelet_form(int32_t R, const int32_t* left, const int32_t* righ
     }
 #pragma unroll
     for (int j = 0; j < kTreeletLeaves; ++j) out.leaf[j] = lf[j];
-#pragma unroll
-    for (int j = 0; j < kTreeletLeaves - 1; ++j) out.pool[j] = pool[j];
     return true;
 }
 
-// DP step for the treelet-leaf subsets of size K.  A subset S's splits {P, S\P} with P containing S's lowest
-// leaf are P = low | Q for the proper subsets Q of S\low (2^(K-1) - 1 of them).  G consecutive lanes (G a power
-// of two, G x C(7, K) <= 64) share a subset, lane r taking the Q of index r, r + G, ... (the index's bits placed
-// on S\low's leaves); the group then takes the minimum (cost, P), with (inf, 0) while no finite split was seen -
-// the same result as one lane scanning every split, whatever the order.
-template <int K, int G>
-__device__ __forceinline__ void treelet_dp_size(TreeletLds& T, uint32_t lane) {
-    constexpr uint32_t kOffset[kTreeletLeaves] = {0, 0, 7, 28, 63, 98, 119};
-    constexpr uint32_t kCount[kTreeletLeaves] = {0, 7, 21, 35, 35, 21, 7};
-    constexpr uint32_t kSplits = (1u << (K - 1)) - 1u;
-    constexpr uint32_t kPerLane = (kSplits + G - 1) / G;
-    static_assert((G & (G - 1)) == 0 && G * kCount[K] <= 64u, "one wave per subset size");
-    const uint32_t sub = lane / G, r = lane % G;
-    uint32_t S = 0;
-    float best = INFINITY;
-    uint32_t bp = 0;
-    if (sub < kCount[K]) {
-        S = kSubsetsBySize[kOffset[K] + sub];
-        const uint32_t low = S & (0u - S), rest = S ^ low;
+__device__ __forceinline__ void stage_form(TreeletLds& T, const TreeletForm& f) {
 #pragma unroll
-        for (uint32_t t = 0; t < kPerLane; ++t) {
-            const uint32_t i = r + t * G;
-            if (i < kSplits) {
-                uint32_t q = 0, m = rest;
+    for (int j = 0; j < kTreeletLeaves; ++j) T.leaf[j] = f.leaf[j];
 #pragma unroll
-                for (int b = 0; b < K - 1; ++b) {
-                    const uint32_t bit = m & (0u - m);
-                    if (i & (1u << b)) q |= bit;
-                    m ^= bit;
-                }
-                const uint32_t P = low | q;
-                const float c = T.cost[P] + T.cost[S ^ P];
-                if (c < best || (c == best && P < bp)) {
-                    best = c;
-                    bp = P;
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int off = G / 2; off > 0; off >>= 1) {
-        const float oc = __shfl_xor(best, off);
-        const uint32_t op = (uint32_t)__shfl_xor((int)bp, off);
-        if (oc < best || (oc == best && op < bp)) {
-            best = oc;
-            bp = op;
-        }
-    }
-    if (sub < kCount[K] && r == 0) {
-        T.cost[S] = T.area[S] + best;
-        T.part[S] = bp;
-    }
-    __syncthreads();
+    for (uint32_t j = 0; j < kTreeletNodes; ++j) T.pool[j] = f.pool[j];
 }
 
 // Whole-wave treelet restructuring below internal node R (uniform arguments) from its formation, which lane
-// `owner` holds in `f` (formed = true).  Returns R's cost and height afterwards through new_cost / new_h.
-__device__ void treelet_optimize(TreeletLds& T, uint32_t n, int32_t R, float old_cost, uint32_t old_h,
-                                 uint32_t owner, bool formed, const TreeletForm& f, int32_t* left, int32_t* right,
-                                 int32_t* parent, float* nboxes, float* cost, uint32_t* cnt, uint32_t* hgt,
-                                 float& new_cost, uint32_t& new_h) {
+// `owner` holds in `f`, in global memory.  Returns R's cost and height afterwards through new_cost / new_h.
+__device__ __forceinline__ void treelet_optimize(TreeletLds& T, const SplitRegs& sr, uint32_t n, float old_cost,
+                                                 uint32_t old_h, uint32_t owner, const TreeletForm& f, int32_t* left,
+                                                 int32_t* right, int32_t* parent, float* nboxes, float* cost,
+                                                 uint32_t* cnt, uint32_t* hgt, float& new_cost, uint32_t& new_h) {
     const uint32_t lane = threadIdx.x;
     __syncthreads();
-    if (!formed) {  // fewer than 7 primitives below R: nothing to restructure
-        new_cost = old_cost;
-        new_h = old_h;
-        return;
-    }
-    if (lane == owner) {
-#pragma unroll
-        for (int j = 0; j < kTreeletLeaves; ++j) T.leaf[j] = f.leaf[j];
-#pragma unroll
-        for (int j = 0; j < kTreeletLeaves - 1; ++j) T.pool[j] = f.pool[j];
-    }
+    if (lane == owner) stage_form(T, f);
     __syncthreads();
     if (lane < (uint32_t)kTreeletLeaves) {
         const int32_t c = T.leaf[lane];
         const uint64_t bi = node_index(n, c);
 #pragma unroll
         for (int k = 0; k < 6; ++k) T.box[lane][k] = load_coherent(nboxes + 6 * bi + k);
-        T.lcost[lane] = c >= 0 ? load_coherent(cost + c) : 0.0f;
+        T.cost[1u << lane] = c >= 0 ? load_coherent(cost + c) : 0.0f;
         T.lcnt[lane] = c >= 0 ? load_coherent_u32(cnt + c) : 1u;
         T.lhgt[lane] = c >= 0 ? load_coherent_u32(hgt + c) : 0u;
     }
     __syncthreads();
-    // surface area of every subset's union box; singleton costs
-    for (uint32_t S = lane + 1; S <= (uint32_t)kTreeletSubsets; S += 64) {
-        float b[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-#pragma unroll
-        for (int j = 0; j < kTreeletLeaves; ++j)
-            if (S & (1u << j)) {
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    b[a] = fminf(b[a], T.box[j][a]);
-                    b[3 + a] = fmaxf(b[3 + a], T.box[j][3 + a]);
-                }
-            }
-        T.area[S] = box_area(b);
-        if (__popc(S) == 1) {
-            T.cost[S] = T.lcost[__ffs(S) - 1];
-            T.part[S] = 0;
-        }
-    }
-    __syncthreads();
-    // subsets of size 2..6, each size after the smaller ones
-    treelet_dp_size<2, 1>(T, lane);
-    treelet_dp_size<3, 1>(T, lane);
-    treelet_dp_size<4, 1>(T, lane);
-    treelet_dp_size<5, 2>(T, lane);
-    treelet_dp_size<6, 8>(T, lane);
-    // all 7 leaves: the 63 splits containing leaf 0, one per lane, then a (cost, split) minimum over the wave
-    float c7 = INFINITY;
-    uint32_t p7 = 0xFFFFFFFFu;
-    if (lane < 63u) {
-        p7 = 1u | (lane << 1);
-        c7 = T.cost[p7] + T.cost[127u ^ p7];
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const float oc = __shfl_xor(c7, off);
-        const uint32_t op = (uint32_t)__shfl_xor((int)p7, off);
-        if (oc < c7 || (oc == c7 && op < p7)) {
-            c7 = oc;
-            p7 = op;
-        }
-    }
-    const float total = T.area[127] + c7;
+    const TreeletPlan plan = treelet_solve(T, sr, old_cost, old_h);
     new_cost = old_cost;
     new_h = old_h;
-    if (!(total < old_cost)) return;
-    if (lane == 0) {
-        T.part[127] = p7;
-        T.ls[0] = 127u;
-        T.lx[0] = R;
-        uint32_t cntl = 1, next = 1;
-        bool ok = true;
-        for (uint32_t i = 0; i < cntl && ok; ++i) {
-            const uint32_t S = T.ls[i];
-            const uint32_t P = T.part[S];
-            const uint32_t C[2] = {P, S ^ P};
-            if (P == 0u || (P & S) != P || P == S) {  // no finite split was found
-                ok = false;
-                break;
-            }
-            for (int h = 0; h < 2; ++h) {
-                if (__popc(C[h]) == 1) {
-                    T.lc[i][h] = T.leaf[__ffs(C[h]) - 1];
-                    T.li[i][h] = -1 - (__ffs(C[h]) - 1);
-                } else {
-                    const int32_t x = T.pool[next++];
-                    T.ls[cntl] = C[h];
-                    T.lx[cntl] = x;
-                    T.lc[i][h] = x;
-                    T.li[i][h] = (int32_t)cntl;
-                    ++cntl;
-                }
-            }
-        }
-        for (int i = kTreeletLeaves - 2; ok && i >= 0; --i) {
-            uint32_t hc[2];
-            for (int h = 0; h < 2; ++h) {
-                const int32_t q = T.li[i][h];
-                hc[h] = q >= 0 ? T.lh[q] : T.lhgt[-1 - q];
-            }
-            T.lh[i] = 1u + (hc[0] > hc[1] ? hc[0] : hc[1]);
-        }
-        T.commit = ok && T.lh[0] <= old_h ? 1u : 0u;
-    }
-    __syncthreads();
-    if (!T.commit) return;
-    if (lane < (uint32_t)(kTreeletLeaves - 1)) {
-        const int32_t x = T.lx[lane];
-        const uint32_t S = T.ls[lane];
-        store_coherent_i32(left + x, T.lc[lane][0]);
-        store_coherent_i32(right + x, T.lc[lane][1]);
-        store_coherent_i32(parent + node_index(n, T.lc[lane][0]), x);
-        store_coherent_i32(parent + node_index(n, T.lc[lane][1]), x);
+    if (!plan.commit) return;
+    if (lane < kTreeletNodes) {
+        const int32_t x = T.pool[lane];
+        const int32_t c0 = plan_child(T, plan, lane, 0), c1 = plan_child(T, plan, lane, 1);
+        store_coherent_i32(left + x, c0);
+        store_coherent_i32(right + x, c1);
+        store_coherent_i32(parent + node_index(n, c0), x);
+        store_coherent_i32(parent + node_index(n, c1), x);
         if (lane > 0) {  // the root's box is unchanged; its cost and height are published by its owner
-            float b[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-            uint32_t np = 0;
-            for (int j = 0; j < kTreeletLeaves; ++j)
-                if (S & (1u << j)) {
-                    for (int a = 0; a < 3; ++a) {
-                        b[a] = fminf(b[a], T.box[j][a]);
-                        b[3 + a] = fmaxf(b[3 + a], T.box[j][3 + a]);
-                    }
-                    np += T.lcnt[j];
-                }
+            const uint32_t S = (uint32_t)(plan.sets >> (8 * lane)) & 127u;
+            float b[6];
+            const uint32_t np = plan_bounds(T, S, b);
 #pragma unroll
             for (int k = 0; k < 6; ++k) store_coherent(nboxes + 6 * (uint64_t)x + k, b[k]);
             store_coherent(cost + x, T.cost[S]);
             store_coherent_u32(cnt + x, np);
-            store_coherent_u32(hgt + x, T.lh[lane]);
+            store_coherent_u32(hgt + x, (uint32_t)(plan.heights >> (8 * lane)) & 255u);
         }
     }
-    new_cost = total;
-    new_h = T.lh[0];
+    new_cost = plan.total;
+    new_h = (uint32_t)plan.heights & 255u;
+}
+
+// ---- subtrees in LDS ------------------------------------------------------------------------------------------
+//
+// A maximal subtree of at most kSubtree primitives as one wave holds it: internal nodes 0 .. nint - 1 breadth-first
+// from the root, primitives at kSubtree + 0 .. (local ids), each with its code in the binary tree.
+// 112: 9.6 KB of LDS, so that 16 waves share a CU, the four per SIMD that 128 registers allow; the two passes over 15.5M
+// triangles of 64 meshes take 11.0 + 2.5 ms (subtrees + the nodes above), with 96 primitives 11.1 + 3.0 ms, with 128
+// 14.8 + 2.2 ms.
+constexpr uint32_t kSubtree = 112;
+struct SubtreeLds {
+    float box[2 * kSubtree][6];
+    int32_t code[2 * kSubtree];
+    uint32_t kids[kSubtree];          // local ids of the children, 16 bits each
+    uint16_t level[kSubtree + 1];     // first node of each breadth-first level
+    uint32_t nint, nleaf, nlevel;
+};
+
+// Loads the codes and links of the subtree below `root` (an internal node).
+__device__ __forceinline__ void load_subtree(SubtreeLds& U, int32_t root, const int32_t* __restrict__ left,
+                                             const int32_t* __restrict__ right, uint32_t& nint, uint32_t& nleaf,
+                                             uint32_t& nlevel) {
+    const uint32_t lane = threadIdx.x;
+    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    __syncthreads();
+    if (lane == 0) {
+        U.code[0] = root;
+        U.level[0] = 0;
+    }
+    __syncthreads();
+    nint = 1;
+    nleaf = 0;
+    nlevel = 0;
+    for (uint32_t a = 0; a < nint;) {
+        const uint32_t end = nint;  // the level is [a, end)
+        ++nlevel;
+        if (lane == 0) U.level[nlevel] = (uint16_t)end;
+        for (; a < end; a += 64u) {
+            const bool on = a + lane < end;
+            int32_t c[2] = {0, 0};
+            if (on) {
+                const int32_t x = U.code[a + lane];
+                c[0] = left[x];
+                c[1] = right[x];
+            }
+            uint32_t id[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint64_t mi = __ballot(on && c[h] >= 0), ml = __ballot(on && c[h] < 0);
+                id[h] = c[h] >= 0 ? nint + (uint32_t)__popcll(mi & below)
+                                  : kSubtree + nleaf + (uint32_t)__popcll(ml & below);
+                nint += (uint32_t)__popcll(mi);
+                nleaf += (uint32_t)__popcll(ml);
+                if (on) U.code[id[h]] = c[h];
+            }
+            if (on) U.kids[a + lane] = id[0] | id[1] << 16;
+        }
+        a = end;
+        __syncthreads();
+    }
+}
+
+// Lists the maximal subtrees of at most kSubtree primitives (internal node or leaf codes) and clears the arrival
+// counts of the nodes above them.  A block looks at kFindNodes nodes and takes its places in the list at once (an atomic
+// on one word costs about 10 ns in turn: one per listed node took 1.1 ms on 15.5M triangles).
+constexpr uint32_t kFindNodes = 4096;
+__global__ __launch_bounds__(256) void find_subtrees_kernel(uint32_t n, const int32_t* __restrict__ left,
+                                                            const int32_t* __restrict__ right,
+                                                            const uint32_t* __restrict__ cnt,
+                                                            uint32_t* __restrict__ arrivals,
+                                                            int32_t* __restrict__ list, uint32_t* __restrict__ count) {
+    __shared__ uint32_t s_at, s_base;
+    if (n == 1 || cnt[0] <= kSubtree) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            list[0] = n == 1 ? -1 : 0;
+            *count = 1;
+        }
+        return;
+    }
+    const uint32_t first = blockIdx.x * kFindNodes;
+    uint32_t above = 0;  // bit t: this thread's t-th node lies above the listed subtrees
+    uint32_t want = 0;
+    if (threadIdx.x == 0) s_at = 0;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t t = 0; t < kFindNodes / 256u; ++t) {
+        const uint32_t i = first + t * 256u + threadIdx.x;
+        if (i >= n - 1 || cnt[i] <= kSubtree) continue;
+        arrivals[i] = 0;
+        above |= 1u << t;
+        const int32_t l = left[i], r = right[i];
+        want += (l < 0 || cnt[l] <= kSubtree ? 1u : 0u) + (r < 0 || cnt[r] <= kSubtree ? 1u : 0u);
+    }
+    uint32_t at = want ? atomicAdd(&s_at, want) : 0u;
+    __syncthreads();
+    if (threadIdx.x == 0) s_base = s_at ? atomicAdd(count, s_at) : 0u;
+    __syncthreads();
+    if (!want) return;
+    at += s_base;
+    for (; above; above &= above - 1u) {
+        const uint32_t i = first + ((uint32_t)__ffs((int)above) - 1u) * 256u + threadIdx.x;
+        const int32_t l = left[i], r = right[i];
+        if (l < 0 || cnt[l] <= kSubtree) list[at++] = l;
+        if (r < 0 || cnt[r] <= kSubtree) list[at++] = r;
+    }
+}
+
+struct RefineArgs {
+    uint32_t n;
+    int32_t* left;
+    int32_t* right;
+    int32_t* parent;
+    const uint32_t* order;
+    const float* prim_boxes;  // boxes of the primitives, for the first pass; nullptr: nboxes holds the leaves' boxes
+    float* nboxes;
+    float* cost;
+    uint32_t* cnt;
+    uint32_t* hgt;
+    uint32_t* arrivals;
+    uint32_t min_prims;  // 0xFFFFFFFF: plain refit
+    const uint32_t* node_blas;
+    const int32_t* list;  // subtree roots and their number
+    const uint32_t* count;
+};
+
+// Refit and refinement of the listed subtrees, one wave each.  A pass whose every node went through global memory
+// (agent-scope loads that miss the L2, about 16 dependent ones per treelet) took 18.0 and 12.3 ms for the two rounds on
+// 15.5M triangles, 4.4 ms for the first one on 4M; here the links and boxes of a subtree are read once.  What bounds it now:
+// the instructions of the treelets (about 600 VALU and 450 SALU each) at four waves per SIMD.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void subtree_refine_kernel(RefineArgs a) {
+    __shared__ SubtreeLds U;
+    __shared__ TreeletLds T;
+    __shared__ float ucost[kSubtree], uarea[kSubtree];
+    __shared__ uint32_t ucnt[kSubtree], uhgt[kSubtree];
+    const uint32_t lane = threadIdx.x;
+    SplitRegs sr;
+    load_splits(sr);
+    const uint32_t count = *a.count;
+    for (uint32_t ti = blockIdx.x; ti < count; ti += gridDim.x) {
+        const int32_t root = a.list[ti];
+        if (root < 0) {
+            if (a.prim_boxes && lane < 6u) {
+                const uint64_t pos = (uint64_t)(-1 - root);
+                a.nboxes[6 * ((uint64_t)a.n - 1 + pos) + lane] = a.prim_boxes[6 * (uint64_t)a.order[pos] + lane];
+            }
+            continue;
+        }
+        uint32_t nint, nleaf, nlevel;
+        load_subtree(U, root, a.left, a.right, nint, nleaf, nlevel);
+        for (uint32_t i = lane; i < nleaf; i += 64u) {
+            const uint64_t pos = (uint64_t)(-1 - U.code[kSubtree + i]);
+            float* nb = a.nboxes + 6 * ((uint64_t)a.n - 1 + pos);
+            const float* src = a.prim_boxes ? a.prim_boxes + 6 * (uint64_t)a.order[pos] : nb;
+#pragma unroll
+            for (int k = 0; k < 6; ++k) {
+                const float v = src[k];
+                U.box[kSubtree + i][k] = v;
+                if (a.prim_boxes) nb[k] = v;
+            }
+        }
+        __syncthreads();
+        auto children = [&](int32_t c, int32_t& l, int32_t& r, float& al, float& ar) {
+            const uint32_t k = U.kids[c];
+            const uint32_t kl = k & 0xFFFFu, kr = k >> 16;
+            // leaves as negative codes: -1 - local id
+            l = kl >= kSubtree ? -1 - (int32_t)kl : (int32_t)kl;
+            r = kr >= kSubtree ? -1 - (int32_t)kr : (int32_t)kr;
+            al = kl >= kSubtree ? -1.0f : uarea[kl];
+            ar = kr >= kSubtree ? -1.0f : uarea[kr];
+        };
+        for (uint32_t lv = nlevel; lv-- > 0;) {
+            const uint32_t end = U.level[lv + 1];
+            for (uint32_t at = U.level[lv]; at < end; at += 64u) {
+                const uint32_t x = at + lane;
+                bool need = false;
+                float ccost = 0.0f;
+                uint32_t chgt = 0;
+                if (x < end) {
+                    const uint32_t k = U.kids[x], l = k & 0xFFFFu, r = k >> 16;
+                    float b[6];
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        b[c] = fminf(U.box[l][c], U.box[r][c]);
+                        b[3 + c] = fmaxf(U.box[l][3 + c], U.box[r][3 + c]);
+                    }
+#pragma unroll
+                    for (int c = 0; c < 6; ++c) U.box[x][c] = b[c];
+                    const bool il = l < kSubtree, ir = r < kSubtree;
+                    const float area = box_area(b);
+                    ccost = area + ((il ? ucost[l] : 0.0f) + (ir ? ucost[r] : 0.0f));
+                    const uint32_t ccnt = (il ? ucnt[l] : 1u) + (ir ? ucnt[r] : 1u);
+                    const uint32_t hl = il ? uhgt[l] : 0u, hr = ir ? uhgt[r] : 0u;
+                    chgt = 1u + (hl > hr ? hl : hr);
+                    ucost[x] = ccost;
+                    uarea[x] = area;
+                    ucnt[x] = ccnt;
+                    uhgt[x] = chgt;
+                    // batched builds never restructure across BLASes
+                    need = ccnt >= a.min_prims && (!a.node_blas || a.node_blas[U.code[x]] != kMixedBlas);
+                }
+                __syncthreads();
+                TreeletForm form;
+                uint64_t todo = __ballot(need && treelet_form((int32_t)x, children, form));
+                while (todo) {
+                    const int L = __ffsll((unsigned long long)todo) - 1;
+                    todo &= todo - 1;
+                    const float rc = __shfl(ccost, L);
+                    const uint32_t rh = (uint32_t)__shfl((int)chgt, L);
+                    if ((int)lane == L) stage_form(T, form);
+                    __syncthreads();
+                    if (lane < (uint32_t)kTreeletLeaves) {
+                        const int32_t c = T.leaf[lane];
+                        const uint32_t id = c >= 0 ? (uint32_t)c : (uint32_t)(-1 - c);
+                        T.leaf[lane] = (int32_t)id;
+#pragma unroll
+                        for (int k = 0; k < 6; ++k) T.box[lane][k] = U.box[id][k];
+                        T.cost[1u << lane] = c >= 0 ? ucost[id] : 0.0f;
+                        T.lcnt[lane] = c >= 0 ? ucnt[id] : 1u;
+                        T.lhgt[lane] = c >= 0 ? uhgt[id] : 0u;
+                    }
+                    __syncthreads();
+                    const TreeletPlan plan = treelet_solve(T, sr, rc, rh);
+                    if (plan.commit && lane < kTreeletNodes) {
+                        const uint32_t y = (uint32_t)T.pool[lane];
+                        U.kids[y] = (uint32_t)plan_child(T, plan, lane, 0) | (uint32_t)plan_child(T, plan, lane, 1) << 16;
+                        uhgt[y] = (uint32_t)(plan.heights >> (8 * lane)) & 255u;
+                        if (lane == 0) {
+                            ucost[y] = plan.total;
+                        } else {
+                            const uint32_t S = (uint32_t)(plan.sets >> (8 * lane)) & 127u;
+                            float b[6];
+                            ucnt[y] = plan_bounds(T, S, b);
+#pragma unroll
+                            for (int k = 0; k < 6; ++k) U.box[y][k] = b[k];
+                            uarea[y] = box_area(b);
+                            ucost[y] = T.cost[S];
+                        }
+                    }
+                    __syncthreads();
+                }
+            }
+        }
+        for (uint32_t i = lane; i < nint; i += 64u) {
+            const int32_t x = U.code[i];
+            const uint32_t k = U.kids[i];
+            const int32_t c0 = U.code[k & 0xFFFFu], c1 = U.code[k >> 16];
+            a.left[x] = c0;
+            a.right[x] = c1;
+            a.parent[node_index(a.n, c0)] = x;
+            a.parent[node_index(a.n, c1)] = x;
+#pragma unroll
+            for (int c = 0; c < 6; ++c) a.nboxes[6 * (uint64_t)x + c] = U.box[i][c];
+            a.cost[x] = ucost[i];
+            a.cnt[x] = ucnt[i];
+            a.hgt[x] = uhgt[i];
+        }
+    }
 }
 
 // Treelet refinement rounds: default kTreeletRounds, none under PREFER_FAST_BUILD, RTX_BUILD_TREELET_ROUNDS_*
@@ -852,97 +1157,115 @@ int treelet_rounds(uint32_t flags, uint32_t n) {
     return (flags & RTX_BUILD_PREFER_FAST_BUILD_BIT) ? 0 : kTreeletRounds;
 }
 
-// One wave per block.  min_prims = 0xFFFFFFFF: plain refit.
-__global__ __launch_bounds__(64) void refit_refine_kernel(uint32_t n, int32_t* left, int32_t* right, int32_t* parent,
-                                                          const uint32_t* __restrict__ order,
-                                                          const float* __restrict__ prim_boxes, float* nboxes,
-                                                          float* cost, uint32_t* cnt, uint32_t* hgt,
-                                                          uint32_t* arrivals, uint32_t min_prims,
-                                                          const uint32_t* __restrict__ node_blas) {
+// Refit and refinement of the nodes above the listed subtrees, one wave per block, one subtree per lane; with no list
+// (an update's refit, whose kept hierarchy has no counts) of the whole tree, one leaf per lane.
+__global__ __launch_bounds__(64) void refit_refine_kernel(RefineArgs a) {
     __shared__ TreeletLds T;
     const uint32_t lane = threadIdx.x;
-    const uint32_t pos = blockIdx.x * 64u + lane;
-    bool active = pos < n;
-    float cur[6] = {0, 0, 0, 0, 0, 0};
-    float ccost = 0.0f;
-    uint32_t ccnt = 1, chgt = 0;
-    uint64_t self = 0;
-    int32_t node = -1;
-    if (active) {
-        const float* pb = prim_boxes + 6 * (uint64_t)order[pos];
-#pragma unroll
-        for (int k = 0; k < 6; ++k) cur[k] = pb[k];
-        self = (uint64_t)n - 1 + pos;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) store_coherent(nboxes + 6 * self + k, cur[k]);
-        node = load_coherent_i32(parent + self);
-    }
-    while (__ballot(active)) {
-        bool own = false;
+    const uint32_t n = a.n;
+    SplitRegs sr;
+    load_splits(sr);
+    auto children = [&](int32_t c, int32_t& l, int32_t& r, float& al, float& ar) {
+        l = load_coherent_i32(a.left + c);
+        r = load_coherent_i32(a.right + c);
+        al = l >= 0 ? coherent_area(a.nboxes, (uint64_t)l) : -1.0f;
+        ar = r >= 0 ? coherent_area(a.nboxes, (uint64_t)r) : -1.0f;
+    };
+    // a wave takes a batch of subtrees: as few as the waves of the launch allow, since it works on its lanes' treelets
+    // one after another
+    const uint32_t count = a.list ? *a.count : n;
+    const uint32_t share = (count - 1u) / gridDim.x + 1u;
+    const uint32_t batch = a.list && share < 64u ? share : 64u;
+    for (uint32_t first = blockIdx.x * batch; first < count; first += gridDim.x * batch) {
+        bool active = lane < batch && first + lane < count;
+        float cur[6] = {0, 0, 0, 0, 0, 0};
+        float ccost = 0.0f;
+        uint32_t ccnt = 1, chgt = 0;
+        uint64_t self = 0;
+        int32_t node = -1;
         if (active) {
-            if (node < 0) {
-                active = false;
-            } else {
-                __atomic_signal_fence(__ATOMIC_SEQ_CST);
-                __builtin_amdgcn_s_waitcnt(0);
-                __atomic_signal_fence(__ATOMIC_SEQ_CST);
-                const uint32_t old = __hip_atomic_fetch_add(&arrivals[node], 1u, __ATOMIC_RELAXED,
-                                                            __HIP_MEMORY_SCOPE_AGENT);
-                if (old == 0u) {
+            const int32_t c = a.list ? a.list[first + lane] : -1 - (int32_t)(first + lane);
+            self = node_index(n, c);
+            const float* src = a.list ? a.nboxes + 6 * self : a.prim_boxes + 6 * (uint64_t)a.order[first + lane];
+#pragma unroll
+            for (int k = 0; k < 6; ++k) cur[k] = src[k];
+            if (!a.list) {
+#pragma unroll
+                for (int k = 0; k < 6; ++k) store_coherent(a.nboxes + 6 * self + k, cur[k]);
+            }
+            if (c >= 0) {
+                ccost = a.cost[c];
+                ccnt = a.cnt[c];
+                chgt = a.hgt[c];
+            }
+            node = load_coherent_i32(a.parent + self);
+        }
+        // the vote stands in the loop's single latch: with two latches (after the last `if`, and past it) the compiler
+        // may nest the loop, and the lanes without a node would leave it while the others still work as a wave
+        for (bool any = __any(active); any; any = __any(active)) {
+            bool own = false;
+            if (active) {
+                if (node < 0) {
                     active = false;
                 } else {
-                    own = true;
-                    const int32_t l = load_coherent_i32(left + node), r = load_coherent_i32(right + node);
-                    const uint64_t li = node_index(n, l), ri = node_index(n, r);
-                    const bool self_left = li == self;
-                    const int32_t sc = self_left ? r : l;
-                    const uint64_t sib = self_left ? ri : li;
-                    const float scost = sc >= 0 ? load_coherent(cost + sc) : 0.0f;
-                    const uint32_t scnt = sc >= 0 ? load_coherent_u32(cnt + sc) : 1u;
-                    const uint32_t shgt = sc >= 0 ? load_coherent_u32(hgt + sc) : 0u;
+                    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+                    __builtin_amdgcn_s_waitcnt(0);
+                    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+                    const uint32_t old = __hip_atomic_fetch_add(&a.arrivals[node], 1u, __ATOMIC_RELAXED,
+                                                                __HIP_MEMORY_SCOPE_AGENT);
+                    if (old == 0u) {
+                        active = false;
+                    } else {
+                        own = true;
+                        const int32_t l = load_coherent_i32(a.left + node), r = load_coherent_i32(a.right + node);
+                        const uint64_t li = node_index(n, l), ri = node_index(n, r);
+                        const bool self_left = li == self;
+                        const int32_t sc = self_left ? r : l;
+                        const uint64_t sib = self_left ? ri : li;
+                        const float scost = sc >= 0 ? load_coherent(a.cost + sc) : 0.0f;
+                        const uint32_t scnt = sc >= 0 ? load_coherent_u32(a.cnt + sc) : 1u;
+                        const uint32_t shgt = sc >= 0 ? load_coherent_u32(a.hgt + sc) : 0u;
 #pragma unroll
-                    for (int a = 0; a < 3; ++a) {
-                        cur[a] = fminf(cur[a], load_coherent(nboxes + 6 * sib + a));
-                        cur[3 + a] = fmaxf(cur[3 + a], load_coherent(nboxes + 6 * sib + 3 + a));
+                        for (int k = 0; k < 3; ++k) {
+                            cur[k] = fminf(cur[k], load_coherent(a.nboxes + 6 * sib + k));
+                            cur[3 + k] = fmaxf(cur[3 + k], load_coherent(a.nboxes + 6 * sib + 3 + k));
+                        }
+                        const float cl = self_left ? ccost : scost, cr = self_left ? scost : ccost;
+                        ccost = box_area(cur) + (cl + cr);
+                        ccnt += scnt;
+                        chgt = 1u + (chgt > shgt ? chgt : shgt);
                     }
-                    const float cl = self_left ? ccost : scost, cr = self_left ? scost : ccost;
-                    ccost = box_area(cur) + (cl + cr);
-                    ccnt += scnt;
-                    chgt = 1u + (chgt > shgt ? chgt : shgt);
                 }
             }
-        }
-        // batched builds never restructure across BLASes
-        const bool root = own && ccnt >= min_prims && (!node_blas || node_blas[node] != kMixedBlas);
-        uint64_t need = __ballot(root);
-        // every lane with a treelet root forms its treelet at once (the dependent child / box loads overlap), then
-        // the wave restructures them one after another
-        TreeletForm form;
-        const bool formed = root && treelet_form(node, left, right, nboxes, form);
-        const uint64_t formed_mask = __ballot(formed);
-        while (need) {
-            const int L = __ffsll((unsigned long long)need) - 1;
-            need &= need - 1;
-            const int32_t R = __shfl(node, L);
-            const float rc = __shfl(ccost, L);
-            const uint32_t rh = (uint32_t)__shfl((int)chgt, L);
-            float nc;
-            uint32_t nh;
-            treelet_optimize(T, n, R, rc, rh, (uint32_t)L, ((formed_mask >> L) & 1ull) != 0ull, form, left, right,
-                             parent, nboxes, cost, cnt, hgt, nc, nh);
-            if ((int)lane == L) {
-                ccost = nc;
-                chgt = nh;
+            // batched builds never restructure across BLASes
+            const bool root = own && ccnt >= a.min_prims && (!a.node_blas || a.node_blas[node] != kMixedBlas);
+            // every lane with a treelet root forms its treelet at once (the dependent child / box loads overlap),
+            // then the wave restructures them one after another
+            TreeletForm form;
+            uint64_t need = __ballot(root && treelet_form(node, children, form));
+            while (need) {
+                const int L = __ffsll((unsigned long long)need) - 1;
+                need &= need - 1;
+                const float rc = __shfl(ccost, L);
+                const uint32_t rh = (uint32_t)__shfl((int)chgt, L);
+                float nc;
+                uint32_t nh;
+                treelet_optimize(T, sr, n, rc, rh, (uint32_t)L, form, a.left, a.right, a.parent, a.nboxes, a.cost,
+                                 a.cnt, a.hgt, nc, nh);
+                if ((int)lane == L) {
+                    ccost = nc;
+                    chgt = nh;
+                }
             }
-        }
-        if (own) {
+            if (own) {
 #pragma unroll
-            for (int k = 0; k < 6; ++k) store_coherent(nboxes + 6 * (uint64_t)node + k, cur[k]);
-            store_coherent(cost + node, ccost);
-            store_coherent_u32(cnt + node, ccnt);
-            store_coherent_u32(hgt + node, chgt);
-            self = (uint64_t)node;
-            node = load_coherent_i32(parent + node);
+                for (int k = 0; k < 6; ++k) store_coherent(a.nboxes + 6 * (uint64_t)node + k, cur[k]);
+                store_coherent(a.cost + node, ccost);
+                store_coherent_u32(a.cnt + node, ccnt);
+                store_coherent_u32(a.hgt + node, chgt);
+                self = (uint64_t)node;
+                node = load_coherent_i32(a.parent + node);
+            }
         }
     }
 }
@@ -1562,6 +1885,10 @@ __global__ void set_update_offset_kernel(AsHeader* h, uint64_t off) {
 constexpr float kLeafCostTri = 0.3f;
 constexpr float kLeafCostInstance = 1.0f;
 
+// Persistent one-wave blocks of the subtree passes.
+constexpr uint32_t kSubtreeBlocks = 4096;
+
+// counted: cnt holds the primitive counts of the internal nodes (written with the hierarchy).
 // Refit with treelet refinement; each further round restructures the tree the previous one left.  Then the costs
 // of the 8-wide collapse (wcost) over the final tree.
 // Children per wide node: RTX_BUILD_MAX_WIDTH(w) caps it at w (2..7), 0 = 8.
@@ -1571,16 +1898,45 @@ int node_width(uint32_t flags) {
 }
 
 void refit_passes(uint32_t n, uint32_t flags, uint8_t* scratch, const Layout& L, const float* prim_boxes,
-                  hipStream_t s, const uint32_t* node_blas = nullptr, float c_leaf = kLeafCostTri) {
+                  hipStream_t s, const uint32_t* node_blas = nullptr, float c_leaf = kLeafCostTri,
+                  bool counted = true) {
     const int rounds = treelet_rounds(flags, n);
     uint32_t* arrivals = (uint32_t*)(scratch + L.arrivals);
-    for (int round = 0; round < (rounds ? rounds : 1); ++round) {
+    RefineArgs a;
+    a.n = n;
+    a.left = (int32_t*)(scratch + L.left);
+    a.right = (int32_t*)(scratch + L.right);
+    a.parent = (int32_t*)(scratch + L.parent);
+    a.order = (const uint32_t*)(scratch + L.vals);
+    a.prim_boxes = prim_boxes;
+    a.nboxes = (float*)(scratch + L.nboxes);
+    a.cost = (float*)(scratch + L.cost);
+    a.cnt = (uint32_t*)(scratch + L.cnt);
+    a.hgt = (uint32_t*)(scratch + L.hgt);
+    a.arrivals = arrivals;
+    a.node_blas = node_blas;
+    a.list = nullptr;
+    a.count = nullptr;
+    if (!counted) {
         if (n > 1) fill_kernel<<<256, 256, 0, s>>>(arrivals, n, 0u);
-        refit_refine_kernel<<<(n + 63) / 64, 64, 0, s>>>(
-            n, (int32_t*)(scratch + L.left), (int32_t*)(scratch + L.right), (int32_t*)(scratch + L.parent),
-            (const uint32_t*)(scratch + L.vals), prim_boxes, (float*)(scratch + L.nboxes), (float*)(scratch + L.cost),
-            (uint32_t*)(scratch + L.cnt), (uint32_t*)(scratch + L.hgt), arrivals,
-            rounds ? kTreeletMinPrims[round] : 0xFFFFFFFFu, node_blas);
+        a.min_prims = 0xFFFFFFFFu;
+        refit_refine_kernel<<<(n + 63) / 64, 64, 0, s>>>(a);
+    } else {
+        // the list of subtrees lies where the collapse keeps its tasks later
+        int32_t* list = (int32_t*)(scratch + L.tasks1);
+        uint32_t* counts = (uint32_t*)(scratch + L.misc) + 8;  // one word per round
+        fill_kernel<<<1, 64, 0, s>>>(counts, 4, 0u);
+        a.list = list;
+        for (int round = 0; round < (rounds ? rounds : 1); ++round) {
+            a.count = counts + round;
+            a.min_prims = rounds ? kTreeletMinPrims[round] : 0xFFFFFFFFu;
+            if (round) a.prim_boxes = nullptr;
+            find_subtrees_kernel<<<(n - 1) / kFindNodes + 1, 256, 0, s>>>(n, a.left, a.right, a.cnt, arrivals, list,
+                                                                 counts + round);
+            const uint32_t few = n / 8 + 1;  // at most this many waves
+            subtree_refine_kernel<<<std::min(few, kSubtreeBlocks), 64, 0, s>>>(a);
+            if (n > kSubtree) refit_refine_kernel<<<std::min(few, kSubtreeBlocks), 64, 0, s>>>(a);
+        }
     }
     if (n > 1) {
         fill_kernel<<<256, 256, 0, s>>>(arrivals, n, 0u);
@@ -1621,9 +1977,11 @@ hipError_t lbvh_common(uint32_t n, bool k64, uint32_t type, uint32_t flags, uint
         }
         if (n > 1) {
             if (k64)
-                karras_kernel<uint64_t><<<gb, 256, 0, s>>>((uint64_t*)(scratch + L.keys), n, left, right, parent);
+                karras_kernel<uint64_t><<<gb, 256, 0, s>>>((uint64_t*)(scratch + L.keys), n, left, right, parent,
+                                                           (uint32_t*)(scratch + L.cnt));
             else
-                karras_kernel<uint32_t><<<gb, 256, 0, s>>>((uint32_t*)(scratch + L.keys), n, left, right, parent);
+                karras_kernel<uint32_t><<<gb, 256, 0, s>>>((uint32_t*)(scratch + L.keys), n, left, right, parent,
+                                                           (uint32_t*)(scratch + L.cnt));
         } else {
             fill_kernel<<<1, 64, 0, s>>>((uint32_t*)parent, 1, 0xFFFFFFFFu);
         }
@@ -1671,13 +2029,15 @@ hipError_t debug_tree(const float* boxes, uint32_t n, bool k64, int rounds, void
             e = sort_pairs_u64((uint64_t*)(sc + L.keys), vals, n, sc + L.sort, err_flags, s);
             if (!e && n > 1)
                 karras_kernel<uint64_t><<<gb, 256, 0, s>>>((uint64_t*)(sc + L.keys), n, (int32_t*)(sc + L.left),
-                                                           (int32_t*)(sc + L.right), (int32_t*)(sc + L.parent));
+                                                           (int32_t*)(sc + L.right), (int32_t*)(sc + L.parent),
+                                                           (uint32_t*)(sc + L.cnt));
         } else {
             morton_kernel<uint32_t><<<gb, 256, 0, s>>>(boxes, n, cb, (uint32_t*)(sc + L.keys));
             e = sort_pairs_u32((uint32_t*)(sc + L.keys), vals, n, sc + L.sort, err_flags, s);
             if (!e && n > 1)
                 karras_kernel<uint32_t><<<gb, 256, 0, s>>>((uint32_t*)(sc + L.keys), n, (int32_t*)(sc + L.left),
-                                                           (int32_t*)(sc + L.right), (int32_t*)(sc + L.parent));
+                                                           (int32_t*)(sc + L.right), (int32_t*)(sc + L.parent),
+                                                           (uint32_t*)(sc + L.cnt));
         }
     }
     if (!e && rounds >= 0 && n > 1)
@@ -1815,7 +2175,7 @@ hipError_t update_blas(const GeomDesc* geoms_host, uint32_t ngeom, uint32_t n, u
         if ((err = hipMemcpyAsync(sc + L.parent, u + 4ull * (3 * n - 2), 4ull * (2 * n - 1),
                                   hipMemcpyDeviceToDevice, s)))
             return err;
-        refit_passes(n, flags | RTX_BUILD_NO_TREELET_BIT, sc, L, (const float*)(sc + L.boxes), s);
+        refit_passes(n, flags | RTX_BUILD_NO_TREELET_BIT, sc, L, (const float*)(sc + L.boxes), s, nullptr, kLeafCostTri, false);
     }
     uint32_t* levels = (uint32_t*)(sc + L.levels);
     uint2* t0 = (uint2*)(sc + L.tasks0);
@@ -1898,7 +2258,7 @@ hipError_t build_blas_batch(const GeomDesc* geoms_host, uint32_t ngeom, const ui
         morton_batch_kernel<<<gb, 256, 0, s>>>(boxes, n, cb, pblas, keys);
         if ((err = sort_pairs_u64(keys, vals, n, sc + L.sort, err_flags, s))) return err;
         if (n > 1) {
-            karras_kernel<uint64_t><<<gb, 256, 0, s>>>(keys, n, left, right, parent, nblas);
+            karras_kernel<uint64_t><<<gb, 256, 0, s>>>(keys, n, left, right, parent, (uint32_t*)(sc + L.cnt), nblas);
         } else {
             fill_kernel<<<1, 64, 0, s>>>((uint32_t*)parent, 1, 0xFFFFFFFFu);
         }

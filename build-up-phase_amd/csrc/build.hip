@@ -10,11 +10,9 @@
 //   karras    binary radix tree over the sorted codes (Karras 2012), one thread per internal node
 //   refit     bottom-up boxes and treelet refinement: subtrees of up to kSubtree primitives a wave each in LDS, then the
 //             nodes above them, the second thread to reach a node merging its children (atomic arrival count)
-//   collapse  level-synchronous top-down conversion to 8-wide nodes: each node adopts up to 8 children by
-//             repeatedly opening the child with the largest surface area, places them by octant, quantises
-//             their boxes to 8 bits per plane and allocates their slots with one atomic add.
-// Karras trees over 30-bit codes with 32-bit index tie-breaks are at most 64 levels deep (63-bit codes: 96),
-// so the host enqueues that many collapse levels; a level whose frontier is empty returns at once.
+//   collapse  top-down conversion to 8-wide nodes: each node adopts the children that the SAH-optimal choice gives it,
+//             places them by octant, quantises their boxes to 8 bits per plane and gives them consecutive slots; the
+//             nodes above the subtrees through a queue, then the subtrees a wave each.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -26,10 +24,6 @@
 namespace rtx {
 
 namespace {
-
-constexpr int kCollapseBlocks = 1024;
-constexpr int kMaxLevels32 = 66;
-constexpr int kMaxLevels64 = 98;
 
 struct Box {
     float lo[3], hi[3];
@@ -897,11 +891,9 @@ __device__ __forceinline__ void treelet_optimize(TreeletLds& T, const SplitRegs&
 // 14.8 + 2.2 ms.
 constexpr uint32_t kSubtree = 112;
 struct SubtreeLds {
-    float box[2 * kSubtree][6];
     int32_t code[2 * kSubtree];
     uint32_t kids[kSubtree];          // local ids of the children, 16 bits each
     uint16_t level[kSubtree + 1];     // first node of each breadth-first level
-    uint32_t nint, nleaf, nlevel;
 };
 
 // Loads the codes and links of the subtree below `root` (an internal node).
@@ -950,14 +942,18 @@ __device__ __forceinline__ void load_subtree(SubtreeLds& U, int32_t root, const 
 
 // Lists the maximal subtrees of at most kSubtree primitives (internal node or leaf codes) and clears the arrival
 // counts of the nodes above them.  A block looks at kFindNodes nodes and takes its places in the list at once (an atomic
-// on one word costs about 10 ns in turn: one per listed node took 1.1 ms on 15.5M triangles).
+// on one word costs about 10 ns in turn: one per listed node took 1.1 ms on 15.5M triangles).  queue: an empty place for
+// each of the nodes above, which the collapse queues its tasks in.
 constexpr uint32_t kFindNodes = 4096;
+constexpr uint64_t kNoTask = ~0ull;
 __global__ __launch_bounds__(256) void find_subtrees_kernel(uint32_t n, const int32_t* __restrict__ left,
                                                             const int32_t* __restrict__ right,
                                                             const uint32_t* __restrict__ cnt,
                                                             uint32_t* __restrict__ arrivals,
-                                                            int32_t* __restrict__ list, uint32_t* __restrict__ count) {
-    __shared__ uint32_t s_at, s_base;
+                                                            int32_t* __restrict__ list, uint32_t* __restrict__ count,
+                                                            uint64_t* __restrict__ queue,
+                                                            uint32_t* __restrict__ queue_size) {
+    __shared__ uint32_t s_at, s_base, s_above, s_above_base;
     if (n == 1 || cnt[0] <= kSubtree) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             list[0] = n == 1 ? -1 : 0;
@@ -968,7 +964,7 @@ __global__ __launch_bounds__(256) void find_subtrees_kernel(uint32_t n, const in
     const uint32_t first = blockIdx.x * kFindNodes;
     uint32_t above = 0;  // bit t: this thread's t-th node lies above the listed subtrees
     uint32_t want = 0;
-    if (threadIdx.x == 0) s_at = 0;
+    if (threadIdx.x == 0) s_at = s_above = 0;
     __syncthreads();
 #pragma unroll
     for (uint32_t t = 0; t < kFindNodes / 256u; ++t) {
@@ -980,9 +976,16 @@ __global__ __launch_bounds__(256) void find_subtrees_kernel(uint32_t n, const in
         want += (l < 0 || cnt[l] <= kSubtree ? 1u : 0u) + (r < 0 || cnt[r] <= kSubtree ? 1u : 0u);
     }
     uint32_t at = want ? atomicAdd(&s_at, want) : 0u;
+    const uint32_t nabove = queue ? (uint32_t)__popc(above) : 0u;
+    uint32_t qat = nabove ? atomicAdd(&s_above, nabove) : 0u;
     __syncthreads();
-    if (threadIdx.x == 0) s_base = s_at ? atomicAdd(count, s_at) : 0u;
+    if (threadIdx.x == 0) {
+        s_base = s_at ? atomicAdd(count, s_at) : 0u;
+        s_above_base = s_above ? atomicAdd(queue_size, s_above) : 0u;
+    }
     __syncthreads();
+    qat += s_above_base;
+    for (uint32_t k = 0; k < nabove; ++k) queue[qat + k] = kNoTask;
     if (!want) return;
     at += s_base;
     for (; above; above &= above - 1u) {
@@ -1017,6 +1020,7 @@ struct RefineArgs {
 // the instructions of the treelets (about 600 VALU and 450 SALU each) at four waves per SIMD.
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void subtree_refine_kernel(RefineArgs a) {
     __shared__ SubtreeLds U;
+    __shared__ float ubox[2 * kSubtree][6];
     __shared__ TreeletLds T;
     __shared__ float ucost[kSubtree], uarea[kSubtree];
     __shared__ uint32_t ucnt[kSubtree], uhgt[kSubtree];
@@ -1042,7 +1046,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void su
 #pragma unroll
             for (int k = 0; k < 6; ++k) {
                 const float v = src[k];
-                U.box[kSubtree + i][k] = v;
+                ubox[kSubtree + i][k] = v;
                 if (a.prim_boxes) nb[k] = v;
             }
         }
@@ -1068,11 +1072,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void su
                     float b[6];
 #pragma unroll
                     for (int c = 0; c < 3; ++c) {
-                        b[c] = fminf(U.box[l][c], U.box[r][c]);
-                        b[3 + c] = fmaxf(U.box[l][3 + c], U.box[r][3 + c]);
+                        b[c] = fminf(ubox[l][c], ubox[r][c]);
+                        b[3 + c] = fmaxf(ubox[l][3 + c], ubox[r][3 + c]);
                     }
 #pragma unroll
-                    for (int c = 0; c < 6; ++c) U.box[x][c] = b[c];
+                    for (int c = 0; c < 6; ++c) ubox[x][c] = b[c];
                     const bool il = l < kSubtree, ir = r < kSubtree;
                     const float area = box_area(b);
                     ccost = area + ((il ? ucost[l] : 0.0f) + (ir ? ucost[r] : 0.0f));
@@ -1101,7 +1105,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void su
                         const uint32_t id = c >= 0 ? (uint32_t)c : (uint32_t)(-1 - c);
                         T.leaf[lane] = (int32_t)id;
 #pragma unroll
-                        for (int k = 0; k < 6; ++k) T.box[lane][k] = U.box[id][k];
+                        for (int k = 0; k < 6; ++k) T.box[lane][k] = ubox[id][k];
                         T.cost[1u << lane] = c >= 0 ? ucost[id] : 0.0f;
                         T.lcnt[lane] = c >= 0 ? ucnt[id] : 1u;
                         T.lhgt[lane] = c >= 0 ? uhgt[id] : 0u;
@@ -1119,7 +1123,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void su
                             float b[6];
                             ucnt[y] = plan_bounds(T, S, b);
 #pragma unroll
-                            for (int k = 0; k < 6; ++k) U.box[y][k] = b[k];
+                            for (int k = 0; k < 6; ++k) ubox[y][k] = b[k];
                             uarea[y] = box_area(b);
                             ucost[y] = T.cost[S];
                         }
@@ -1137,7 +1141,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void su
             a.parent[node_index(a.n, c0)] = x;
             a.parent[node_index(a.n, c1)] = x;
 #pragma unroll
-            for (int c = 0; c < 6; ++c) a.nboxes[6 * (uint64_t)x + c] = U.box[i][c];
+            for (int c = 0; c < 6; ++c) a.nboxes[6 * (uint64_t)x + c] = ubox[i][c];
             a.cost[x] = ucost[i];
             a.cnt[x] = ucnt[i];
             a.hgt[x] = uhgt[i];
@@ -1273,86 +1277,247 @@ __global__ __launch_bounds__(64) void refit_refine_kernel(RefineArgs a) {
 // ---- costs of the 8-wide collapse ------------------------------------------------------------------------------
 //
 // The SAH-optimal collapse of the binary tree into 8-wide nodes (Ylitie, Karras & Laine 2017, section 4), for
-// this layout's leaves (one primitive per child slot).  wc[8x + j - 1] = C(x, j), the least cost of the subtree of
+// this layout's leaves (one primitive per child slot).  C(x, j), j = 1..8, is the least cost of the subtree of
 // x spread over at most j child slots of its parent:
 //   leaf:      C(x, j) = c_leaf * A(x)
 //   internal:  D(x, j) = min over k in [1, j-1] of C(l, k) + C(r, j - k)        (x dissolved into j slots)
 //              C(x, 1) = A(x) + D(x, W)                                         (x becomes a wide node)
 //              C(x, j) = min(C(x, j - 1), D(x, j)),  j >= 2
-// computed bottom-up (second arrival merges, as the refit).  The collapse then takes, for each wide node x, the
-// children that D(x, W) picks.  W is the build's node width (8, or 2..7 from RTX_BUILD_MAX_WIDTH): narrower trees
-// use the same 64-B node with fewer children.
-__device__ __forceinline__ void wide_table(uint32_t n, int32_t c, const float* nboxes, const float* wc, float c_leaf,
-                                           float* t) {
-    if (c < 0) {
-        float b[6];
-        const uint64_t bi = (uint64_t)n - 1 + (uint64_t)(-1 - c);
+// computed bottom-up: the listed subtrees a wave each in LDS, then the nodes above (second arrival merges, as the
+// refit).  The collapse then takes, for each wide node x, the children that D(x, W) picks.  W is the build's node width
+// (8, or 2..7 from RTX_BUILD_MAX_WIDTH): narrower trees use the same 64-B node with fewer children.
+//
+// wdec[x], 4 bits for each j = 2..8: the left child's slot count k that D(x, j) takes, and 8 where D(x, j) beats
+// C(x, j - 1).  Along with the costs go the slots that the choice takes in all (the primitives with a box and the wide
+// nodes) and its depth in wide nodes, so that the collapse of a subtree knows its place before it starts: sub[x], for
+// the nodes of the listed subtrees: slots below x as a wide node (8 bits) | wide nodes from x down << 8 | depth << 16.
+__device__ __forceinline__ bool box_valid(const float* b) { return b[0] <= b[3] && b[1] <= b[4] && b[2] <= b[5]; }
+
+struct WideRow {
+    float c[8];
+    uint64_t slots, depth;  // a byte for each j (slots: listed subtrees only)
+};
+
+// Row j = 2..W.. of x from its children's rows; returns wdec, and in `dissolved` the row of D(x, W).
+__device__ __forceinline__ uint32_t wide_merge(const WideRow& l, const WideRow& r, float area, bool valid, int width,
+                                               WideRow& out, uint32_t& slots_below) {
+    float d[9];
+    uint32_t k[9];
+    uint32_t dec = 0;
 #pragma unroll
-        for (int k = 0; k < 6; ++k) b[k] = load_coherent(nboxes + 6 * bi + k);
-        const float a = c_leaf * box_area(b);
+    for (int j = 2; j <= 8; ++j) {
+        d[j] = INFINITY;
+        k[j] = 1;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) t[j] = a;
-    } else {
+        for (int i = 1; i < j; ++i) {
+            const float c = l.c[i - 1] + r.c[j - i - 1];
+            if (c < d[j]) {
+                d[j] = c;
+                k[j] = (uint32_t)i;
+            }
+        }
+    }
+    float dw = d[8];
+    uint32_t kw = k[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) t[j] = load_coherent(wc + 8 * (uint64_t)c + j);
+    for (int j = 2; j < 8; ++j)
+        if (j == width) {
+            dw = d[j];
+            kw = k[j];
+        }
+    auto at = [](uint64_t v, uint32_t j) { return (uint32_t)(v >> (8 * (j - 1))) & 255u; };
+    auto both = [&](uint32_t j, uint32_t kk, uint32_t& sl, uint32_t& de) {
+        sl = at(l.slots, kk) + at(r.slots, j - kk);
+        const uint32_t a = at(l.depth, kk), b = at(r.depth, j - kk);
+        de = a > b ? a : b;
+    };
+    uint32_t sl, de;
+    both((uint32_t)width, kw, sl, de);
+    slots_below = sl;
+    sl = valid ? 1u + sl : 0u;
+    de = valid ? 1u + de : 0u;
+    out.c[0] = area + dw;
+    out.slots = sl;
+    out.depth = de;
+#pragma unroll
+    for (uint32_t j = 2; j <= 8; ++j) {
+        const bool split = d[j] < out.c[j - 2];
+        dec |= (k[j] | (split ? 8u : 0u)) << (4 * (j - 2));
+        out.c[j - 1] = fminf(out.c[j - 2], d[j]);
+        if (split) both(j, k[j], sl, de);
+        out.slots |= (uint64_t)(sl & 255u) << (8 * (j - 1));
+        out.depth |= (uint64_t)(de & 255u) << (8 * (j - 1));
+    }
+    return dec;
+}
+
+__device__ __forceinline__ void wide_leaf(const float* b, float c_leaf, WideRow& t) {
+    const float a = c_leaf * box_area(b);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) t.c[j] = a;
+    t.slots = box_valid(b) ? 0x0101010101010101ull : 0ull;
+    t.depth = 0;
+}
+
+struct CostArgs {
+    uint32_t n;
+    const int32_t* left;
+    const int32_t* right;
+    const int32_t* parent;
+    const float* nboxes;
+    float* wc;        // rows of the listed roots and the nodes above: 8 costs, and the depths
+    uint64_t* depths;
+    uint32_t* wdec;
+    uint32_t* sub;
+    uint32_t* arrivals;
+    float c_leaf;
+    int width;
+    const int32_t* list;
+    const uint32_t* count;
+};
+
+// (The two passes took 1.2 ms on 4M triangles through global memory, node by node; 0.24 + 0.08 ms.)
+__global__ __launch_bounds__(64) void subtree_cost_kernel(CostArgs a) {
+    __shared__ SubtreeLds U;
+    __shared__ WideRow row[kSubtree];
+    __shared__ float leaf_cost[kSubtree];  // negative: no box
+    __shared__ uint8_t leaves[kSubtree];   // primitives with a box below each node
+    const uint32_t lane = threadIdx.x;
+    const uint32_t count = *a.count;
+    for (uint32_t ti = blockIdx.x; ti < count; ti += gridDim.x) {
+        const int32_t root = a.list[ti];
+        if (root < 0) continue;
+        uint32_t nint, nleaf, nlevel;
+        load_subtree(U, root, a.left, a.right, nint, nleaf, nlevel);
+        for (uint32_t i = lane; i < nleaf; i += 64u) {
+            float b[6];
+            const float* src = a.nboxes + 6 * ((uint64_t)a.n - 1 + (uint64_t)(-1 - U.code[kSubtree + i]));
+#pragma unroll
+            for (int k = 0; k < 6; ++k) b[k] = src[k];
+            leaf_cost[i] = box_valid(b) ? a.c_leaf * box_area(b) : -1.0f;
+        }
+        __syncthreads();
+        for (uint32_t lv = nlevel; lv-- > 0;) {
+            const uint32_t end = U.level[lv + 1];
+            for (uint32_t x = U.level[lv] + lane; x < end; x += 64u) {
+                const int32_t code = U.code[x];
+                float b[6];
+#pragma unroll
+                for (int k = 0; k < 6; ++k) b[k] = a.nboxes[6 * (uint64_t)code + k];
+                WideRow t[2];
+                uint32_t nl = 0;
+                const uint32_t kids = U.kids[x];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const uint32_t c = h ? kids >> 16 : kids & 0xFFFFu;
+                    if (c < kSubtree) {
+                        t[h] = row[c];
+                        nl += leaves[c];
+                    } else {
+                        const float lc = leaf_cost[c - kSubtree];
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) t[h].c[j] = lc < 0.0f ? 0.0f : lc;
+                        t[h].slots = lc < 0.0f ? 0ull : 0x0101010101010101ull;
+                        t[h].depth = 0;
+                        nl += lc < 0.0f ? 0u : 1u;
+                    }
+                }
+                WideRow o;
+                uint32_t below;
+                a.wdec[code] = wide_merge(t[0], t[1], box_area(b), box_valid(b), a.width, o, below);
+                a.sub[code] = below | (1u + below - nl) << 8 | ((uint32_t)o.depth & 255u) << 16;
+                row[x] = o;
+                leaves[x] = (uint8_t)nl;
+                if (x == 0) {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) a.wc[8 * (uint64_t)code + j] = o.c[j];
+                    a.depths[code] = o.depth;
+                }
+            }
+            __syncthreads();
+        }
     }
 }
 
-// D(x, j) from the children's tables: the least cost and the left child's slot count k.
-__device__ __forceinline__ float wide_split(const float* tl, const float* tr, int j, int& best_k) {
-    float best = INFINITY;
-    best_k = 1;
-    for (int k = 1; k < j; ++k) {
-        const float c = tl[k - 1] + tr[j - k - 1];
-        if (c < best) {
-            best = c;
-            best_k = k;
+__global__ __launch_bounds__(64) void wide_cost_kernel(CostArgs a) {
+    const uint32_t count = *a.count;
+    auto load_row = [&](int32_t c, WideRow& t) {
+        if (c < 0) {
+            float b[6];
+            const uint64_t bi = node_index(a.n, c);
+#pragma unroll
+            for (int k = 0; k < 6; ++k) b[k] = a.nboxes[6 * bi + k];
+            wide_leaf(b, a.c_leaf, t);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) t.c[j] = load_coherent(a.wc + 8 * (uint64_t)c + j);
+            t.depth = __hip_atomic_load(a.depths + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        t.slots = 0;
+    };
+    for (uint32_t at = blockIdx.x * 64u + threadIdx.x; at < count; at += gridDim.x * 64u) {
+        int32_t node = a.parent[node_index(a.n, a.list[at])];
+        while (node >= 0) {
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            __builtin_amdgcn_s_waitcnt(0);
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            const uint32_t old =
+                __hip_atomic_fetch_add(&a.arrivals[node], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (old == 0u) break;  // the sibling's thread merges
+            WideRow l, r, o;
+            load_row(a.left[node], l);
+            load_row(a.right[node], r);
+            float b[6];
+#pragma unroll
+            for (int k = 0; k < 6; ++k) b[k] = a.nboxes[6 * (uint64_t)node + k];
+            uint32_t below;
+            a.wdec[node] = wide_merge(l, r, box_area(b), box_valid(b), a.width, o, below);  // read by later launches
+#pragma unroll
+            for (int j = 0; j < 8; ++j) store_coherent(a.wc + 8 * (uint64_t)node + j, o.c[j]);
+            __hip_atomic_store(a.depths + node, o.depth, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            node = a.parent[node];
         }
     }
-    return best;
 }
 
-__global__ __launch_bounds__(256) void wide_cost_kernel(uint32_t n, const int32_t* __restrict__ left,
-                                                        const int32_t* __restrict__ right,
-                                                        const int32_t* __restrict__ parent, const float* nboxes,
-                                                        float* wc, uint32_t* __restrict__ wdec, uint32_t* arrivals,
-                                                        float c_leaf, int width) {
-    const uint32_t pos = blockIdx.x * blockDim.x + threadIdx.x;
-    if (pos >= n) return;
-    int32_t node = load_coherent_i32(parent + (uint64_t)n - 1 + pos);
-    while (node >= 0) {
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        __builtin_amdgcn_s_waitcnt(0);
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        const uint32_t old =
-            __hip_atomic_fetch_add(&arrivals[node], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (old == 0u) return;  // the sibling's thread merges
-        float tl[8], tr[8], b[6];
-        wide_table(n, load_coherent_i32(left + node), nboxes, wc, c_leaf, tl);
-        wide_table(n, load_coherent_i32(right + node), nboxes, wc, c_leaf, tr);
-#pragma unroll
-        for (int k = 0; k < 6; ++k) b[k] = load_coherent(nboxes + 6 * (uint64_t)node + k);
-        float c[8];
-        int k;
-        c[0] = box_area(b) + wide_split(tl, tr, width, k);
-        uint32_t dec = 0;
-        for (int j = 2; j <= 8; ++j) {
-            const float d = wide_split(tl, tr, j, k);
-            dec |= ((uint32_t)k | (d < c[j - 2] ? 8u : 0u)) << (4 * (j - 2));
-            c[j - 1] = fminf(c[j - 2], d);
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) store_coherent(wc + 8 * (uint64_t)node + j, c[j]);
-        wdec[node] = dec;  // read by later launches only
-        node = load_coherent_i32(parent + node);
+// ---- collapse tasks ---------------------------------------------------------------------------------------------
+//
+// The wide nodes above the listed subtrees go through a queue: a task is (binary node, slot) in one 64-bit word, its
+// place empty (kNoTask) until it is published.  `open` counts the tasks published and not yet done.  The subtrees
+// below come in a second list, each with the place of its slots.
+struct CollapseQueue {
+    uint32_t head, pad0[31];
+    uint32_t tail, pad1[31];
+    uint32_t open, pad2[31];
+    uint32_t subs, pad3[31];
+};
+static_assert(sizeof(CollapseQueue) == 512, "the scratch layout's queue words");
+__device__ __forceinline__ uint64_t pack_task(int32_t node, uint32_t slot) { return (uint32_t)node | (uint64_t)slot << 32; }
+
+// Root of a structure (header fields set, slot 0): its subtree task or its queue task, and what the header says of it.
+__device__ void push_root(AsHeader* h, int32_t root, uint32_t blas, const uint32_t* cnt, const uint32_t* sub,
+                          const uint64_t* depths, CollapseQueue* q, uint64_t* queue, uint4* subs) {
+    if (root < 0 || cnt[root] <= kSubtree) {
+        const uint32_t w = root < 0 ? 1u | 1u << 8 | 1u << 16 : sub[root];
+        h->slot_count = 1u + (w & 255u);
+        h->node_count = w >> 8 & 255u;
+        h->max_depth = w >> 16 & 255u;
+        subs[atomicAdd(&q->subs, 1u)] = make_uint4((uint32_t)root, 0u, 1u, blas);
+        return;
     }
+    h->slot_count = 1u;
+    h->max_depth = (uint32_t)depths[root] & 255u;
+    atomicAdd(&q->open, 1u);
+    queue[atomicAdd(&q->tail, 1u)] = pack_task(root, 0u);
 }
 
 // Header setup after refit: root box and the 16-bit origin quantisation step.
 __global__ void header_kernel(AsHeader* h, uint32_t type, uint32_t flags, uint32_t n, uint32_t ngeom,
                               const float* nboxes, const float* cost, uint64_t capacity_slots, uint64_t table_offset,
-                              uint32_t* level_counts, uint2* tasks0) {
+                              const uint32_t* cnt, const uint32_t* sub, const uint64_t* depths, CollapseQueue* q,
+                              uint64_t* queue, uint4* subs) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    q->head = q->tail = q->open = q->subs = 0;
     h->magic = type ? kMagicTlas : kMagicBlas;
     h->version = kVersion;
     h->type = type;
@@ -1394,14 +1559,9 @@ __global__ void header_kernel(AsHeader* h, uint32_t type, uint32_t flags, uint32
         h->qscale[a] = ext > 0.0f ? ext / 65535.0f : 0.0f;
     }
     h->lo[3] = h->hi[3] = h->qscale[3] = 0.0f;
-    if (empty) {
-        level_counts[0] = 0;
-        return;
-    }
-    h->slot_count = 1;  // slot 0 = root
-    level_counts[0] = 1;
-    // root task: BVH2 root is internal node 0, or leaf 0 (encoded -1) when n == 1
-    tasks0[0] = make_uint2(n == 1 ? 0xFFFFFFFFu : 0u, 0u);
+    if (empty) return;
+    // root: internal node 0, or leaf 0 (code -1) when n == 1
+    push_root(h, n == 1 ? -1 : 0, 0u, cnt, sub, depths, q, queue, subs);
 }
 
 __device__ __forceinline__ float exp_scale(uint32_t e) { return __uint_as_float(e << 23); }
@@ -1445,253 +1605,423 @@ __device__ __forceinline__ void quant_child(float clo, float chi, float p, uint3
     qhi = (uint8_t)qh;
 }
 
-// atomicAdd(addr, val), val < 16, for the active lanes of a wave whose addresses may differ (batched builds: one
-// header per task): one atomic per distinct address, lanes of one address get consecutive ranges in lane order.
-// Prefixes come from ballots of val's four bit planes, so lanes that are not active contribute nothing.  Every
-// active lane of the wave must call it.
-__device__ __forceinline__ uint32_t grouped_atomic_add(uint32_t* addr, uint32_t val) {
-    const uint32_t lane = __lane_id();
-    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    const unsigned long long a = (unsigned long long)(uintptr_t)addr;
-    uint64_t todo = __ballot(1);
-    uint32_t out = 0;
-    while (todo) {
-        const int leader = __ffsll((unsigned long long)todo) - 1;
-        const unsigned long long la = __shfl(a, leader);
-        const bool mine = a == la;
-        uint32_t prefix = 0, total = 0;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const uint64_t m = __ballot(mine && ((val >> b) & 1u));
-            prefix += (uint32_t)__popcll(m & below) << b;
-            total += (uint32_t)__popcll(m) << b;
-        }
-        uint32_t base = 0;
-        if ((int)lane == leader) base = atomicAdd(addr, total);
-        base = __shfl(base, leader);
-        if (mine) out = base + prefix;
-        todo &= ~__ballot(mine);
-    }
-    return out;
+// ---- wide nodes ---------------------------------------------------------------------------------------------------
+//
+// A wave makes 8 wide nodes at a time, 8 lanes each, a lane per child slot: it finds the children (collapse_walk), gives
+// them their octant positions and slots, quantises their boxes and writes the node and its leaves.  A launch per level of
+// the wide tree with a thread per node, 66 launches for the deepest tree there can be, took 1.75 ms on 4M triangles and
+// 7.0 ms on 15.5M of 64 meshes: most of it a dozen atomics per wave on the same few header words.  Through the queue and
+// by subtrees, whose slots are known beforehand, 0.20 + 0.77 ms and 0.6 + 4.4 ms.  The subtrees are bound by VALU
+// (65% busy: 8-lane placement and IEEE divisions of the quantisation).
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
 }
-
-// atomicMax(addr, val) with a wave-uniform val, one atomic per distinct address of the active lanes.
-__device__ __forceinline__ void grouped_atomic_max(uint32_t* addr, uint32_t val) {
-    const unsigned long long a = (unsigned long long)(uintptr_t)addr;
-    uint64_t todo = __ballot(1);
-    while (todo) {
-        const int leader = __ffsll((unsigned long long)todo) - 1;
-        const unsigned long long la = __shfl(a, leader);
-        const uint64_t grp = __ballot(a == la) & todo;
-        if ((int)__lane_id() == leader) atomicMax(addr, val);
-        todo &= ~grp;
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_u(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
+}
+// lane patterns that reduce over 8 lanes: quad_perm [1, 0, 3, 2], [2, 3, 0, 1], then row_half_mirror
+constexpr int kSwap1 = 0xB1, kSwap2 = 0x4E, kMirror8 = 0x141;
+__device__ __forceinline__ float min8(float v) {
+    v = fminf(v, dpp_f<kSwap1>(v));
+    v = fminf(v, dpp_f<kSwap2>(v));
+    return fminf(v, dpp_f<kMirror8>(v));
+}
+__device__ __forceinline__ float max8(float v) {
+    v = fmaxf(v, dpp_f<kSwap1>(v));
+    v = fmaxf(v, dpp_f<kSwap2>(v));
+    return fmaxf(v, dpp_f<kMirror8>(v));
+}
+template <int CTRL>
+__device__ __forceinline__ void best8_step(float& score, uint32_t& id) {
+    const float os = dpp_f<CTRL>(score);
+    const uint32_t oi = dpp_u<CTRL>(id);
+    if (os > score || (os == score && oi >> 3 > id >> 3)) {
+        score = os;
+        id = oi;
     }
 }
 
-// One collapse level.  Task = (BVH2 node code, destination slot); a negative node code is a leaf that is the
-// root itself (one-primitive structure).  Batched builds (BATCHED, as_ptr) carry each task's BLAS in a parallel
-// array and write into that BLAS's structure.  Single builds keep the header pointer a kernel argument: the
-// per-node atomics on it then have a wave-uniform address, which the compiler combines into one atomic per wave
-// (a per-task pointer would send 64 times as many atomics to the same few words).
-template <bool BATCHED>
-__global__ __launch_bounds__(256) void collapse_level_kernel(uint32_t n, const int32_t* __restrict__ left,
-                                                             const int32_t* __restrict__ right,
-                                                             const uint32_t* __restrict__ order,
-                                                             const float* __restrict__ nboxes,
-                                                             const uint4* __restrict__ leaf_src,
-                                                             AsHeader* __restrict__ h1, uint4* __restrict__ slots1,
-                                                             uint32_t* __restrict__ level_counts, int level,
-                                                             const uint2* __restrict__ tasks_in,
-                                                             uint2* __restrict__ tasks_out,
-                                                             AsHeader* const* __restrict__ as_ptr,
-                                                             const uint32_t* __restrict__ tblas_in,
-                                                             uint32_t* __restrict__ tblas_out,
-                                                             const uint32_t* __restrict__ wdec, int width) {
-    const uint32_t count = level_counts[level];
-    if (count == 0) return;
-    for (uint32_t ti = blockIdx.x * blockDim.x + threadIdx.x; ti < count; ti += gridDim.x * blockDim.x) {
-        uint2 task = tasks_in[ti];
-        const uint32_t tb = BATCHED ? tblas_in[ti] : 0u;
-        AsHeader* h = BATCHED ? as_ptr[tb] : h1;
-        uint4* slots = BATCHED ? (uint4*)((uint8_t*)h + kHeaderBytes) : slots1;
-        const float rlo[3] = {h->lo[0], h->lo[1], h->lo[2]};
-        const float qs[3] = {h->qscale[0], h->qscale[1], h->qscale[2]};
-        int32_t ch[8];
-        int cnt;
-        if ((int32_t)task.x < 0) {
-            ch[0] = (int32_t)task.x;
-            cnt = 1;
-        } else if (wdec) {
-            // the children D(task, W) picks: a stack of (subtree, slots) pairs whose slots add up to W; each visited
-            // node's split and "fewer slots" choices for every slot count come from the cost pass (wdec)
-            int32_t sn[8];
-            int si[8];
-            int sp = 0;
-            sn[sp] = (int32_t)task.x;
-            si[sp++] = width;
-            bool root = true;  // the task node itself is always split
-            cnt = 0;
-            while (sp > 0) {
-                --sp;
-                const int32_t x = sn[sp];
-                const int j = si[sp];
-                if (x < 0 || (j == 1 && !root)) {
-                    ch[cnt++] = x;
-                    continue;
-                }
-                const int32_t l = left[x], r = right[x];
-                const uint32_t dj = wdec[x] >> (4 * (j - 2));
-                const int k = (int)(dj & 7u);
-                if (!root && !(dj & 8u)) {
-                    sn[sp] = x;  // fewer slots cost no more
-                    si[sp++] = j - 1;
-                } else {
-                    sn[sp] = l;
-                    si[sp++] = k;
-                    sn[sp] = r;
-                    si[sp++] = j - k;
-                }
-                root = false;
-            }
-        } else {
-            ch[0] = left[task.x];
-            ch[1] = right[task.x];
-            cnt = 2;
+struct WideLds {
+    uint32_t item[8][8];   // a lane's part of the wide node being dissolved, and its slots
+    uint32_t slots[8][8];
+    alignas(16) uint8_t node[8][64];
+};
+
+// The children D(x, W) picks for the node x of each group (`on`), a child per lane (item; kNoItem: none).  A lane's part
+// takes the slots from its own on: a part dissolved over j slots leaves its left child, which takes k of them, in the
+// lane, and its right child k lanes on.  parts(x, l, r, dec): children and choices of an internal part, false for a leaf.
+constexpr uint32_t kNoItem = 0x80000000u;  // no local id and no code: leaf codes start at -(2^30 - 1)
+template <typename Parts>
+__device__ __forceinline__ uint32_t collapse_walk(WideLds& W, uint32_t x, bool on, uint32_t width, Parts parts) {
+    const uint32_t g = threadIdx.x >> 3, c = threadIdx.x & 7u;
+    W.item[g][c] = on && c == 0 ? x : kNoItem;
+    W.slots[g][c] = width;
+    __syncthreads();
+    bool root = true;
+    for (bool more = true; more;) {
+        const uint32_t it = W.item[g][c];
+        uint32_t j = W.slots[g][c];
+        bool split = false;
+        uint32_t l = 0, r = 0, dec = 0, k = 0;
+        if (it != kNoItem && (root || j > 1u) && parts(it, l, r, dec)) {
+            // fewer slots cost no more: take one less (the node itself is always dissolved)
+            while (!root && j > 1u && !(dec >> (4u * (j - 2u)) & 8u)) --j;
+            split = j > 1u;
+            if (split) k = dec >> (4u * (j - 2u)) & 7u;
         }
-        // greedy (no cost table): open the internal child with the largest surface area until W children
-        while (!wdec && cnt < width) {
-            int best = -1;
-            float best_a = -1.0f;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                if (j < cnt && ch[j] >= 0) {
-                    float a = box_area(nboxes + 6 * (uint64_t)ch[j]);
-                    if (a > best_a) {
-                        best_a = a;
-                        best = j;
-                    }
-                }
-            }
-            if (best < 0) break;
-            int32_t c = 0;
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (j == best) c = ch[j];
-            int32_t l = left[c], r = right[c];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                if (j == best) ch[j] = l;
-                if (j == cnt) ch[j] = r;
-            }
-            ++cnt;
+        __syncthreads();
+        if (split) {
+            W.item[g][c] = l;
+            W.slots[g][c] = k;
+            W.item[g][c + k] = r;
+            W.slots[g][c + k] = j - k;
+        } else if (it != kNoItem) {
+            W.slots[g][c] = 1u;
         }
-        // child boxes; drop empty ones
-        float cb[8][6];
-        bool cv[8];
-        float nlo[3] = {INFINITY, INFINITY, INFINITY}, nhi[3] = {-INFINITY, -INFINITY, -INFINITY};
+        __syncthreads();
+        root = false;
+        more = __any(split);
+    }
+    return W.item[g][c];
+}
+
+// Octant positions of the valid children (greedy assignment by centroid direction: the best (child, position) pair
+// first, the higher lane of equal ones) and the box of the node.
+__device__ __forceinline__ void place_children(bool valid, const float* b, uint32_t& pos, uint32_t& used, float* nlo,
+                                               float* nhi) {
+    const uint32_t g = threadIdx.x >> 3, c = threadIdx.x & 7u;
+    float d[3];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            cv[j] = false;
-            if (j < cnt) {
-                int32_t c = ch[j];
-                uint64_t bi = c >= 0 ? (uint64_t)c : (uint64_t)n - 1 + (uint64_t)(-1 - c);
+    for (int a = 0; a < 3; ++a) {
+        nlo[a] = min8(valid ? b[a] : INFINITY);
+        nhi[a] = max8(valid ? b[3 + a] : -INFINITY);
+        d[a] = 0.5f * (b[a] + b[3 + a]) - 0.5f * (nlo[a] + nhi[a]);
+    }
+    float sc[8];
 #pragma unroll
-                for (int k = 0; k < 6; ++k) cb[j][k] = nboxes[6 * bi + k];
-                cv[j] = cb[j][0] <= cb[j][3] && cb[j][1] <= cb[j][4] && cb[j][2] <= cb[j][5];
-                if (cv[j]) {
+    for (int p = 0; p < 8; ++p) sc[p] = ((p & 1) ? d[0] : -d[0]) + ((p & 2) ? d[1] : -d[1]) + ((p & 4) ? d[2] : -d[2]);
+    pos = 8;
+    used = 0;
+    for (;;) {
+        float best = -INFINITY;
+        uint32_t id = c << 3;
+        if (valid && pos == 8u) {
 #pragma unroll
-                    for (int a = 0; a < 3; ++a) {
-                        nlo[a] = fminf(nlo[a], cb[j][a]);
-                        nhi[a] = fmaxf(nhi[a], cb[j][3 + a]);
-                    }
+            for (uint32_t p = 0; p < 8; ++p)
+                if (!(used & (1u << p)) && sc[p] > best) {
+                    best = sc[p];
+                    id = c << 3 | p;
                 }
-            }
         }
-        // octant placement: greedy assignment of children to positions by centroid direction
-        int pos_of[8];
-        uint32_t used = 0;
-        float nc[3] = {0.5f * (nlo[0] + nhi[0]), 0.5f * (nlo[1] + nhi[1]), 0.5f * (nlo[2] + nhi[2])};
-#pragma unroll
-        for (int j = 0; j < 8; ++j) pos_of[j] = -1;
-        for (int it = 0; it < 8; ++it) {
-            float best = -INFINITY;
-            int bj = -1, bp = -1;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                if (!cv[j] || pos_of[j] >= 0) continue;
-                float dx = 0.5f * (cb[j][0] + cb[j][3]) - nc[0];
-                float dy = 0.5f * (cb[j][1] + cb[j][4]) - nc[1];
-                float dz = 0.5f * (cb[j][2] + cb[j][5]) - nc[2];
-#pragma unroll
-                for (int p = 0; p < 8; ++p) {
-                    if (used & (1u << p)) continue;
-                    float sc = ((p & 1) ? dx : -dx) + ((p & 2) ? dy : -dy) + ((p & 4) ? dz : -dz);
-                    if (sc > best) {
-                        best = sc;
-                        bj = j;
-                        bp = p;
-                    }
-                }
-            }
-            if (bj < 0) break;
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (j == bj) pos_of[j] = bp;
-            used |= 1u << bp;
+        best8_step<kSwap1>(best, id);
+        best8_step<kSwap2>(best, id);
+        best8_step<kMirror8>(best, id);
+        const bool found = best > -INFINITY;
+        if (!__any(found)) break;
+        if (found) {
+            if (c == id >> 3) pos = id & 7u;
+            used |= 1u << (id & 7u);
         }
-        // node frame; the 64-B node is assembled in registers (child bytes placed by shifts: a per-child byte
-        // index into a local array would put the node in private memory)
-        float p[3];
-        uint32_t e[3];
-        uint16_t pq[3];
+    }
+    // children whose centroid overflows have no direction: the free positions in order
+    for (uint64_t left; (left = __ballot(valid && pos == 8u)) != 0ull;) {
+        const uint32_t m = (uint32_t)(left >> (8u * g)) & 255u;
+        const uint32_t free = (uint32_t)__ffs((int)(~used & 255u)) - 1u;
+        if (m) {
+            if (c == (uint32_t)__ffs((int)m) - 1u) pos = free;
+            used |= 1u << free;
+        }
+    }
+}
+
+// Quantises the children of each group and writes its node to slots[4 slot ..] (on), child slots from `base`.
+__device__ __forceinline__ void write_node(WideLds& W, bool on, uint4* slots, uint32_t slot, uint32_t base, bool valid,
+                                           const float* b, uint32_t pos, uint32_t used, bool internal, const float* nlo,
+                                           const float* nhi, const float* rlo, const float* qs) {
+    const uint32_t g = threadIdx.x >> 3, c = threadIdx.x & 7u;
+    float p[3];
+    uint32_t e[3];
+    uint16_t pq[3];
+    if (on) {
 #pragma unroll
         for (int a = 0; a < 3; ++a) make_frame(nlo[a], nhi[a], rlo[a], qs[a], pq[a], p[a], e[a]);
-        uint64_t qlo[3] = {0, 0, 0}, qhi[3] = {0, 0, 0};
-        uint32_t imask = 0;
-        const uint32_t nvalid = (uint32_t)__popc(used);
-        const uint32_t base = BATCHED ? grouped_atomic_add(&h->slot_count, nvalid) : atomicAdd(&h->slot_count, nvalid);
+    }
+    *(uint64_t*)(W.node[g] + 8u * c) = 0ull;
+    __syncthreads();
+    uint32_t im = valid && internal ? 1u << pos : 0u;
+    im |= dpp_u<kSwap1>(im);
+    im |= dpp_u<kSwap2>(im);
+    im |= dpp_u<kMirror8>(im);
+    if (valid) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            if (!cv[j]) continue;
-            int k = pos_of[j];
+        for (int a = 0; a < 3; ++a) {
+            uint8_t ql, qh;
+            quant_child(b[a], b[3 + a], p[a], e[a], ql, qh);
+            W.node[g][16 + 8 * a + pos] = ql;
+            W.node[g][40 + 8 * a + pos] = qh;
+        }
+    }
+    __syncthreads();
+    // Node8 layout: pq[3] (bytes 0-5), e[3] (6-8), imask (9), vmask (10), pad (11), base (12-15),
+    // qlo[3][8] (16-39), qhi[3][8] (40-63)
+    if (on && c < 4u) {
+        uint4 w = *(const uint4*)(W.node[g] + 16u * c);
+        if (c == 0)
+            w = make_uint4((uint32_t)pq[0] | (uint32_t)pq[1] << 16, (uint32_t)pq[2] | e[0] << 16 | e[1] << 24,
+                           e[2] | im << 8 | used << 16, base);
+        slots[4 * (uint64_t)slot + c] = w;
+    }
+    __syncthreads();
+}
+
+__device__ __forceinline__ void copy_leaf(uint4* slots, uint32_t slot, const uint4* __restrict__ leaf_src, uint32_t prim) {
+    const uint4* src = leaf_src + 4 * (uint64_t)prim;
+    uint4* dst = slots + 4 * (uint64_t)slot;
+    const uint4 w0 = src[0], w1 = src[1], w2 = src[2], w3 = src[3];
+    dst[0] = w0;
+    dst[1] = w1;
+    dst[2] = w2;
+    dst[3] = w3;
+}
+
+struct CollapseArgs {
+    uint32_t n;
+    const int32_t* left;
+    const int32_t* right;
+    const uint32_t* order;
+    const float* nboxes;
+    const uint4* leaf_src;
+    const uint32_t* cnt;
+    const uint32_t* wdec;
+    const uint32_t* sub;
+    AsHeader* h;                // single builds
+    AsHeader* const* as_ptr;    // batched builds
+    const uint32_t* node_blas;
+    CollapseQueue* q;
+    uint64_t* queue;
+    const uint32_t* queue_size;
+    uint4* subs;
+    uint32_t* err;
+    uint32_t width;
+};
+
+__device__ __forceinline__ void node_box(const CollapseArgs& a, int32_t code, float* b) {
+    const float* src = a.nboxes + 6 * node_index(a.n, code);
 #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                uint8_t ql, qh;
-                quant_child(cb[j][a], cb[j][3 + a], p[a], e[a], ql, qh);
-                qlo[a] |= (uint64_t)ql << (8 * k);
-                qhi[a] |= (uint64_t)qh << (8 * k);
+    for (int k = 0; k < 6; ++k) b[k] = src[k];
+}
+
+// The wide nodes above the subtrees.  Waves of 8 groups; a group holds a ticket of the queue and works on the task of
+// that place once it is published.  A wave never waits while it has a task, and a place that stays empty belongs to a
+// node that a running wave is still about to reach, or to none (open = 0), so the waits end; a bound on them
+// (kQueueSpins) turns a mistake into an error flag.
+constexpr uint32_t kQueueSpins = 1u << 20;
+template <bool BATCHED>
+__global__ __launch_bounds__(64) void collapse_top_kernel(CollapseArgs a) {
+    __shared__ WideLds W;
+    const uint32_t lane = threadIdx.x, g = lane >> 3, c = lane & 7u;
+    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    const uint32_t limit = *a.queue_size;
+    if (limit == 0) return;
+    uint32_t ticket = kNoItem;
+    uint32_t nodes = 0, spins = 0;
+    auto parts = [&](uint32_t x, uint32_t& l, uint32_t& r, uint32_t& dec) {
+        if ((int32_t)x < 0) return false;
+        l = (uint32_t)a.left[x];
+        r = (uint32_t)a.right[x];
+        dec = a.wdec[x];
+        return true;
+    };
+    for (;;) {
+        // a ticket for each group without one
+        const uint64_t none = __ballot(ticket == kNoItem && c == 0);
+        if (none) {
+            uint32_t t = 0;
+            if (lane == 0) t = atomicAdd(&a.q->head, (uint32_t)__popcll(none));
+            t = __shfl(t, 0);
+            if (ticket == kNoItem) ticket = t + (uint32_t)__popcll(none & ((1ull << (8u * g)) - 1ull));
+        }
+        const uint32_t open = __hip_atomic_load(&a.q->open, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint64_t task = ticket < limit
+                                  ? __hip_atomic_load(a.queue + ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                  : kNoTask;
+        const bool on = task != kNoTask;
+        const uint64_t onm = __ballot(on && c == 0);
+        if (!onm) {
+            if (__shfl(open, 0) == 0u) break;
+            if (++spins > kQueueSpins) {
+                if (lane == 0) atomicOr(a.err, kErrBuildDepth);
+                break;
             }
-            uint32_t slot = base + (uint32_t)__popc(used & ((1u << k) - 1u));
-            int32_t c = ch[j];
-            if (c >= 0) {
-                imask |= 1u << k;
-                uint32_t o = atomicAdd(&level_counts[level + 1], 1u);
-                tasks_out[o] = make_uint2((uint32_t)c, slot);
-                if (BATCHED) tblas_out[o] = tb;
-            } else {
-                uint32_t prim = order[-1 - c];
-                const uint4* src = leaf_src + 4 * (uint64_t)prim;
-                uint4* dst = slots + 4 * (uint64_t)slot;
-                dst[0] = src[0];
-                dst[1] = src[1];
-                dst[2] = src[2];
-                dst[3] = src[3];
+            __builtin_amdgcn_s_sleep(4);
+            continue;
+        }
+        spins = 0;
+        const uint32_t x = (uint32_t)task, slot = (uint32_t)(task >> 32);
+        const uint32_t blas = BATCHED && on ? a.node_blas[x] : 0u;
+        AsHeader* h = BATCHED ? (on ? a.as_ptr[blas] : nullptr) : a.h;
+        uint4* slots = (uint4*)((uint8_t*)h + kHeaderBytes);
+        const uint32_t item = collapse_walk(W, x, on, a.width, parts);
+        const int32_t code = (int32_t)item;
+        float b[6] = {0, 0, 0, 0, 0, 0}, rlo[3] = {0, 0, 0}, qs[3] = {0, 0, 0};
+        const bool child = on && item != kNoItem;
+        bool valid = false;
+        if (child) {
+            node_box(a, code, b);
+            valid = box_valid(b);
+        }
+        if (on) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                rlo[k] = h->lo[k];
+                qs[k] = h->qscale[k];
             }
         }
-        // Node8 layout: pq[3] (bytes 0-5), e[3] (6-8), imask (9), vmask (10), pad (11), base (12-15),
-        // qlo[3][8] (16-39), qhi[3][8] (40-63)
-        uint4* ndst = slots + 4 * (uint64_t)task.y;
-        ndst[0] = make_uint4((uint32_t)pq[0] | (uint32_t)pq[1] << 16, (uint32_t)pq[2] | e[0] << 16 | e[1] << 24,
-                             e[2] | imask << 8 | used << 16, base);
-        ndst[1] = make_uint4((uint32_t)qlo[0], (uint32_t)(qlo[0] >> 32), (uint32_t)qlo[1], (uint32_t)(qlo[1] >> 32));
-        ndst[2] = make_uint4((uint32_t)qlo[2], (uint32_t)(qlo[2] >> 32), (uint32_t)qhi[0], (uint32_t)(qhi[0] >> 32));
-        ndst[3] = make_uint4((uint32_t)qhi[1], (uint32_t)(qhi[1] >> 32), (uint32_t)qhi[2], (uint32_t)(qhi[2] >> 32));
+        uint32_t pos, used;
+        float nlo[3], nhi[3];
+        place_children(valid, b, pos, used, nlo, nhi);
+        const bool internal = valid && code >= 0;
+        const bool small = internal && a.cnt[code] <= kSubtree;
+        const uint32_t w = small ? a.sub[code] : 0u;
+        const uint32_t size = w & 255u;  // slots below a subtree child
+        // slots: the group's children, then the subtrees below them
+        uint32_t run = size, wide = w >> 8 & 255u;
+#pragma unroll
+        for (int off = 1; off < 8; off <<= 1) {
+            const uint32_t v = __shfl_up(run, off, 8);
+            if ((int)c >= off) run += v;
+            wide += __shfl_xor(wide, off, 8);
+        }
+        const uint32_t nvalid = (uint32_t)__popc(used);
+        const uint32_t total = nvalid + __shfl(run, 7, 8);
+        uint32_t base = 0;
         if (BATCHED) {
-            grouped_atomic_add(&h->node_count, 1u);
-            grouped_atomic_max(&h->max_depth, (uint32_t)(level + 1));
+            if (on && c == 0) {
+                base = atomicAdd(&h->slot_count, total);
+                atomicAdd(&h->node_count, 1u + wide);
+            }
+            base = __shfl(base, 0, 8);
         } else {
-            atomicAdd(&h->node_count, 1u);
-            atomicMax(&h->max_depth, (uint32_t)(level + 1));
+            uint32_t before = 0, all = 0;
+            for (uint32_t k = 0; k < 8; ++k) {
+                const uint32_t v = __shfl(total, (int)(8 * k));
+                before += k < g ? v : 0u;
+                all += v;
+            }
+            if (lane == 0) base = atomicAdd(&h->slot_count, all);
+            base = __shfl(base, 0) + before;
+            nodes += on && c == 0 ? 1u + wide : 0u;
+        }
+        write_node(W, on, slots, slot, base, valid, b, pos, used, internal, nlo, nhi, rlo, qs);
+        const uint32_t cslot = base + (uint32_t)__popc(used & ((1u << (pos & 7u)) - 1u));
+        if (valid && code < 0) copy_leaf(slots, cslot, a.leaf_src, a.order[-1 - code]);
+        const uint64_t sm = __ballot(small), tm = __ballot(internal && !small);
+        if (sm) {
+            uint32_t at = 0;
+            if (lane == 0) at = atomicAdd(&a.q->subs, (uint32_t)__popcll(sm));
+            at = __shfl(at, 0) + (uint32_t)__popcll(sm & below);
+            if (small) a.subs[at] = make_uint4((uint32_t)code, cslot, base + nvalid + run - size, blas);
+        }
+        if (tm) {
+            uint32_t at = 0;
+            if (lane == 0) {
+                // counted as open before anybody can see them
+                atomicAdd(&a.q->open, (uint32_t)__popcll(tm));
+                at = atomicAdd(&a.q->tail, (uint32_t)__popcll(tm));
+            }
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            __builtin_amdgcn_s_waitcnt(0);
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            at = __shfl(at, 0) + (uint32_t)__popcll(tm & below);
+            if (internal && !small)
+                __hip_atomic_store(a.queue + at, pack_task(code, cslot), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (lane == 0) atomicSub(&a.q->open, (uint32_t)__popcll(onm));
+        if (on) ticket = kNoItem;
+    }
+    if (!BATCHED) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) nodes += __shfl_xor(nodes, off);
+        if (lane == 0 && nodes) atomicAdd(&a.h->node_count, nodes);
+    }
+}
+
+// The wide nodes of the listed subtrees, a wave each, breadth-first into the slots that the subtree was given.
+template <bool BATCHED>
+__global__ __launch_bounds__(64) void collapse_subtree_kernel(CollapseArgs a) {
+    __shared__ SubtreeLds U;
+    __shared__ WideLds W;
+    __shared__ uint32_t udec[kSubtree];
+    __shared__ uint32_t qslot[kSubtree];
+    __shared__ uint16_t qnode[kSubtree];
+    const uint32_t lane = threadIdx.x, g = lane >> 3;
+    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    const uint32_t count = a.q->subs;
+    auto parts = [&](uint32_t x, uint32_t& l, uint32_t& r, uint32_t& dec) {
+        if (x >= kSubtree) return false;
+        l = U.kids[x] & 0xFFFFu;
+        r = U.kids[x] >> 16;
+        dec = udec[x];
+        return true;
+    };
+    for (uint32_t ti = blockIdx.x; ti < count; ti += gridDim.x) {
+        const uint4 task = a.subs[ti];
+        AsHeader* h = BATCHED ? a.as_ptr[task.w] : a.h;
+        uint4* slots = (uint4*)((uint8_t*)h + kHeaderBytes);
+        float rlo[3], qs[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            rlo[k] = h->lo[k];
+            qs[k] = h->qscale[k];
+        }
+        __syncthreads();
+        uint32_t nint = 1, nleaf, nlevel;
+        if ((int32_t)task.x < 0) {  // a structure of one primitive: a wide node with one child
+            if (lane == 0) {
+                U.code[kSubtree] = (int32_t)task.x;
+                qnode[0] = (uint16_t)kSubtree;
+            }
+        } else {
+            load_subtree(U, (int32_t)task.x, a.left, a.right, nint, nleaf, nlevel);
+            for (uint32_t i = lane; i < nint; i += 64u) udec[i] = a.wdec[U.code[i]];
+            if (lane == 0) qnode[0] = 0;
+        }
+        if (lane == 0) qslot[0] = task.y;
+        __syncthreads();
+        uint32_t head = 0, tail = 1, next = task.z;
+        while (head < tail) {
+            const bool on = head + g < tail;
+            const uint32_t x = on ? qnode[head + g] : 0u, slot = on ? qslot[head + g] : 0u;
+            const uint32_t item = collapse_walk(W, x, on, a.width, parts);
+            float b[6] = {0, 0, 0, 0, 0, 0};
+            bool valid = false;
+            int32_t code = 0;
+            if (on && item != kNoItem) {
+                code = U.code[item];
+                node_box(a, code, b);
+                valid = box_valid(b);
+            }
+            uint32_t pos, used;
+            float nlo[3], nhi[3];
+            place_children(valid, b, pos, used, nlo, nhi);
+            const uint64_t vm = __ballot(valid);
+            const uint32_t base = next + (uint32_t)__popcll(vm & ((1ull << (8u * g)) - 1ull));
+            next += (uint32_t)__popcll(vm);
+            const bool internal = valid && code >= 0;
+            write_node(W, on, slots, slot, base, valid, b, pos, used, internal, nlo, nhi, rlo, qs);
+            const uint32_t cslot = base + (uint32_t)__popc(used & ((1u << (pos & 7u)) - 1u));
+            if (valid && code < 0) copy_leaf(slots, cslot, a.leaf_src, a.order[-1 - code]);
+            const uint64_t im = __ballot(internal);
+            head = head + 8u < tail ? head + 8u : tail;
+            if (internal) {
+                const uint32_t at = tail + (uint32_t)__popcll(im & below);
+                qnode[at] = (uint16_t)item;
+                qslot[at] = cslot;
+            }
+            tail += (uint32_t)__popcll(im);
+            __syncthreads();
         }
     }
 }
@@ -1702,8 +2032,10 @@ __global__ __launch_bounds__(64) void batch_header_kernel(AsHeader* const* __res
                                                           const int32_t* __restrict__ roots, uint32_t n,
                                                           uint32_t flags, const float* __restrict__ nboxes,
                                                           const float* __restrict__ cost,
-                                                          uint32_t* __restrict__ level_counts,
-                                                          uint2* __restrict__ tasks0, uint32_t* __restrict__ tblas0) {
+                                                          const uint32_t* __restrict__ cnt,
+                                                          const uint32_t* __restrict__ sub,
+                                                          const uint64_t* __restrict__ depths, CollapseQueue* q,
+                                                          uint64_t* queue, uint4* subs) {
     const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= nbatch) return;
     AsHeader* h = as_ptr[b];
@@ -1752,10 +2084,7 @@ __global__ __launch_bounds__(64) void batch_header_kernel(AsHeader* const* __res
     }
     h->lo[3] = h->hi[3] = h->qscale[3] = 0.0f;
     if (empty) return;
-    h->slot_count = 1;
-    const uint32_t o = atomicAdd(&level_counts[0], 1u);
-    tasks0[o] = make_uint2((uint32_t)root, 0u);
-    tblas0[o] = b;
+    push_root(h, root, b, cnt, sub, depths, q, queue, subs);
 }
 
 __global__ void batch_finish_kernel(AsHeader* const* __restrict__ as_ptr, uint32_t nbatch) {
@@ -1766,14 +2095,6 @@ __global__ void batch_finish_kernel(AsHeader* const* __restrict__ as_ptr, uint32
 __global__ void fill_bounds_kernel(uint32_t* __restrict__ cb, uint32_t nbatch) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < 6 * nbatch) cb[i] = (i % 6) < 3 ? 0xFFFFFFFFu : 0u;
-}
-
-// Tasks left after the last enqueued level mean the binary tree was deeper than the level bound.
-__global__ void collapse_check_kernel(AsHeader* h, const uint32_t* level_counts, int max_levels, uint32_t* err) {
-    if (threadIdx.x == 0 && blockIdx.x == 0 && level_counts[max_levels] != 0u) {
-        if (h) h->build_error = 1u;
-        atomicOr(err, kErrBuildDepth);
-    }
 }
 
 __global__ void finish_tlas_kernel(AsHeader* h, const uint32_t* max_blas_depth) {
@@ -1816,9 +2137,14 @@ __global__ void arg_blob_kernel(ArgBlob b, uint32_t* __restrict__ dst, uint32_t 
 // ---- scratch layout --------------------------------------------------------------------------------------------
 struct Layout {
     uint64_t leaves, boxes, keys, vals, sort, left, right, parent, nboxes, arrivals, cost, cnt, hgt, wcost, wdec,
-        tasks0, tasks1, levels, cbounds, misc, geoms, total;
+        subs, queue, queue_words, cbounds, misc, geoms, total;
     // batched builds only
-    uint64_t pblas = 0, nblas = 0, roots = 0, asptr = 0, binfo = 0, tblas0 = 0, tblas1 = 0, bcb = 0;
+    uint64_t pblas = 0, nblas = 0, roots = 0, asptr = 0, binfo = 0, bcb = 0;
+    // space that is free again by the time of the bottom-up passes: subtree lists in the sort's scratch, sub words in
+    // the keys, depths in the primitive boxes (which the first pass reads)
+    uint64_t list() const { return sort; }
+    uint64_t sub() const { return keys; }
+    uint64_t depths() const { return boxes; }
 };
 
 Layout make_layout(uint32_t n, int key_bytes, uint32_t ngeom, uint32_t nbatch = 0) {
@@ -1845,9 +2171,9 @@ Layout make_layout(uint32_t n, int key_bytes, uint32_t ngeom, uint32_t nbatch = 
     L.hgt = take(nn * 4);
     L.wcost = take(nn * 32);
     L.wdec = take(nn * 4);
-    L.tasks0 = take(nn * 8);
-    L.tasks1 = take(nn * 8);
-    L.levels = take(128 * 4);
+    L.subs = take(nn * 8 + 16ull * (nbatch ? nbatch : 1));  // subtree tasks: of two primitives or more, or a whole BLAS
+    L.queue = take(nn * 8);
+    L.queue_words = take(sizeof(CollapseQueue));
     L.cbounds = take(8 * 4);
     L.misc = take(64);
     L.geoms = take((uint64_t)(ngeom ? ngeom : 1) * sizeof(GeomDesc));
@@ -1857,8 +2183,6 @@ Layout make_layout(uint32_t n, int key_bytes, uint32_t ngeom, uint32_t nbatch = 
         L.roots = take((uint64_t)nbatch * 4);
         L.asptr = take((uint64_t)nbatch * 8);
         L.binfo = take((uint64_t)nbatch * 8);
-        L.tblas0 = take(nn * 4);
-        L.tblas1 = take(nn * 4);
         L.bcb = take((uint64_t)nbatch * 24);
     }
     L.total = o;
@@ -1885,8 +2209,16 @@ __global__ void set_update_offset_kernel(AsHeader* h, uint64_t off) {
 constexpr float kLeafCostTri = 0.3f;
 constexpr float kLeafCostInstance = 1.0f;
 
-// Persistent one-wave blocks of the subtree passes.
-constexpr uint32_t kSubtreeBlocks = 4096;
+// One-wave blocks of the subtree passes (4M triangles: refinement 2.08 ms, collapse 1.13 ms with 4,096 blocks, which
+// share the subtrees out unevenly, 1.71 and 0.77 ms with 65,536), of the passes over the nodes above (whose waves take
+// several subtrees each: 0.57 ms with 4,096, 0.78 ms with 16,384), and of the collapse's queue.
+constexpr uint32_t kSubtreeBlocks = 65536;
+constexpr uint32_t kAboveBlocks = 4096;
+constexpr uint32_t kQueueBlocks = 512;
+
+// Counters of the bottom-up passes: subtrees listed for the refinement rounds and the costs, and the queue's places.
+constexpr uint32_t kPassCounts = 5;
+uint32_t* pass_counts(uint8_t* scratch, const Layout& L) { return (uint32_t*)(scratch + L.misc) + 8; }
 
 // counted: cnt holds the primitive counts of the internal nodes (written with the hierarchy).
 // Refit with treelet refinement; each further round restructures the tree the previous one left.  Then the costs
@@ -1917,33 +2249,82 @@ void refit_passes(uint32_t n, uint32_t flags, uint8_t* scratch, const Layout& L,
     a.node_blas = node_blas;
     a.list = nullptr;
     a.count = nullptr;
+    uint32_t* counts = pass_counts(scratch, L);
+    fill_kernel<<<1, 64, 0, s>>>(counts, kPassCounts, 0u);
+    const uint32_t few = n / 8 + 1;  // at most this many waves
+    // pass 0 .. 2: a refinement round; 3: the costs, with the collapse's queue
+    auto find = [&](int pass) {
+        find_subtrees_kernel<<<(n - 1) / kFindNodes + 1, 256, 0, s>>>(
+            n, a.left, a.right, a.cnt, arrivals, (int32_t*)(scratch + L.list()), counts + pass,
+            pass == 3 ? (uint64_t*)(scratch + L.queue) : nullptr, counts + 4);
+    };
     if (!counted) {
         if (n > 1) fill_kernel<<<256, 256, 0, s>>>(arrivals, n, 0u);
         a.min_prims = 0xFFFFFFFFu;
         refit_refine_kernel<<<(n + 63) / 64, 64, 0, s>>>(a);
     } else {
-        // the list of subtrees lies where the collapse keeps its tasks later
-        int32_t* list = (int32_t*)(scratch + L.tasks1);
-        uint32_t* counts = (uint32_t*)(scratch + L.misc) + 8;  // one word per round
-        fill_kernel<<<1, 64, 0, s>>>(counts, 4, 0u);
-        a.list = list;
+        a.list = (int32_t*)(scratch + L.list());
         for (int round = 0; round < (rounds ? rounds : 1); ++round) {
             a.count = counts + round;
             a.min_prims = rounds ? kTreeletMinPrims[round] : 0xFFFFFFFFu;
             if (round) a.prim_boxes = nullptr;
-            find_subtrees_kernel<<<(n - 1) / kFindNodes + 1, 256, 0, s>>>(n, a.left, a.right, a.cnt, arrivals, list,
-                                                                 counts + round);
-            const uint32_t few = n / 8 + 1;  // at most this many waves
+            find(round);
             subtree_refine_kernel<<<std::min(few, kSubtreeBlocks), 64, 0, s>>>(a);
-            if (n > kSubtree) refit_refine_kernel<<<std::min(few, kSubtreeBlocks), 64, 0, s>>>(a);
+            if (n > kSubtree) refit_refine_kernel<<<std::min(few, kAboveBlocks), 64, 0, s>>>(a);
         }
     }
     if (n > 1) {
-        fill_kernel<<<256, 256, 0, s>>>(arrivals, n, 0u);
-        wide_cost_kernel<<<(n + 255) / 256, 256, 0, s>>>(
-            n, (const int32_t*)(scratch + L.left), (const int32_t*)(scratch + L.right),
-            (const int32_t*)(scratch + L.parent), (const float*)(scratch + L.nboxes), (float*)(scratch + L.wcost),
-            (uint32_t*)(scratch + L.wdec), arrivals, c_leaf, node_width(flags));
+        find(3);
+        CostArgs c;
+        c.n = n;
+        c.left = a.left;
+        c.right = a.right;
+        c.parent = a.parent;
+        c.nboxes = a.nboxes;
+        c.wc = (float*)(scratch + L.wcost);
+        c.depths = (uint64_t*)(scratch + L.depths());
+        c.wdec = (uint32_t*)(scratch + L.wdec);
+        c.sub = (uint32_t*)(scratch + L.sub());
+        c.arrivals = arrivals;
+        c.c_leaf = c_leaf;
+        c.width = node_width(flags);
+        c.list = (const int32_t*)(scratch + L.list());
+        c.count = counts + 3;
+        subtree_cost_kernel<<<std::min(few, kSubtreeBlocks), 64, 0, s>>>(c);
+        if (n > kSubtree) wide_cost_kernel<<<std::min(n / 2048 + 1, kAboveBlocks), 64, 0, s>>>(c);
+    }
+}
+
+// The wide nodes of the structures whose roots the header kernel queued.
+void collapse_passes(uint32_t n, uint32_t flags, uint8_t* scratch, const Layout& L, AsHeader* h,
+                     AsHeader* const* as_ptr, const uint32_t* node_blas, uint32_t* err_flags, hipStream_t s) {
+    CollapseArgs a;
+    a.n = n;
+    a.left = (const int32_t*)(scratch + L.left);
+    a.right = (const int32_t*)(scratch + L.right);
+    a.order = (const uint32_t*)(scratch + L.vals);
+    a.nboxes = (const float*)(scratch + L.nboxes);
+    a.leaf_src = (const uint4*)(scratch + L.leaves);
+    a.cnt = (const uint32_t*)(scratch + L.cnt);
+    a.wdec = (const uint32_t*)(scratch + L.wdec);
+    a.sub = (const uint32_t*)(scratch + L.sub());
+    a.h = h;
+    a.as_ptr = as_ptr;
+    a.node_blas = node_blas;
+    a.q = (CollapseQueue*)(scratch + L.queue_words);
+    a.queue = (uint64_t*)(scratch + L.queue);
+    a.queue_size = pass_counts(scratch, L) + 4;
+    a.subs = (uint4*)(scratch + L.subs);
+    a.err = err_flags;
+    a.width = (uint32_t)node_width(flags);
+    const uint32_t top = std::min(n / 2048 + 1, kQueueBlocks);
+    const uint32_t sub = std::min(n / 8 + 1, kSubtreeBlocks);
+    if (as_ptr) {
+        if (n > kSubtree) collapse_top_kernel<true><<<top, 64, 0, s>>>(a);
+        collapse_subtree_kernel<true><<<sub, 64, 0, s>>>(a);
+    } else {
+        if (n > kSubtree) collapse_top_kernel<false><<<top, 64, 0, s>>>(a);
+        collapse_subtree_kernel<false><<<sub, 64, 0, s>>>(a);
     }
 }
 
@@ -1951,7 +2332,6 @@ void refit_passes(uint32_t n, uint32_t flags, uint8_t* scratch, const Layout& L,
 hipError_t lbvh_common(uint32_t n, bool k64, uint32_t type, uint32_t flags, uint32_t ngeom, uint8_t* scratch,
                        const Layout& L, uint8_t* dst, uint64_t table_offset, uint32_t* err_flags, hipStream_t s) {
     AsHeader* h = (AsHeader*)dst;
-    uint4* slots = (uint4*)(dst + kHeaderBytes);
     float* boxes = (float*)(scratch + L.boxes);
     uint32_t* cb = (uint32_t*)(scratch + L.cbounds);
     uint32_t* vals = (uint32_t*)(scratch + L.vals);
@@ -1960,9 +2340,6 @@ hipError_t lbvh_common(uint32_t n, bool k64, uint32_t type, uint32_t flags, uint
     int32_t* parent = (int32_t*)(scratch + L.parent);
     float* nboxes = (float*)(scratch + L.nboxes);
     float* cost = (float*)(scratch + L.cost);
-    uint32_t* levels = (uint32_t*)(scratch + L.levels);
-    uint2* t0 = (uint2*)(scratch + L.tasks0);
-    uint2* t1 = (uint2*)(scratch + L.tasks1);
     const unsigned gb = (unsigned)((n + 255) / 256);
     hipError_t err;
     if (n > 0) {
@@ -1987,22 +2364,12 @@ hipError_t lbvh_common(uint32_t n, bool k64, uint32_t type, uint32_t flags, uint
         }
         refit_passes(n, flags, scratch, L, boxes, s, nullptr, type == 1 ? kLeafCostInstance : kLeafCostTri);
     }
-    fill_kernel<<<1, 128, 0, s>>>(levels, 128, 0u);
     // root box: internal node 0, or the single leaf (stored at index n-1 == 0)
-    header_kernel<<<1, 64, 0, s>>>(h, type, flags, n, ngeom, nboxes, cost, 2ull * (n ? n : 1) + 1, table_offset, levels, t0);
-    if (n > 0) {
-        const int max_levels = k64 ? kMaxLevels64 : kMaxLevels32;
-        for (int lv = 0; lv < max_levels; ++lv) {
-            uint2* tin = (lv & 1) ? t1 : t0;
-            uint2* tout = (lv & 1) ? t0 : t1;
-            collapse_level_kernel<false><<<kCollapseBlocks, 256, 0, s>>>(n, left, right, vals, nboxes,
-                                                                  (const uint4*)(scratch + L.leaves), h, slots, levels,
-                                                                  lv, tin, tout, nullptr, nullptr, nullptr,
-                                                                  n > 1 ? (const uint32_t*)(scratch + L.wdec) : nullptr,
-                                                                  node_width(flags));
-        }
-        collapse_check_kernel<<<1, 64, 0, s>>>(h, levels, max_levels, err_flags);
-    }
+    header_kernel<<<1, 64, 0, s>>>(h, type, flags, n, ngeom, nboxes, cost, 2ull * (n ? n : 1) + 1, table_offset,
+                                   (const uint32_t*)(scratch + L.cnt), (const uint32_t*)(scratch + L.sub()),
+                                   (const uint64_t*)(scratch + L.depths()), (CollapseQueue*)(scratch + L.queue_words),
+                                   (uint64_t*)(scratch + L.queue), (uint4*)(scratch + L.subs));
+    if (n > 0) collapse_passes(n, flags, scratch, L, h, nullptr, nullptr, err_flags, s);
     return hipGetLastError();
 }
 
@@ -2177,24 +2544,12 @@ hipError_t update_blas(const GeomDesc* geoms_host, uint32_t ngeom, uint32_t n, u
             return err;
         refit_passes(n, flags | RTX_BUILD_NO_TREELET_BIT, sc, L, (const float*)(sc + L.boxes), s, nullptr, kLeafCostTri, false);
     }
-    uint32_t* levels = (uint32_t*)(sc + L.levels);
-    uint2* t0 = (uint2*)(sc + L.tasks0);
-    uint2* t1 = (uint2*)(sc + L.tasks1);
-    fill_kernel<<<1, 128, 0, s>>>(levels, 128, 0u);
     header_kernel<<<1, 64, 0, s>>>(h, 0, flags, n, ngeom, (const float*)(sc + L.nboxes), (const float*)(sc + L.cost),
-                                   2ull * (n ? n : 1) + 1, 0, levels, t0);
-    if (n > 0) {
-        for (int lv = 0; lv < kMaxLevels32; ++lv) {
-            uint2* tin = (lv & 1) ? t1 : t0;
-            uint2* tout = (lv & 1) ? t0 : t1;
-            collapse_level_kernel<false><<<kCollapseBlocks, 256, 0, s>>>(
-                n, (const int32_t*)(sc + L.left), (const int32_t*)(sc + L.right), (const uint32_t*)(sc + L.vals),
-                (const float*)(sc + L.nboxes), (const uint4*)(sc + L.leaves), h, (uint4*)((uint8_t*)dst + kHeaderBytes),
-                levels, lv, tin, tout, nullptr, nullptr, nullptr, n > 1 ? (const uint32_t*)(sc + L.wdec) : nullptr,
-                node_width(flags));
-        }
-        collapse_check_kernel<<<1, 64, 0, s>>>(h, levels, kMaxLevels32, err_flags);
-    }
+                                   2ull * (n ? n : 1) + 1, 0, (const uint32_t*)(sc + L.cnt),
+                                   (const uint32_t*)(sc + L.sub()), (const uint64_t*)(sc + L.depths()),
+                                   (CollapseQueue*)(sc + L.queue_words), (uint64_t*)(sc + L.queue),
+                                   (uint4*)(sc + L.subs));
+    if (n > 0) collapse_passes(n, flags, sc, L, h, nullptr, nullptr, err_flags, s);
     if (ngeom) content_kernel<<<(ngeom + 255) / 256, 256, 0, s>>>(gd, ngeom, h, nullptr);
     finish_blas_kernel<<<1, 64, 0, s>>>(h);
     set_update_offset_kernel<<<1, 64, 0, s>>>(h, off);
@@ -2249,7 +2604,6 @@ hipError_t build_blas_batch(const GeomDesc* geoms_host, uint32_t ngeom, const ui
     int32_t* parent = (int32_t*)(sc + L.parent);
     float* nboxes = (float*)(sc + L.nboxes);
     float* boxes = (float*)(sc + L.boxes);
-    uint32_t* levels = (uint32_t*)(sc + L.levels);
     const unsigned gb = (unsigned)((n + 255) / 256);
     fill_bounds_kernel<<<(6 * nbatch + 255) / 256, 256, 0, s>>>(cb, nbatch);
     fill_kernel<<<(nbatch + 255) / 256, 256, 0, s>>>((uint32_t*)roots, nbatch, 0x7FFFFFFFu);
@@ -2265,24 +2619,12 @@ hipError_t build_blas_batch(const GeomDesc* geoms_host, uint32_t ngeom, const ui
         blas_roots_kernel<<<(unsigned)((2ull * n - 1 + 255) / 256), 256, 0, s>>>(n, keys, parent, nblas, roots);
         refit_passes(n, flags, sc, L, boxes, s, n > 1 ? nblas : nullptr);
     }
-    fill_kernel<<<1, 128, 0, s>>>(levels, 128, 0u);
-    batch_header_kernel<<<(nbatch + 63) / 64, 64, 0, s>>>(as_ptr, binfo, nbatch, roots, n, flags, nboxes,
-                                                          (const float*)(sc + L.cost), levels,
-                                                          (uint2*)(sc + L.tasks0), (uint32_t*)(sc + L.tblas0));
-    if (n > 0) {
-        for (int lv = 0; lv < kMaxLevels32; ++lv) {
-            uint2* tin = (uint2*)(sc + ((lv & 1) ? L.tasks1 : L.tasks0));
-            uint2* tout = (uint2*)(sc + ((lv & 1) ? L.tasks0 : L.tasks1));
-            uint32_t* bin = (uint32_t*)(sc + ((lv & 1) ? L.tblas1 : L.tblas0));
-            uint32_t* bout = (uint32_t*)(sc + ((lv & 1) ? L.tblas0 : L.tblas1));
-            collapse_level_kernel<true><<<kCollapseBlocks, 256, 0, s>>>(n, left, right, vals, nboxes,
-                                                                  (const uint4*)(sc + L.leaves), nullptr, nullptr,
-                                                                  levels, lv, tin, tout, as_ptr, bin, bout,
-                                                                  n > 1 ? (const uint32_t*)(sc + L.wdec) : nullptr,
-                                                                  node_width(flags));
-        }
-        collapse_check_kernel<<<1, 64, 0, s>>>(nullptr, levels, kMaxLevels32, err_flags);
-    }
+    fill_kernel<<<1, 128, 0, s>>>((uint32_t*)(sc + L.queue_words), sizeof(CollapseQueue) / 4, 0u);
+    batch_header_kernel<<<(nbatch + 63) / 64, 64, 0, s>>>(
+        as_ptr, binfo, nbatch, roots, n, flags, nboxes, (const float*)(sc + L.cost), (const uint32_t*)(sc + L.cnt),
+        (const uint32_t*)(sc + L.sub()), (const uint64_t*)(sc + L.depths()), (CollapseQueue*)(sc + L.queue_words),
+        (uint64_t*)(sc + L.queue), (uint4*)(sc + L.subs));
+    if (n > 0) collapse_passes(n, flags, sc, L, nullptr, as_ptr, nblas, err_flags, s);
     if (ngeom) content_kernel<<<(ngeom + 255) / 256, 256, 0, s>>>(gd, ngeom, nullptr, as_ptr);
     batch_finish_kernel<<<(nbatch + 63) / 64, 64, 0, s>>>(as_ptr, nbatch);
     return hipGetLastError();

@@ -47,3 +47,84 @@ def test_refined_tree_bit_exact(ctx, n, shape):
             assert np.array_equal(left, el) and np.array_equal(right, er), (n, shape, bits, rounds)
             assert np.array_equal(height, eh)
             assert np.array_equal(cost, ec)
+
+
+def _check_structure(ctx, blas, n, width=8):
+    """Walks a built BLAS: every slot below slot_count reached once, every triangle once, the header's counts and depth,
+    and every child's decoded box around what lies below it."""
+    info = ctx.as_info(blas)
+    raw = blas.storage.cpu().numpy()
+    head = raw[:256]
+    lo, qs = head[48:60].view(np.float32), head[80:92].view(np.float32)
+    slots = raw[256:256 + 64 * info.slot_count].reshape(-1, 64)
+    seen = np.zeros(info.slot_count, bool)
+    prims, nodes, deepest = [], 0, 0
+    stack = [(0, 1, None)]
+    seen[0] = True
+    while stack:
+        at, depth, outer = stack.pop()
+        w = slots[at]
+        nodes += 1
+        deepest = max(deepest, depth)
+        pq, e, imask, vmask, base = w[:6].view(np.uint16), w[6:9], int(w[9]), int(w[10]), int(w[12:16].view(np.uint32)[0])
+        assert bin(vmask).count("1") <= width and imask & ~vmask == 0
+        p = np.float32(np.float64(pq) * np.float64(qs) + np.float64(lo))
+        scale = np.ldexp(np.float64(1.0), e.astype(int) - 127)
+        k = 0
+        for c in range(8):
+            if not vmask >> c & 1:
+                assert not w[16:64].reshape(6, 8)[:, c].any()
+                continue
+            slot = base + k
+            k += 1
+            assert slot < info.slot_count and not seen[slot]
+            seen[slot] = True
+            clo = p + scale * w[16:40].reshape(3, 8)[:, c]
+            chi = p + scale * w[40:64].reshape(3, 8)[:, c]
+            tol = 1e-5 * (np.abs(clo) + np.abs(chi) + scale)
+            if imask >> c & 1:
+                stack.append((slot, depth + 1, (clo - tol, chi + tol)))
+            else:
+                v = slots[slot][:36].view(np.float32).reshape(3, 3)
+                prims.append(int(slots[slot][36:40].view(np.uint32)[0]))
+                assert (v >= clo - tol).all() and (v <= chi + tol).all()
+    assert seen.all() and sorted(prims) == list(range(n))
+    assert (info.node_count, info.max_depth) == (nodes, deepest)
+
+
+def _mesh(n, seed):
+    g = torch.Generator().manual_seed(seed)
+    v = torch.rand(n, 1, 3, generator=g) * 10 + 0.3 * torch.rand(n, 3, 3, generator=g)
+    return {"vertices": v.reshape(-1, 3).contiguous().cuda(),
+            "indices": torch.arange(3 * n, dtype=torch.int32).reshape(-1, 3).cuda()}
+
+
+@pytest.mark.parametrize("width", [2, 5, 8])
+@pytest.mark.parametrize("n", [1, 2, 8, 9, 111, 112, 113, 900, 20011])
+def test_wide_structure(ctx, n, width):
+    import pyrtx
+    flags = pyrtx.RTX_BUILD_PREFER_FAST_TRACE_BIT | pyrtx.RTX_BUILD_MAX_WIDTH(width if width < 8 else 0)
+    for f in (flags, flags | pyrtx.RTX_BUILD_MORTON63_BIT | pyrtx.RTX_BUILD_NO_TREELET_BIT):
+        blas = ctx.build_blas([_mesh(n, n)], f)
+        ctx.sync()
+        _check_structure(ctx, blas, n, width)
+
+
+def test_wide_structure_batched_and_updated(ctx):
+    import pyrtx
+    sizes = [1, 2, 1, 5000, 3, 112, 113, 7, 1, 40, 1500]
+    meshes = [_mesh(n, 100 + k) for k, n in enumerate(sizes)]
+    for blas, n in zip(ctx.build_blas_batch([[m] for m in meshes]), sizes):
+        ctx.sync()
+        _check_structure(ctx, blas, n)
+    many = [[_mesh(1, k)] for k in range(70)]  # more structures than half their primitives
+    for blas in ctx.build_blas_batch(many):
+        ctx.sync()
+        _check_structure(ctx, blas, 1)
+    for n in (1, 112, 113, 3000):
+        blas = ctx.build_blas([_mesh(n, n)], pyrtx.RTX_BUILD_ALLOW_UPDATE_BIT)
+        moved = _mesh(n, n)
+        moved["vertices"] = (moved["vertices"] * 1.5 + torch.sin(moved["vertices"])).contiguous()
+        ctx.update_blas(blas, [moved])
+        ctx.sync()
+        _check_structure(ctx, blas, n)

@@ -2685,7 +2685,9 @@ hipError_t build_blas_batch(const GeomDesc* geoms_host, uint32_t ngeom, const ui
         prep_tris_kernel<<<(n - 1) / prep_chunk(n) + 1, 256, 0, s>>>(gd, (int)ngeom, n, (TriSlot*)(sc + L.leaves), boxes,
                                                                      cb, pblas, prep_chunk(n));
         morton_batch_kernel<<<gb, 256, 0, s>>>(boxes, n, cb, pblas, keys);
-        if ((err = sort_pairs_u64(keys, vals, n, sc + L.sort, err_flags, s))) return err;
+        int bits = 30;
+        while (bits < 64 && (nbatch - 1) >> (bits - 30)) ++bits;
+        if ((err = sort_pairs_u64(keys, vals, n, sc + L.sort, err_flags, s, bits))) return err;
         if (n > 1) {
             karras_kernel<uint64_t><<<gb, 256, 0, s>>>(keys, n, left, right, parent, (uint32_t*)(sc + L.cnt), nblas);
         } else {

@@ -12,7 +12,8 @@ uint64_t sort_scratch_bytes(uint32_t n, int key_bytes);
 // (the sorted permutation).  Stable.  err_flags receives kErrSortTimeout if a look-back spin ran out.
 hipError_t sort_pairs_u32(uint32_t* keys, uint32_t* vals, uint32_t n, void* scratch, uint32_t* err_flags,
                           hipStream_t stream);
+// key_bits: the keys' bits above are zero.
 hipError_t sort_pairs_u64(uint64_t* keys, uint32_t* vals, uint32_t n, void* scratch, uint32_t* err_flags,
-                          hipStream_t stream);
+                          hipStream_t stream, int key_bits = 64);
 
 }  // namespace rtx

@@ -3,10 +3,11 @@
 // Method: Adinets & Merrill 2022, "Onesweep: A Faster Least Significant Digit Radix Sort for GPUs".
 //   1. one pass over the keys builds the 256-bin histogram of every 8-bit digit (LDS-privatised);
 //   2. one 256-thread block turns the histograms into digit start offsets;
-//   3. per digit pass, each block takes a 4096-key tile (tile id from an atomic ticket, so every tile it
+//   3. per digit pass, each block takes a tile of keys (tile id from an atomic ticket, so every tile it
 //      waits for belongs to a block that is already running), ranks its keys stably in LDS using 64-lane
 //      ballots, publishes its per-digit counts and resolves its global offsets with decoupled look-back,
 //      stages the tile in LDS in digit order and writes it out in runs.
+// Up to one tile of keys is sorted by one block in one launch, the digit passes going back and forth in LDS.
 // The look-back spin is bounded: past the limit the block raises kErrSortTimeout and finishes.
 #include "rtx_internal.h"
 #include "sort.h"
@@ -16,8 +17,12 @@ namespace rtx {
 namespace {
 
 constexpr int kSortBlock = 256;
-constexpr int kSortItems = 16;
-constexpr int kTile = kSortBlock * kSortItems;
+// Keys per thread: 16 (4,096-key tiles); below kLargeFrom keys 4 (1,024-key tiles), so that more blocks share a pass
+// (655K keys: 20 us a pass with 16, 27 us with 4, whose look-back goes over four times the tiles).
+constexpr int kItemsLarge = 16, kItemsSmall = 4;
+constexpr uint32_t kLargeFrom = 1u << 17;
+constexpr uint32_t kOneBlock = kSortBlock * kItemsLarge;
+uint32_t tile_keys(uint32_t n) { return (uint32_t)kSortBlock * (uint32_t)(n >= kLargeFrom ? kItemsLarge : kItemsSmall); }
 constexpr int kRadix = 256;
 constexpr uint32_t kFlagAgg = 1u << 30;
 constexpr uint32_t kFlagInc = 2u << 30;
@@ -71,7 +76,66 @@ __device__ __forceinline__ void status_store(uint32_t* p, uint32_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <typename K>
+// Ranks of a tile's keys by one digit.  A wave takes ITEMS x 64 consecutive keys, 64 at a time, and counts its digits in
+// its own row of LDS: the lanes of one digit find each other by ballots, take their places after the wave's count so far,
+// and the first of them moves the count on.  (A row of counts shared by the waves, with two barriers per 64 keys of each,
+// took twice as long.)
+struct RankLds {
+    uint32_t cnt[4][kRadix];  // counts of each wave, then its first place
+    uint32_t excl[kRadix];    // digits' first places in the tile
+    uint32_t sum[4];
+};
+
+// Returns the count of digit threadIdx.x in the tile; rank[i] is the place among the tile's keys of that digit.
+template <typename K, int ITEMS>
+__device__ __forceinline__ uint32_t rank_tile(RankLds& R, const K* key, const bool* valid, int shift, uint32_t* rank) {
+    const int t = threadIdx.x, w = t >> 6, lane = t & 63;
+    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) R.cnt[k][t] = 0;
+    __syncthreads();
+    volatile uint32_t* const mine = R.cnt[w];
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const uint32_t d = (uint32_t)(key[i] >> shift) & 255u;
+        uint64_t peers = __ballot(valid[i]);
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            const uint64_t bits = __ballot((d >> b) & 1u);
+            peers &= ((d >> b) & 1u) ? bits : ~bits;
+        }
+        const uint32_t lr = (uint32_t)__popcll(peers & lt_mask);
+        const uint32_t before = mine[d];
+        rank[i] = before + lr;
+        if (valid[i] && lr == 0) mine[d] = before + (uint32_t)__popcll(peers);
+    }
+    __syncthreads();
+    // digit t: the waves' first places, and the exclusive prefix over the digits
+    const uint32_t c0 = R.cnt[0][t], c1 = R.cnt[1][t], c2 = R.cnt[2][t], c3 = R.cnt[3][t];
+    const uint32_t count = c0 + c1 + c2 + c3;
+    R.cnt[0][t] = 0;
+    R.cnt[1][t] = c0;
+    R.cnt[2][t] = c0 + c1;
+    R.cnt[3][t] = c0 + c1 + c2;
+    uint32_t incl = count;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t v = __shfl_up(incl, off);
+        if (lane >= off) incl += v;
+    }
+    if (lane == 63) R.sum[w] = incl;
+    __syncthreads();
+    uint32_t base = 0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) base += k < w ? R.sum[k] : 0u;
+    R.excl[t] = base + incl - count;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) rank[i] += R.cnt[w][(uint32_t)(key[i] >> shift) & 255u];
+    __syncthreads();
+    return count;
+}
+
+template <typename K, int ITEMS>
 __global__ __launch_bounds__(kSortBlock) void onesweep_kernel(const K* __restrict__ keys_in,
                                                               const uint32_t* __restrict__ vals_in,
                                                               K* __restrict__ keys_out, uint32_t* __restrict__ vals_out,
@@ -80,80 +144,32 @@ __global__ __launch_bounds__(kSortBlock) void onesweep_kernel(const K* __restric
                                                               uint32_t* __restrict__ status,
                                                               uint32_t* __restrict__ tile_counter,
                                                               uint32_t* __restrict__ err_flags) {
+    constexpr int kTile = kSortBlock * ITEMS;
     __shared__ uint32_t s_tile;
-    __shared__ uint32_t s_wave_cnt[4][kRadix];
-    __shared__ uint32_t s_wave_off[4][kRadix];
-    __shared__ uint32_t s_run[kRadix];
-    __shared__ uint32_t s_excl[kRadix];
+    __shared__ RankLds R;
     __shared__ uint32_t s_global[kRadix];
     __shared__ K s_keys[kTile];
     __shared__ uint32_t s_vals[kTile];
 
     const int t = threadIdx.x;
-    const int w = t >> 6;
-    const int lane = t & 63;
     if (t == 0) s_tile = atomicAdd(tile_counter, 1u);
-    for (int i = t; i < 4 * kRadix; i += kSortBlock) (&s_wave_cnt[0][0])[i] = 0;
-    s_run[t] = 0;
     __syncthreads();
     const uint32_t tile = s_tile;
     const uint64_t tile_start = (uint64_t)tile * kTile;
+    const uint64_t first = tile_start + (uint64_t)(t >> 6) * (64 * ITEMS) + (t & 63);
 
-    K key[kSortItems];
-    uint32_t val[kSortItems];
-    uint32_t rank[kSortItems];
-    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-
+    K key[ITEMS];
+    uint32_t val[ITEMS];
+    uint32_t rank[ITEMS];
+    bool valid[ITEMS];
 #pragma unroll
-    for (int i = 0; i < kSortItems; ++i) {
-        uint64_t idx = tile_start + (uint64_t)i * kSortBlock + t;
-        bool valid = idx < n;
-        key[i] = valid ? keys_in[idx] : (K)0;
-        val[i] = valid ? (vals_in ? vals_in[idx] : (uint32_t)idx) : 0u;
+    for (int i = 0; i < ITEMS; ++i) {
+        const uint64_t idx = first + 64u * i;
+        valid[i] = idx < n;
+        key[i] = valid[i] ? keys_in[idx] : (K)0;
+        val[i] = valid[i] ? (vals_in ? vals_in[idx] : (uint32_t)idx) : 0u;
     }
-
-#pragma unroll
-    for (int i = 0; i < kSortItems; ++i) {
-        uint64_t idx = tile_start + (uint64_t)i * kSortBlock + t;
-        bool valid = idx < n;
-        uint32_t d = (uint32_t)(key[i] >> shift) & 255u;
-        uint64_t peers = __ballot(valid);
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            uint64_t bits = __ballot((d >> b) & 1u);
-            peers &= ((d >> b) & 1u) ? bits : ~bits;
-        }
-        uint32_t lr = (uint32_t)__popcll(peers & lt_mask);
-        if (valid && lr == 0) s_wave_cnt[w][d] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        {
-            uint32_t c0 = s_wave_cnt[0][t], c1 = s_wave_cnt[1][t], c2 = s_wave_cnt[2][t], c3 = s_wave_cnt[3][t];
-            uint32_t run = s_run[t];
-            s_wave_off[0][t] = run;
-            s_wave_off[1][t] = run + c0;
-            s_wave_off[2][t] = run + c0 + c1;
-            s_wave_off[3][t] = run + c0 + c1 + c2;
-            s_run[t] = run + c0 + c1 + c2 + c3;
-            s_wave_cnt[0][t] = 0;
-            s_wave_cnt[1][t] = 0;
-            s_wave_cnt[2][t] = 0;
-            s_wave_cnt[3][t] = 0;
-        }
-        __syncthreads();
-        rank[i] = valid ? s_wave_off[w][d] + lr : 0xFFFFFFFFu;
-    }
-
-    // tile-local exclusive prefix over digits (positions inside the staged tile)
-    const uint32_t count = s_run[t];
-    s_excl[t] = count;
-    __syncthreads();
-    for (int off = 1; off < kRadix; off <<= 1) {
-        uint32_t v = t >= off ? s_excl[t - off] : 0u;
-        __syncthreads();
-        s_excl[t] += v;
-        __syncthreads();
-    }
-    s_excl[t] -= count;
+    const uint32_t count = rank_tile<K, ITEMS>(R, key, valid, shift, rank);
 
     // decoupled look-back for digit t
     {
@@ -184,13 +200,10 @@ __global__ __launch_bounds__(kSortBlock) void onesweep_kernel(const K* __restric
         }
         s_global[t] = digit_start[t] + excl;
     }
-    __syncthreads();
-
 #pragma unroll
-    for (int i = 0; i < kSortItems; ++i) {
-        if (rank[i] != 0xFFFFFFFFu) {
-            uint32_t d = (uint32_t)(key[i] >> shift) & 255u;
-            uint32_t pos = s_excl[d] + rank[i];
+    for (int i = 0; i < ITEMS; ++i) {
+        if (valid[i]) {
+            const uint32_t pos = R.excl[(uint32_t)(key[i] >> shift) & 255u] + rank[i];
             s_keys[pos] = key[i];
             s_vals[pos] = val[i];
         }
@@ -199,12 +212,12 @@ __global__ __launch_bounds__(kSortBlock) void onesweep_kernel(const K* __restric
     const uint64_t rem = (uint64_t)n - tile_start;
     const uint32_t tile_n = rem < (uint64_t)kTile ? (uint32_t)rem : (uint32_t)kTile;
 #pragma unroll
-    for (int i = 0; i < kSortItems; ++i) {
+    for (int i = 0; i < ITEMS; ++i) {
         uint32_t pos = (uint32_t)i * kSortBlock + t;
         if (pos < tile_n) {
             K k = s_keys[pos];
             uint32_t d = (uint32_t)(k >> shift) & 255u;
-            uint32_t o = s_global[d] + (pos - s_excl[d]);
+            uint32_t o = s_global[d] + (pos - R.excl[d]);
             if (o < n) {  // only false after a look-back timeout (reported through err_flags)
                 keys_out[o] = k;
                 vals_out[o] = s_vals[pos];
@@ -213,10 +226,58 @@ __global__ __launch_bounds__(kSortBlock) void onesweep_kernel(const K* __restric
     }
 }
 
+// At most one tile of keys: every pass in one block.
+template <typename K, int ITEMS>
+__global__ __launch_bounds__(kSortBlock) void one_block_sort_kernel(K* __restrict__ keys, uint32_t* __restrict__ vals,
+                                                                    uint32_t n, int passes) {
+    constexpr int kTile = kSortBlock * ITEMS;
+    __shared__ RankLds R;
+    __shared__ K s_keys[kTile];
+    __shared__ uint32_t s_vals[kTile];
+    const int t = threadIdx.x;
+    const uint32_t first = (uint32_t)(t >> 6) * (64 * ITEMS) + (t & 63);
+    K key[ITEMS];
+    uint32_t val[ITEMS], rank[ITEMS];
+    bool valid[ITEMS];
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        val[i] = first + 64u * i;
+        valid[i] = val[i] < n;
+        key[i] = valid[i] ? keys[val[i]] : (K)0;
+    }
+    for (int p = 0; p < passes; ++p) {
+        rank_tile<K, ITEMS>(R, key, valid, 8 * p, rank);
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            if (valid[i]) {
+                const uint32_t pos = R.excl[(uint32_t)(key[i] >> (8 * p)) & 255u] + rank[i];
+                s_keys[pos] = key[i];
+                s_vals[pos] = val[i];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            if (valid[i]) {
+                key[i] = s_keys[first + 64u * i];
+                val[i] = s_vals[first + 64u * i];
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        if (valid[i]) {
+            keys[first + 64u * i] = key[i];
+            vals[first + 64u * i] = val[i];
+        }
+    }
+}
+
 }  // namespace
 
 uint64_t sort_scratch_bytes(uint32_t n, int key_bytes) {
-    uint64_t tiles = (n + kTile - 1) / kTile;
+    uint64_t tiles = ((uint64_t)n + tile_keys(n) - 1) / tile_keys(n);
     int passes = key_bytes;  // 8-bit digits
     uint64_t b = 0;
     b += align_up((uint64_t)n * key_bytes, 256);       // alternate keys
@@ -232,7 +293,17 @@ template <typename K>
 static hipError_t sort_pairs_impl(K* keys, uint32_t* vals, uint32_t n, int passes, void* scratch,
                                   uint32_t* err_flags, hipStream_t stream) {
     if (n == 0) return hipSuccess;
-    uint64_t tiles = (n + kTile - 1) / kTile;
+    if (n <= kOneBlock) {
+        if (n <= kSortBlock)
+            one_block_sort_kernel<K, 1><<<1, kSortBlock, 0, stream>>>(keys, vals, n, passes);
+        else if (n <= kSortBlock * kItemsSmall)
+            one_block_sort_kernel<K, kItemsSmall><<<1, kSortBlock, 0, stream>>>(keys, vals, n, passes);
+        else
+            one_block_sort_kernel<K, kItemsLarge><<<1, kSortBlock, 0, stream>>>(keys, vals, n, passes);
+        return hipGetLastError();
+    }
+    const bool large = n >= kLargeFrom;
+    uint64_t tiles = ((uint64_t)n + tile_keys(n) - 1) / tile_keys(n);
     uint8_t* p = (uint8_t*)scratch;
     K* keys_alt = (K*)p;
     p += align_up((uint64_t)n * sizeof(K), 256);
@@ -256,9 +327,13 @@ static hipError_t sort_pairs_impl(K* keys, uint32_t* vals, uint32_t n, int passe
     uint32_t* vin = nullptr;
     uint32_t* vout = vals_alt;
     for (int pass = 0; pass < passes; ++pass) {
-        onesweep_kernel<K><<<(unsigned)tiles, kSortBlock, 0, stream>>>(
-            kin, vin, kout, vout, n, 8 * pass, start + pass * kRadix, status + (uint64_t)pass * tiles * kRadix,
-            counters + pass, err_flags);
+        uint32_t* st = status + (uint64_t)pass * tiles * kRadix;
+        if (large)
+            onesweep_kernel<K, kItemsLarge><<<(unsigned)tiles, kSortBlock, 0, stream>>>(
+                kin, vin, kout, vout, n, 8 * pass, start + pass * kRadix, st, counters + pass, err_flags);
+        else
+            onesweep_kernel<K, kItemsSmall><<<(unsigned)tiles, kSortBlock, 0, stream>>>(
+                kin, vin, kout, vout, n, 8 * pass, start + pass * kRadix, st, counters + pass, err_flags);
         std::swap(kin, kout);
         vin = vout;
         vout = (vout == vals_alt) ? vals : vals_alt;
@@ -273,8 +348,9 @@ hipError_t sort_pairs_u32(uint32_t* keys, uint32_t* vals, uint32_t n, void* scra
 }
 
 hipError_t sort_pairs_u64(uint64_t* keys, uint32_t* vals, uint32_t n, void* scratch, uint32_t* err_flags,
-                          hipStream_t stream) {
-    return sort_pairs_impl<uint64_t>(keys, vals, n, 8, scratch, err_flags, stream);
+                          hipStream_t stream, int key_bits) {
+    // an even number of passes over the digits that keys of key_bits bits have
+    return sort_pairs_impl<uint64_t>(keys, vals, n, (key_bits + 15) / 16 * 2, scratch, err_flags, stream);
 }
 
 }  // namespace rtx

@@ -128,3 +128,18 @@ def test_wide_structure_batched_and_updated(ctx):
         ctx.update_blas(blas, [moved])
         ctx.sync()
         _check_structure(ctx, blas, n)
+
+
+@pytest.mark.parametrize("n", [3, 255, 256, 257, 1023, 1024, 1025, 4095, 4096, 4097, 5121, (1 << 17) - 1, 1 << 17, (1 << 17) + 4097, 1500001])
+@pytest.mark.parametrize("kb", [4, 8])
+def test_sort_tiles(ctx, n, kb):
+    """The sort at the edges of its tiles and of its forms (one block, small tiles, large tiles), many equal keys."""
+    rng = np.random.default_rng(n + kb)
+    keys = rng.integers(0, 2 ** (8 * kb - 1), n, dtype=np.uint64)
+    keys[: n // 3] &= np.uint64(0xFF00FF)
+    keys[n // 2:] >>= np.uint64(8 * kb - 12)
+    keys = keys.astype(np.uint32 if kb == 4 else np.uint64)
+    got, order = ctx.debug_sort(keys)
+    want = np.argsort(keys, kind="stable")
+    assert np.array_equal(order, want.astype(np.uint32))
+    assert np.array_equal(got, keys[want])

@@ -38,10 +38,7 @@ constexpr float kErrScale = 0x1p-20f;
 constexpr float kTinyDir = 0x1p-80f;
 constexpr uint32_t kEntryLeaf = 1u << 16;
 constexpr uint32_t kEntryTlas = 1u << 17;
-// Triangles a lane tests per leaf step; the rest of its leaf group waits for a later leaf step, so lanes with
-// many candidates do not hold the wave in a long loop with few lanes active (2 measured best: +2.5% closest hit
-// coherent, +2.7% path tracing against testing the whole group).
-constexpr uint32_t kTrisPerStep = 2u;
+constexpr uint32_t kNoSlot = 0xFFFFFFFFu;
 constexpr uint32_t kMaxSteps = 1u << 22;  // per ray; a valid BVH never needs more than ~2 steps per slot
 
 // traceRayEXT ray flags (gl_RayFlags*EXT values) and instance flags (VkGeometryInstanceFlagBitsKHR)
@@ -541,6 +538,9 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
     constexpr int kShadeMode = MODE == kModePixelPaths ? (int)kPtPlain : (int)kPtCache;
     constexpr bool kRayLds = FLAGS || MODE == kModePath || MODE == kModeFused || kTrain;
     extern __shared__ uint2 lds_stack[];
+    __shared__ Words4 task_words[4][32];
+    __attribute__((address_space(3))) Words4* const tasks =
+        (__attribute__((address_space(3))) Words4*)task_words[threadIdx.x >> 6];
     float* const lds_ray = (float*)(lds_stack + args.lds_depth * blockDim.x) + threadIdx.x;
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
@@ -982,11 +982,12 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
         }
 
         int iter = 0;
-        while (active) {
+        bool go = true;
+        while (go) {
             bool done = false;
             uint32_t fault = 0;
             // a lane without pending work pops its next group and processes it in this same step
-            if (!(lg_bits & 255u) && !(ng_bits & 255u)) {
+            if (active && !((lg_bits | ng_bits) & 255u)) {
                 if (sp > 0) {
                     --sp;
                     const uint2 e = stacked(sp);
@@ -1026,16 +1027,139 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
                     done = true;
                 }
             }
-            // Postponed leaves: the leaf step (instance entry in FP64, or triangle tests) runs only once enough lanes
-            // of the wave hold a pending leaf group, or when no lane can traverse; until then lanes with a pending
-            // leaf keep traversing their node group, or wait.
-            const bool has_leaf = !done && (lg_bits & 255u) != 0u;
+            // Postponed leaves: the leaf step (triangle tests, instance entry in FP64) runs only once enough lanes of
+            // the wave hold a pending leaf group, or when no lane can traverse; until then lanes with a pending leaf
+            // keep traversing their node group, or wait.  (Lanes without a ray hold no group.)
+            const bool has_leaf = (lg_bits & 255u) != 0u;
             const uint64_t leaf_lanes = __builtin_amdgcn_ballot_w64(has_leaf);
-            const uint64_t node_lanes = __builtin_amdgcn_ballot_w64(!done && (ng_bits & 255u) != 0u);
-            const bool leaf_phase = (uint32_t)__popcll(leaf_lanes) >= args.leaf_lanes || node_lanes == 0ull;
-            if (done) {
-            } else if (has_leaf && leaf_phase) {
-                if (!in_blas) {
+            const uint64_t node_lanes = __builtin_amdgcn_ballot_w64((ng_bits & 255u) != 0u);
+            if (leaf_lanes && ((uint32_t)__popcll(leaf_lanes) >= args.leaf_lanes || node_lanes == 0ull)) {
+                const bool enter = has_leaf && !in_blas;
+                const uint64_t tri_lanes = __builtin_amdgcn_ballot_w64(has_leaf && in_blas);
+                if (tri_lanes) {
+                    // The next two triangles of each leaf group, one per lane of the wave: 4 to 12 lanes hold a leaf
+                    // group when the leaf step runs, most of them two triangles, so the owners hand theirs out and
+                    // one pass of the whole wave tests them (two passes of the owners alone took 6,000 to 10,000
+                    // cycles, this one takes 2,200 to 3,000).  Owners past the 32nd wait for the next leaf step.
+                    const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(tri_lanes >> 32),
+                                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)tri_lanes, 0u));
+                    const bool owner = has_leaf && in_blas && rank < 32u;
+                    uint32_t slot0 = kNoSlot, slot1 = kNoSlot;
+                    if (owner) {
+                        const uint32_t vm = lg_bits >> 8;
+                        uint32_t m = lg_bits & 255u;
+                        slot0 = lg_base + (uint32_t)__popc(vm & ((m & (0u - m)) - 1u));
+                        m &= m - 1u;
+                        if (m) {
+                            slot1 = lg_base + (uint32_t)__popc(vm & ((m & (0u - m)) - 1u));
+                            m &= m - 1u;
+                        }
+                        lg_bits = m | (vm << 8);
+                        if (slot0 >= cur_nslots || (slot1 != kNoSlot && slot1 >= cur_nslots)) {
+                            fault = kErrBadAs;
+                            slot0 = slot1 = kNoSlot;
+                        }
+                        tasks[rank] = Words4{slot0, slot1, lane, 0u};
+                    }
+                    const uint32_t ntri = 2u * (uint32_t)__popcll(tri_lanes);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    uint32_t from = lane, slot = kNoSlot;
+                    if (lane < ntri) {
+                        const Words4 w = tasks[lane >> 1];
+                        slot = (lane & 1u) ? w.y : w.x;
+                        from = w.z;
+                    }
+                    // the owner's ray
+                    const auto pull = [&](float v) {
+                        return __uint_as_float((uint32_t)__builtin_amdgcn_ds_bpermute((int)(from << 2),
+                                                                                      (int)__float_as_uint(v)));
+                    };
+                    const auto pullu = [&](uint32_t v) {
+                        return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(from << 2), (int)v);
+                    };
+                    Space hs;
+                    Shear hh;
+                    hs.ox = pull(s.ox);
+                    hs.oy = pull(s.oy);
+                    hs.oz = pull(s.oz);
+                    hh.rx0 = pull(sh.rx0);
+                    hh.rx1 = pull(sh.rx1);
+                    hh.rx2 = pull(sh.rx2);
+                    hh.ry0 = pull(sh.ry0);
+                    hh.ry1 = pull(sh.ry1);
+                    hh.ry2 = pull(sh.ry2);
+                    hh.rz0 = pull(sh.rz0);
+                    hh.rz1 = pull(sh.rz1);
+                    hh.rz2 = pull(sh.rz2);
+                    const float smin = pull(wtmin - s.toff);
+                    const float smax = pull(tc - s.toff);
+                    const uint64_t hslots =
+                        pullu((uint32_t)(uint64_t)cslots) | ((uint64_t)pullu((uint32_t)((uint64_t)cslots >> 32)) << 32);
+                    uint32_t hinst = 0;
+                    if (FLAGS) {
+                        hs.dx = pull(s.dx);
+                        hs.dy = pull(s.dy);
+                        hs.dz = pull(s.dz);
+                        hinst = pullu(cur_inst);
+                    }
+                    bool cand = false;
+                    float th = 0.0f;
+                    if (slot != kNoSlot) {
+                        const SlotPtr tp = (SlotPtr)hslots + (uint64_t)slot * kSlotBytes;
+                        const uint4 a = load_words(tp, 0), b = load_words(tp, 1), c = load_words(tp, 2);
+                        if (STATS) ++st_tris;
+                        float bu, bv;
+                        if (FLAGS && (c.w & kTriAabb)) {
+                            // AABB primitive: the intersection program of its hit record
+                            const float lo[3] = {__uint_as_float(a.x), __uint_as_float(a.y), __uint_as_float(a.z)};
+                            const float hi[3] = {__uint_as_float(a.w), __uint_as_float(b.x), __uint_as_float(b.y)};
+                            const float ro[3] = {hs.ox, hs.oy, hs.oz}, rd[3] = {hs.dx, hs.dy, hs.dz};
+                            float pn[3];
+                            cand = !(ray_flags & kRaySkipAabbs) &&
+                                   procedural_hit<float>(
+                                       intersection_program(args, table + (hinst & kInstIdMask), c.z), lo, hi, ro,
+                                       rd, smin, smax, th, bu, bv, pn);
+                        } else {
+                            cand = !(ray_flags & kRaySkipTriangles) &&
+                                   test_triangle(a, b, c, hs, hh, smin, smax, th, bu, bv) &&
+                                   !(ray_flags & (kRayCullBack | kRayCullFront) &&
+                                     facing_culled(a, b, c, hs, ray_flags, table[hinst & kInstIdMask].flags));
+                        }
+                        if (FLAGS && cand) cand = candidate_accepted(args, ray_flags, c.w, c.z, hinst, table, bu, bv);
+                    }
+                    const uint64_t hits = __builtin_amdgcn_ballot_w64(cand);
+                    if (hits) {
+                        if (cand) ((__attribute__((address_space(3))) float*)(tasks + (lane >> 1)))[lane & 1u] = th;
+                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                        const uint32_t own = owner ? (uint32_t)(hits >> (2u * rank)) & 3u : 0u;
+                        if (own) {
+                            if (MODE == kModeAny || ((MODE == kModeFused || kTrain) && shadow_ray)) {
+                                occl = true;
+                                done = true;
+                            } else {
+                                const Words2 w = *(__attribute__((address_space(3))) Words2*)(tasks + rank);
+                                // Exact ties in t go to the smaller (instance, slot), so the closest hit does not
+                                // depend on the order in which a lane meets its candidates (which the wave's leaf
+                                // scheduling can change).  A ray's first hit may round past its tmax.
+                                const uint32_t ci = cur_inst & kInstIdMask;
+#pragma unroll
+                                for (int k = 0; k < 2; ++k) {
+                                    const float tn = s.toff + __uint_as_float(k ? w.y : w.x);
+                                    const uint32_t sl = k ? slot1 : slot0;
+                                    const bool closer = !(tn >= tc) || hit_inst == kNoHit ||
+                                                        (tn == tc && (ci < hit_inst || (ci == hit_inst && sl < hit_slot)));
+                                    if ((own >> k & 1u) && closer) {
+                                        tc = tn;
+                                        hit_inst = ci;
+                                        hit_slot = sl;
+                                    }
+                                }
+                                if (ray_flags & kRayTerminateOnFirstHit) done = true;
+                            }
+                        }
+                    }
+                }
+                if (enter) {
                     // instance leaf: enter its BLAS
                     const uint32_t m = lg_bits & 255u;
                     const uint32_t k = (uint32_t)(__ffs(m) - 1);
@@ -1054,148 +1178,76 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
                     if ((imask & args.cull_mask & 255u) != 0u) {
                         if (STATS) ++st_insts;
                         // push the remaining TLAS work
-                        if (lg_bits & 255u) {
-                            push(make_uint2(lg_base, (lg_bits & 0xFFFFu) | kEntryLeaf | kEntryTlas));
-                        }
-                        if (ng_bits & 255u) {
-                            push(make_uint2(ng_base, (ng_bits & 0xFFFFu) | kEntryTlas));
-                        }
+                        if (lg_bits & 255u) push(make_uint2(lg_base, (lg_bits & 0xFFFFu) | kEntryLeaf | kEntryTlas));
+                        if (ng_bits & 255u) push(make_uint2(ng_base, (ng_bits & 0xFFFFu) | kEntryTlas));
                         lg_bits = 0;
-                        ng_bits = 0;
-                        {
-                            const InstanceInfo* info = table + iid;
-                            const auto* bh = (const __attribute__((address_space(1))) AsHeader*)blas;
-                            double M[12];
+                        const InstanceInfo* info = table + iid;
+                        const auto* bh = (const __attribute__((address_space(1))) AsHeader*)blas;
+                        double M[12];
 #pragma unroll
-                            for (int kk = 0; kk < 12; ++kk) M[kk] = info->inv[kk];
-                            if (kRayLds) {  // in the TLAS the current space is world space
-                                wo[0] = s.ox;
-                                wo[1] = s.oy;
-                                wo[2] = s.oz;
-                                wd[0] = s.dx;
-                                wd[1] = s.dy;
-                                wd[2] = s.dz;
-                            }
-                            double od[3], dd[3];
+                        for (int kk = 0; kk < 12; ++kk) M[kk] = info->inv[kk];
+                        if (kRayLds) {  // in the TLAS the current space is world space
+                            wo[0] = s.ox;
+                            wo[1] = s.oy;
+                            wo[2] = s.oz;
+                            wd[0] = s.dx;
+                            wd[1] = s.dy;
+                            wd[2] = s.dz;
+                        }
+                        double od[3], dd[3];
 #pragma unroll
-                            for (int r = 0; r < 3; ++r) {
-                                od[r] = M[4 * r] * wo[0] + M[4 * r + 1] * wo[1] + M[4 * r + 2] * wo[2] + M[4 * r + 3];
-                                dd[r] = M[4 * r] * wd[0] + M[4 * r + 1] * wd[1] + M[4 * r + 2] * wd[2];
-                            }
-                            // entry distance of the padded BLAS box, in FP32: it only chooses how far the origin
-                            // moves (hits between tmin and te stay in the window, whose lower end becomes
-                            // tmin - te), so its rounding costs nothing but keeps the FP64 divisions off this path
-                            const float lo3[3] = {bh->lo[0], bh->lo[1], bh->lo[2]};
-                            const float hi3[3] = {bh->hi[0], bh->hi[1], bh->hi[2]};
-                            float tn = -INFINITY;
+                        for (int r = 0; r < 3; ++r) {
+                            od[r] = M[4 * r] * wo[0] + M[4 * r + 1] * wo[1] + M[4 * r + 2] * wo[2] + M[4 * r + 3];
+                            dd[r] = M[4 * r] * wd[0] + M[4 * r + 1] * wd[1] + M[4 * r + 2] * wd[2];
+                        }
+                        // entry distance of the padded BLAS box, in FP32: it only chooses how far the origin
+                        // moves (hits between tmin and te stay in the window, whose lower end becomes
+                        // tmin - te), so its rounding costs nothing but keeps the FP64 divisions off this path
+                        const float lo3[3] = {bh->lo[0], bh->lo[1], bh->lo[2]};
+                        const float hi3[3] = {bh->hi[0], bh->hi[1], bh->hi[2]};
+                        float tn = -INFINITY;
 #pragma unroll
-                            for (int a = 0; a < 3; ++a) {
-                                const float pad = (hi3[a] - lo3[a]) * (1.0f / 64.0f) + 1e-30f;
-                                const float da = (float)dd[a], oa = (float)od[a];
-                                if (fabsf(da) > 1e-30f) {
-                                    const float r = __builtin_amdgcn_rcpf(da);
-                                    const float t1 = (lo3[a] - pad - oa) * r, t2 = (hi3[a] + pad - oa) * r;
-                                    tn = fmaxf(tn, fminf(t1, t2));
-                                }
+                        for (int a = 0; a < 3; ++a) {
+                            const float pad = (hi3[a] - lo3[a]) * (1.0f / 64.0f) + 1e-30f;
+                            const float da = (float)dd[a], oa = (float)od[a];
+                            if (fabsf(da) > 1e-30f) {
+                                const float r = __builtin_amdgcn_rcpf(da);
+                                const float t1 = (lo3[a] - pad - oa) * r, t2 = (hi3[a] + pad - oa) * r;
+                                tn = fmaxf(tn, fminf(t1, t2));
                             }
-                            const double te = fmax((double)wtmin, (double)tn);
-                            s.ox = (float)(od[0] + te * dd[0]);
-                            s.oy = (float)(od[1] + te * dd[1]);
-                            s.oz = (float)(od[2] + te * dd[2]);
-                            s.dx = (float)dd[0];
-                            s.dy = (float)dd[1];
-                            s.dz = (float)dd[2];
-                            s.toff = (float)te;
-                            setup_space(s);
-                            setup_shear(s, sh);
-                            cslots = (SlotPtr)blas + kHeaderBytes;
+                        }
+                        const double te = fmax((double)wtmin, (double)tn);
+                        s.ox = (float)(od[0] + te * dd[0]);
+                        s.oy = (float)(od[1] + te * dd[1]);
+                        s.oz = (float)(od[2] + te * dd[2]);
+                        s.dx = (float)dd[0];
+                        s.dy = (float)dd[1];
+                        s.dz = (float)dd[2];
+                        s.toff = (float)te;
+                        setup_space(s);
+                        setup_shear(s, sh);
+                        cslots = (SlotPtr)blas + kHeaderBytes;
 #pragma unroll
-                            for (int a = 0; a < 3; ++a) {
-                                crlo[a] = lo3[a];
-                                cqs[a] = bh->qscale[a];
-                            }
-                            in_blas = true;
-                            cur_inst = FLAGS ? iid | (((imask >> 10) & 3u) << 30) : iid;  // InstSlot mask | flags << 8
-                            cur_nslots = bh->slot_count;
-                            ng_base = 0;
-                            ng_bits = cur_nslots ? ((1u << s.oct) | (1u << 8)) : 0u;
+                        for (int a = 0; a < 3; ++a) {
+                            crlo[a] = lo3[a];
+                            cqs[a] = bh->qscale[a];
                         }
-                    }
-                } else {
-                    // triangles of the leaf group
-                    const uint32_t vm = lg_bits >> 8;
-                    uint32_t m = lg_bits & 255u;
-                    lg_bits = 0;
-                    const float smin = wtmin - s.toff;
-                    uint32_t budget = kTrisPerStep;
-                    while (m) {
-                        if (budget-- == 0u) {  // the rest waits for a later leaf step
-                            lg_bits = m | (vm << 8);
-                            break;
-                        }
-                        const uint32_t k = (uint32_t)(__ffs(m) - 1);
-                        m &= m - 1u;
-                        const uint32_t slot = lg_base + (uint32_t)__popc(vm & ((1u << k) - 1u));
-                        if (slot >= cur_nslots) {
-                            fault = kErrBadAs;
-                            break;
-                        }
-                        const SlotPtr tp = cslots + (uint64_t)slot * kSlotBytes;
-                        const uint4 a = load_words(tp, 0), b = load_words(tp, 1), c = load_words(tp, 2);
-                        if (STATS) ++st_tris;
-                        float th, bu, bv;
-                        const float smax = tc - s.toff;
-                        bool cand;
-                        if (FLAGS && (c.w & kTriAabb)) {
-                            // AABB primitive: the intersection program of its hit record
-                            const float lo[3] = {__uint_as_float(a.x), __uint_as_float(a.y), __uint_as_float(a.z)};
-                            const float hi[3] = {__uint_as_float(a.w), __uint_as_float(b.x), __uint_as_float(b.y)};
-                            const float ro[3] = {s.ox, s.oy, s.oz}, rd[3] = {s.dx, s.dy, s.dz};
-                            float pn[3];
-                            cand = !(ray_flags & kRaySkipAabbs) &&
-                                   procedural_hit<float>(
-                                       intersection_program(args, table + (cur_inst & kInstIdMask), c.z), lo, hi, ro,
-                                       rd, smin, smax, th, bu, bv, pn);
-                        } else {
-                            cand = !(ray_flags & kRaySkipTriangles) &&
-                                   test_triangle(a, b, c, s, sh, smin, smax, th, bu, bv) &&
-                                   !(ray_flags & (kRayCullBack | kRayCullFront) &&
-                                     facing_culled(a, b, c, s, ray_flags, table[cur_inst & kInstIdMask].flags));
-                        }
-                        if (cand &&
-                            (!FLAGS || candidate_accepted(args, ray_flags, c.w, c.z, cur_inst, table, bu, bv))) {
-                            if (MODE == kModeAny || ((MODE == kModeFused || kTrain) && shadow_ray)) {
-                                occl = true;
-                                done = true;
-                                break;
-                            }
-                            // exact ties in t go to the smaller (instance, slot), so the closest hit does not
-                            // depend on the order in which a lane meets its candidates (which the wave's leaf
-                            // scheduling can change)
-                            const float tn = s.toff + th;
-                            const uint32_t ci = cur_inst & kInstIdMask;
-                            if (!(tn == tc && (ci > hit_inst || (ci == hit_inst && slot > hit_slot)))) {
-                                tc = tn;
-                                hit_inst = ci;
-                                hit_slot = slot;
-                            }
-                            if (ray_flags & kRayTerminateOnFirstHit) {
-                                done = true;
-                                break;
-                            }
-                        }
+                        in_blas = true;
+                        cur_inst = FLAGS ? iid | (((imask >> 10) & 3u) << 30) : iid;  // InstSlot mask | flags << 8
+                        cur_nslots = bh->slot_count;
+                        ng_base = 0;
+                        ng_bits = cur_nslots ? ((1u << s.oct) | (1u << 8)) : 0u;
                     }
                 }
-            } else if (ng_bits & 255u) {
+            }
+            if (!done && (ng_bits & 255u)) {
                 const uint32_t om = ng_bits & 255u;
                 const uint32_t j = (uint32_t)(__ffs(om) - 1);
                 const uint32_t k = j ^ s.oct;
                 const uint32_t vm = (ng_bits >> 8) & 255u;
                 const uint32_t slot = ng_base + (uint32_t)__popc(vm & ((1u << k) - 1u));
                 ng_bits &= ~(1u << j);
-                if (ng_bits & 255u) {
-                    push(make_uint2(ng_base, (ng_bits & 0xFFFFu) | (in_blas ? 0u : kEntryTlas)));
-                }
+                if (ng_bits & 255u) push(make_uint2(ng_base, (ng_bits & 0xFFFFu) | (in_blas ? 0u : kEntryTlas)));
                 if (slot >= cur_nslots) {
                     fault = kErrBadAs;
                     ng_bits = 0;
@@ -1227,25 +1279,27 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
                 done = true;
             }
             if (fault) atomicOr(&args.state->error_flags, fault);
-
             if (done) {
                 // the result is written at the next refill, together with the wave's other finished lanes
                 finished = true;
                 active = false;
-                break;
+                lg_bits = 0;
+                ng_bits = 0;
+                sp = 0;
             }
+            const uint64_t busy = __builtin_amdgcn_ballot_w64(active);
+            go = busy != 0ull;
             if (++iter >= (int)args.refill_interval) {
                 iter = 0;
                 steps += args.refill_interval;
                 if (steps > kMaxSteps) {
-                    atomicOr(&args.state->error_flags, kErrBadAs);
+                    if (active) atomicOr(&args.state->error_flags, kErrBadAs);
                     lg_bits = 0;
                     ng_bits = 0;
                     sp = 0;
                 }
-                if (kTrain ? (uint32_t)__popcll(__ballot(true)) <= train_floor
-                           : (!wave_exhausted && __popcll(__ballot(true)) < args.refill_lanes))
-                    break;
+                const uint32_t lanes = (uint32_t)__popcll(busy);
+                go = go && (kTrain ? lanes > train_floor : (wave_exhausted || lanes >= args.refill_lanes));
             }
         }
     }

@@ -972,12 +972,14 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
         }
         if (!__any(active)) break;
         const bool wave_exhausted = !more && pool_next >= pool_end;
-        // kModeTrain: back to the refill point (where ended rays continue their paths) once a quarter of the lanes
-        // that start this round (64 - refill_lanes of 64) have ended their rays, at least one
+        // Whole paths: back to the refill point (where ended rays continue their paths) once half of the lanes that
+        // start this round (64 - refill_lanes of 32) have ended their rays, at least one.  Shading costs as much as
+        // five traversal steps, however few lanes shade: 4 samples of the 1080p Cornell box 15.0 ms with half of the
+        // lanes, 17.2 ms with a quarter, 15.8 ms with three quarters.
         uint32_t train_floor = 0;
         if (kTrain) {
             const uint32_t n0 = (uint32_t)__popcll(__ballot(active));
-            const uint32_t q = n0 * (64u - args.refill_lanes) / 64u;
+            const uint32_t q = std::min(n0, n0 * (64u - args.refill_lanes) / 32u);
             train_floor = n0 - (q > 0u ? q : 1u);
         }
 
@@ -986,8 +988,223 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
         while (go) {
             bool done = false;
             uint32_t fault = 0;
-            // a lane without pending work pops its next group and processes it in this same step
-            if (active && !((lg_bits | ng_bits) & 255u)) {
+            // Postponed leaves: the triangle step runs only once leaf_lanes lanes of the wave hold a pending leaf group
+            // of triangles, the instance step (BLAS entry in FP64) once as many hold one of instances, and both when
+            // no lane can traverse; until then lanes with a pending leaf keep traversing their node group, or wait.
+            // (Lanes without a ray hold no group.)  Each has its own threshold, because an instance step costs twice a
+            // triangle step: with one for both 16.7M incoherent rays took 2.59 ms, now 2.41 ms.
+            const bool has_leaf = (lg_bits & 255u) != 0u;
+            const bool enter = has_leaf && !in_blas;
+            const uint32_t inst_lanes = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(enter));
+            const uint64_t tri_lanes = __builtin_amdgcn_ballot_w64(has_leaf && in_blas);
+            const bool no_node =
+                __builtin_amdgcn_ballot_w64((ng_bits & 255u) || (active && !(lg_bits & 255u))) == 0ull;
+            if (tri_lanes && ((uint32_t)__popcll(tri_lanes) >= args.leaf_lanes || no_node)) {
+                // The next two triangles of each leaf group, one per lane of the wave: 4 to 12 lanes hold a leaf
+                // group when the leaf step runs, most of them two triangles, so the owners hand theirs out and
+                // one pass of the whole wave tests them (two passes of the owners alone took 6,000 to 10,000
+                // cycles, this one takes 2,200 to 3,000).  Owners past the 32nd wait for the next leaf step.
+                const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(tri_lanes >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)tri_lanes, 0u));
+                const bool owner = has_leaf && in_blas && rank < 32u;
+                uint32_t slot0 = kNoSlot, slot1 = kNoSlot;
+                if (owner) {
+                    const uint32_t vm = lg_bits >> 8;
+                    uint32_t m = lg_bits & 255u;
+                    slot0 = lg_base + (uint32_t)__popc(vm & ((m & (0u - m)) - 1u));
+                    m &= m - 1u;
+                    if (m) {
+                        slot1 = lg_base + (uint32_t)__popc(vm & ((m & (0u - m)) - 1u));
+                        m &= m - 1u;
+                    }
+                    lg_bits = m | (vm << 8);
+                    if (slot0 >= cur_nslots || (slot1 != kNoSlot && slot1 >= cur_nslots)) {
+                        fault = kErrBadAs;
+                        slot0 = slot1 = kNoSlot;
+                    }
+                    tasks[rank] = Words4{slot0, slot1, lane, 0u};
+                }
+                const uint32_t ntri = 2u * (uint32_t)__popcll(tri_lanes);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                uint32_t from = lane, slot = kNoSlot;
+                if (lane < ntri) {
+                    const Words4 w = tasks[lane >> 1];
+                    slot = (lane & 1u) ? w.y : w.x;
+                    from = w.z;
+                }
+                // the owner's ray
+                const auto pull = [&](float v) {
+                    return __uint_as_float((uint32_t)__builtin_amdgcn_ds_bpermute((int)(from << 2),
+                                                                                  (int)__float_as_uint(v)));
+                };
+                const auto pullu = [&](uint32_t v) {
+                    return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(from << 2), (int)v);
+                };
+                Space hs;
+                Shear hh;
+                hs.ox = pull(s.ox);
+                hs.oy = pull(s.oy);
+                hs.oz = pull(s.oz);
+                hh.rx0 = pull(sh.rx0);
+                hh.rx1 = pull(sh.rx1);
+                hh.rx2 = pull(sh.rx2);
+                hh.ry0 = pull(sh.ry0);
+                hh.ry1 = pull(sh.ry1);
+                hh.ry2 = pull(sh.ry2);
+                hh.rz0 = pull(sh.rz0);
+                hh.rz1 = pull(sh.rz1);
+                hh.rz2 = pull(sh.rz2);
+                const float smin = pull(wtmin - s.toff);
+                const float smax = pull(tc - s.toff);
+                const uint64_t hslots =
+                    pullu((uint32_t)(uint64_t)cslots) | ((uint64_t)pullu((uint32_t)((uint64_t)cslots >> 32)) << 32);
+                uint32_t hinst = 0;
+                if (FLAGS) {
+                    hs.dx = pull(s.dx);
+                    hs.dy = pull(s.dy);
+                    hs.dz = pull(s.dz);
+                    hinst = pullu(cur_inst);
+                }
+                bool cand = false;
+                float th = 0.0f;
+                if (slot != kNoSlot) {
+                    const SlotPtr tp = (SlotPtr)hslots + (uint64_t)slot * kSlotBytes;
+                    const uint4 a = load_words(tp, 0), b = load_words(tp, 1), c = load_words(tp, 2);
+                    if (STATS) ++st_tris;
+                    float bu, bv;
+                    if (FLAGS && (c.w & kTriAabb)) {
+                        // AABB primitive: the intersection program of its hit record
+                        const float lo[3] = {__uint_as_float(a.x), __uint_as_float(a.y), __uint_as_float(a.z)};
+                        const float hi[3] = {__uint_as_float(a.w), __uint_as_float(b.x), __uint_as_float(b.y)};
+                        const float ro[3] = {hs.ox, hs.oy, hs.oz}, rd[3] = {hs.dx, hs.dy, hs.dz};
+                        float pn[3];
+                        cand = !(ray_flags & kRaySkipAabbs) &&
+                               procedural_hit<float>(
+                                   intersection_program(args, table + (hinst & kInstIdMask), c.z), lo, hi, ro,
+                                   rd, smin, smax, th, bu, bv, pn);
+                    } else {
+                        cand = !(ray_flags & kRaySkipTriangles) &&
+                               test_triangle(a, b, c, hs, hh, smin, smax, th, bu, bv) &&
+                               !(ray_flags & (kRayCullBack | kRayCullFront) &&
+                                 facing_culled(a, b, c, hs, ray_flags, table[hinst & kInstIdMask].flags));
+                    }
+                    if (FLAGS && cand) cand = candidate_accepted(args, ray_flags, c.w, c.z, hinst, table, bu, bv);
+                }
+                const uint64_t hits = __builtin_amdgcn_ballot_w64(cand);
+                if (hits) {
+                    if (cand) ((__attribute__((address_space(3))) float*)(tasks + (lane >> 1)))[lane & 1u] = th;
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    const uint32_t own = owner ? (uint32_t)(hits >> (2u * rank)) & 3u : 0u;
+                    if (own) {
+                        if (MODE == kModeAny || ((MODE == kModeFused || kTrain) && shadow_ray)) {
+                            occl = true;
+                            done = true;
+                        } else {
+                            const Words2 w = *(__attribute__((address_space(3))) Words2*)(tasks + rank);
+                            // Exact ties in t go to the smaller (instance, slot), so the closest hit does not
+                            // depend on the order in which a lane meets its candidates (which the wave's leaf
+                            // scheduling can change).  A ray's first hit may round past its tmax.
+                            const uint32_t ci = cur_inst & kInstIdMask;
+#pragma unroll
+                            for (int k = 0; k < 2; ++k) {
+                                const float tn = s.toff + __uint_as_float(k ? w.y : w.x);
+                                const uint32_t sl = k ? slot1 : slot0;
+                                const bool closer = !(tn >= tc) || hit_inst == kNoHit ||
+                                                    (tn == tc && (ci < hit_inst || (ci == hit_inst && sl < hit_slot)));
+                                if ((own >> k & 1u) && closer) {
+                                    tc = tn;
+                                    hit_inst = ci;
+                                    hit_slot = sl;
+                                }
+                            }
+                            if (ray_flags & kRayTerminateOnFirstHit) done = true;
+                        }
+                    }
+                }
+            }
+            if ((inst_lanes >= args.leaf_lanes || no_node) && enter) {
+                // instance leaf: enter its BLAS
+                const uint32_t m = lg_bits & 255u;
+                const uint32_t k = (uint32_t)(__ffs(m) - 1);
+                const uint32_t vm = lg_bits >> 8;
+                lg_bits &= ~(1u << k);
+                const uint32_t slot = lg_base + (uint32_t)__popc(vm & ((1u << k) - 1u));
+                uint4 q = make_uint4(0u, 0u, 0u, 0u);
+                if (slot < tlas_nslots) {
+                    q = load_words(tslots + (uint64_t)slot * kSlotBytes, 3);
+                    if (q.z >= tlas_ninst) q.w = 0u;
+                } else {
+                    fault = kErrBadAs;
+                }
+                const uint64_t blas = (uint64_t)q.x | ((uint64_t)q.y << 32);
+                const uint32_t iid = q.z, imask = q.w;
+                if ((imask & args.cull_mask & 255u) != 0u) {
+                    if (STATS) ++st_insts;
+                    // push the remaining TLAS work
+                    if (lg_bits & 255u) push(make_uint2(lg_base, (lg_bits & 0xFFFFu) | kEntryLeaf | kEntryTlas));
+                    if (ng_bits & 255u) push(make_uint2(ng_base, (ng_bits & 0xFFFFu) | kEntryTlas));
+                    lg_bits = 0;
+                    const InstanceInfo* info = table + iid;
+                    const auto* bh = (const __attribute__((address_space(1))) AsHeader*)blas;
+                    double M[12];
+#pragma unroll
+                    for (int kk = 0; kk < 12; ++kk) M[kk] = info->inv[kk];
+                    if (kRayLds) {  // in the TLAS the current space is world space
+                        wo[0] = s.ox;
+                        wo[1] = s.oy;
+                        wo[2] = s.oz;
+                        wd[0] = s.dx;
+                        wd[1] = s.dy;
+                        wd[2] = s.dz;
+                    }
+                    double od[3], dd[3];
+#pragma unroll
+                    for (int r = 0; r < 3; ++r) {
+                        od[r] = M[4 * r] * wo[0] + M[4 * r + 1] * wo[1] + M[4 * r + 2] * wo[2] + M[4 * r + 3];
+                        dd[r] = M[4 * r] * wd[0] + M[4 * r + 1] * wd[1] + M[4 * r + 2] * wd[2];
+                    }
+                    // entry distance of the padded BLAS box, in FP32: it only chooses how far the origin
+                    // moves (hits between tmin and te stay in the window, whose lower end becomes
+                    // tmin - te), so its rounding costs nothing but keeps the FP64 divisions off this path
+                    const float lo3[3] = {bh->lo[0], bh->lo[1], bh->lo[2]};
+                    const float hi3[3] = {bh->hi[0], bh->hi[1], bh->hi[2]};
+                    float tn = -INFINITY;
+#pragma unroll
+                    for (int a = 0; a < 3; ++a) {
+                        const float pad = (hi3[a] - lo3[a]) * (1.0f / 64.0f) + 1e-30f;
+                        const float da = (float)dd[a], oa = (float)od[a];
+                        if (fabsf(da) > 1e-30f) {
+                            const float r = __builtin_amdgcn_rcpf(da);
+                            const float t1 = (lo3[a] - pad - oa) * r, t2 = (hi3[a] + pad - oa) * r;
+                            tn = fmaxf(tn, fminf(t1, t2));
+                        }
+                    }
+                    const double te = fmax((double)wtmin, (double)tn);
+                    s.ox = (float)(od[0] + te * dd[0]);
+                    s.oy = (float)(od[1] + te * dd[1]);
+                    s.oz = (float)(od[2] + te * dd[2]);
+                    s.dx = (float)dd[0];
+                    s.dy = (float)dd[1];
+                    s.dz = (float)dd[2];
+                    s.toff = (float)te;
+                    setup_space(s);
+                    setup_shear(s, sh);
+                    cslots = (SlotPtr)blas + kHeaderBytes;
+#pragma unroll
+                    for (int a = 0; a < 3; ++a) {
+                        crlo[a] = lo3[a];
+                        cqs[a] = bh->qscale[a];
+                    }
+                    in_blas = true;
+                    cur_inst = FLAGS ? iid | (((imask >> 10) & 3u) << 30) : iid;  // InstSlot mask | flags << 8
+                    cur_nslots = bh->slot_count;
+                    ng_base = 0;
+                    ng_bits = cur_nslots ? ((1u << s.oct) | (1u << 8)) : 0u;
+                }
+            }
+            // a lane without pending work pops its next group; a node group is taken on in this same step, also by the
+            // lanes that have just tested their last triangles (popping at the start of a step: 4% slower)
+            if (active && !done && !((lg_bits | ng_bits) & 255u)) {
                 if (sp > 0) {
                     --sp;
                     const uint2 e = stacked(sp);
@@ -1025,219 +1242,6 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
                     }
                 } else {
                     done = true;
-                }
-            }
-            // Postponed leaves: the leaf step (triangle tests, instance entry in FP64) runs only once enough lanes of
-            // the wave hold a pending leaf group, or when no lane can traverse; until then lanes with a pending leaf
-            // keep traversing their node group, or wait.  (Lanes without a ray hold no group.)
-            const bool has_leaf = (lg_bits & 255u) != 0u;
-            const uint64_t leaf_lanes = __builtin_amdgcn_ballot_w64(has_leaf);
-            const uint64_t node_lanes = __builtin_amdgcn_ballot_w64((ng_bits & 255u) != 0u);
-            if (leaf_lanes && ((uint32_t)__popcll(leaf_lanes) >= args.leaf_lanes || node_lanes == 0ull)) {
-                const bool enter = has_leaf && !in_blas;
-                const uint64_t tri_lanes = __builtin_amdgcn_ballot_w64(has_leaf && in_blas);
-                if (tri_lanes) {
-                    // The next two triangles of each leaf group, one per lane of the wave: 4 to 12 lanes hold a leaf
-                    // group when the leaf step runs, most of them two triangles, so the owners hand theirs out and
-                    // one pass of the whole wave tests them (two passes of the owners alone took 6,000 to 10,000
-                    // cycles, this one takes 2,200 to 3,000).  Owners past the 32nd wait for the next leaf step.
-                    const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(tri_lanes >> 32),
-                                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)tri_lanes, 0u));
-                    const bool owner = has_leaf && in_blas && rank < 32u;
-                    uint32_t slot0 = kNoSlot, slot1 = kNoSlot;
-                    if (owner) {
-                        const uint32_t vm = lg_bits >> 8;
-                        uint32_t m = lg_bits & 255u;
-                        slot0 = lg_base + (uint32_t)__popc(vm & ((m & (0u - m)) - 1u));
-                        m &= m - 1u;
-                        if (m) {
-                            slot1 = lg_base + (uint32_t)__popc(vm & ((m & (0u - m)) - 1u));
-                            m &= m - 1u;
-                        }
-                        lg_bits = m | (vm << 8);
-                        if (slot0 >= cur_nslots || (slot1 != kNoSlot && slot1 >= cur_nslots)) {
-                            fault = kErrBadAs;
-                            slot0 = slot1 = kNoSlot;
-                        }
-                        tasks[rank] = Words4{slot0, slot1, lane, 0u};
-                    }
-                    const uint32_t ntri = 2u * (uint32_t)__popcll(tri_lanes);
-                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                    uint32_t from = lane, slot = kNoSlot;
-                    if (lane < ntri) {
-                        const Words4 w = tasks[lane >> 1];
-                        slot = (lane & 1u) ? w.y : w.x;
-                        from = w.z;
-                    }
-                    // the owner's ray
-                    const auto pull = [&](float v) {
-                        return __uint_as_float((uint32_t)__builtin_amdgcn_ds_bpermute((int)(from << 2),
-                                                                                      (int)__float_as_uint(v)));
-                    };
-                    const auto pullu = [&](uint32_t v) {
-                        return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(from << 2), (int)v);
-                    };
-                    Space hs;
-                    Shear hh;
-                    hs.ox = pull(s.ox);
-                    hs.oy = pull(s.oy);
-                    hs.oz = pull(s.oz);
-                    hh.rx0 = pull(sh.rx0);
-                    hh.rx1 = pull(sh.rx1);
-                    hh.rx2 = pull(sh.rx2);
-                    hh.ry0 = pull(sh.ry0);
-                    hh.ry1 = pull(sh.ry1);
-                    hh.ry2 = pull(sh.ry2);
-                    hh.rz0 = pull(sh.rz0);
-                    hh.rz1 = pull(sh.rz1);
-                    hh.rz2 = pull(sh.rz2);
-                    const float smin = pull(wtmin - s.toff);
-                    const float smax = pull(tc - s.toff);
-                    const uint64_t hslots =
-                        pullu((uint32_t)(uint64_t)cslots) | ((uint64_t)pullu((uint32_t)((uint64_t)cslots >> 32)) << 32);
-                    uint32_t hinst = 0;
-                    if (FLAGS) {
-                        hs.dx = pull(s.dx);
-                        hs.dy = pull(s.dy);
-                        hs.dz = pull(s.dz);
-                        hinst = pullu(cur_inst);
-                    }
-                    bool cand = false;
-                    float th = 0.0f;
-                    if (slot != kNoSlot) {
-                        const SlotPtr tp = (SlotPtr)hslots + (uint64_t)slot * kSlotBytes;
-                        const uint4 a = load_words(tp, 0), b = load_words(tp, 1), c = load_words(tp, 2);
-                        if (STATS) ++st_tris;
-                        float bu, bv;
-                        if (FLAGS && (c.w & kTriAabb)) {
-                            // AABB primitive: the intersection program of its hit record
-                            const float lo[3] = {__uint_as_float(a.x), __uint_as_float(a.y), __uint_as_float(a.z)};
-                            const float hi[3] = {__uint_as_float(a.w), __uint_as_float(b.x), __uint_as_float(b.y)};
-                            const float ro[3] = {hs.ox, hs.oy, hs.oz}, rd[3] = {hs.dx, hs.dy, hs.dz};
-                            float pn[3];
-                            cand = !(ray_flags & kRaySkipAabbs) &&
-                                   procedural_hit<float>(
-                                       intersection_program(args, table + (hinst & kInstIdMask), c.z), lo, hi, ro,
-                                       rd, smin, smax, th, bu, bv, pn);
-                        } else {
-                            cand = !(ray_flags & kRaySkipTriangles) &&
-                                   test_triangle(a, b, c, hs, hh, smin, smax, th, bu, bv) &&
-                                   !(ray_flags & (kRayCullBack | kRayCullFront) &&
-                                     facing_culled(a, b, c, hs, ray_flags, table[hinst & kInstIdMask].flags));
-                        }
-                        if (FLAGS && cand) cand = candidate_accepted(args, ray_flags, c.w, c.z, hinst, table, bu, bv);
-                    }
-                    const uint64_t hits = __builtin_amdgcn_ballot_w64(cand);
-                    if (hits) {
-                        if (cand) ((__attribute__((address_space(3))) float*)(tasks + (lane >> 1)))[lane & 1u] = th;
-                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                        const uint32_t own = owner ? (uint32_t)(hits >> (2u * rank)) & 3u : 0u;
-                        if (own) {
-                            if (MODE == kModeAny || ((MODE == kModeFused || kTrain) && shadow_ray)) {
-                                occl = true;
-                                done = true;
-                            } else {
-                                const Words2 w = *(__attribute__((address_space(3))) Words2*)(tasks + rank);
-                                // Exact ties in t go to the smaller (instance, slot), so the closest hit does not
-                                // depend on the order in which a lane meets its candidates (which the wave's leaf
-                                // scheduling can change).  A ray's first hit may round past its tmax.
-                                const uint32_t ci = cur_inst & kInstIdMask;
-#pragma unroll
-                                for (int k = 0; k < 2; ++k) {
-                                    const float tn = s.toff + __uint_as_float(k ? w.y : w.x);
-                                    const uint32_t sl = k ? slot1 : slot0;
-                                    const bool closer = !(tn >= tc) || hit_inst == kNoHit ||
-                                                        (tn == tc && (ci < hit_inst || (ci == hit_inst && sl < hit_slot)));
-                                    if ((own >> k & 1u) && closer) {
-                                        tc = tn;
-                                        hit_inst = ci;
-                                        hit_slot = sl;
-                                    }
-                                }
-                                if (ray_flags & kRayTerminateOnFirstHit) done = true;
-                            }
-                        }
-                    }
-                }
-                if (enter) {
-                    // instance leaf: enter its BLAS
-                    const uint32_t m = lg_bits & 255u;
-                    const uint32_t k = (uint32_t)(__ffs(m) - 1);
-                    const uint32_t vm = lg_bits >> 8;
-                    lg_bits &= ~(1u << k);
-                    const uint32_t slot = lg_base + (uint32_t)__popc(vm & ((1u << k) - 1u));
-                    uint4 q = make_uint4(0u, 0u, 0u, 0u);
-                    if (slot < tlas_nslots) {
-                        q = load_words(tslots + (uint64_t)slot * kSlotBytes, 3);
-                        if (q.z >= tlas_ninst) q.w = 0u;
-                    } else {
-                        fault = kErrBadAs;
-                    }
-                    const uint64_t blas = (uint64_t)q.x | ((uint64_t)q.y << 32);
-                    const uint32_t iid = q.z, imask = q.w;
-                    if ((imask & args.cull_mask & 255u) != 0u) {
-                        if (STATS) ++st_insts;
-                        // push the remaining TLAS work
-                        if (lg_bits & 255u) push(make_uint2(lg_base, (lg_bits & 0xFFFFu) | kEntryLeaf | kEntryTlas));
-                        if (ng_bits & 255u) push(make_uint2(ng_base, (ng_bits & 0xFFFFu) | kEntryTlas));
-                        lg_bits = 0;
-                        const InstanceInfo* info = table + iid;
-                        const auto* bh = (const __attribute__((address_space(1))) AsHeader*)blas;
-                        double M[12];
-#pragma unroll
-                        for (int kk = 0; kk < 12; ++kk) M[kk] = info->inv[kk];
-                        if (kRayLds) {  // in the TLAS the current space is world space
-                            wo[0] = s.ox;
-                            wo[1] = s.oy;
-                            wo[2] = s.oz;
-                            wd[0] = s.dx;
-                            wd[1] = s.dy;
-                            wd[2] = s.dz;
-                        }
-                        double od[3], dd[3];
-#pragma unroll
-                        for (int r = 0; r < 3; ++r) {
-                            od[r] = M[4 * r] * wo[0] + M[4 * r + 1] * wo[1] + M[4 * r + 2] * wo[2] + M[4 * r + 3];
-                            dd[r] = M[4 * r] * wd[0] + M[4 * r + 1] * wd[1] + M[4 * r + 2] * wd[2];
-                        }
-                        // entry distance of the padded BLAS box, in FP32: it only chooses how far the origin
-                        // moves (hits between tmin and te stay in the window, whose lower end becomes
-                        // tmin - te), so its rounding costs nothing but keeps the FP64 divisions off this path
-                        const float lo3[3] = {bh->lo[0], bh->lo[1], bh->lo[2]};
-                        const float hi3[3] = {bh->hi[0], bh->hi[1], bh->hi[2]};
-                        float tn = -INFINITY;
-#pragma unroll
-                        for (int a = 0; a < 3; ++a) {
-                            const float pad = (hi3[a] - lo3[a]) * (1.0f / 64.0f) + 1e-30f;
-                            const float da = (float)dd[a], oa = (float)od[a];
-                            if (fabsf(da) > 1e-30f) {
-                                const float r = __builtin_amdgcn_rcpf(da);
-                                const float t1 = (lo3[a] - pad - oa) * r, t2 = (hi3[a] + pad - oa) * r;
-                                tn = fmaxf(tn, fminf(t1, t2));
-                            }
-                        }
-                        const double te = fmax((double)wtmin, (double)tn);
-                        s.ox = (float)(od[0] + te * dd[0]);
-                        s.oy = (float)(od[1] + te * dd[1]);
-                        s.oz = (float)(od[2] + te * dd[2]);
-                        s.dx = (float)dd[0];
-                        s.dy = (float)dd[1];
-                        s.dz = (float)dd[2];
-                        s.toff = (float)te;
-                        setup_space(s);
-                        setup_shear(s, sh);
-                        cslots = (SlotPtr)blas + kHeaderBytes;
-#pragma unroll
-                        for (int a = 0; a < 3; ++a) {
-                            crlo[a] = lo3[a];
-                            cqs[a] = bh->qscale[a];
-                        }
-                        in_blas = true;
-                        cur_inst = FLAGS ? iid | (((imask >> 10) & 3u) << 30) : iid;  // InstSlot mask | flags << 8
-                        cur_nslots = bh->slot_count;
-                        ng_base = 0;
-                        ng_bits = cur_nslots ? ((1u << s.oct) | (1u << 8)) : 0u;
-                    }
                 }
             }
             if (!done && (ng_bits & 255u)) {

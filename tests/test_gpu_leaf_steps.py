@@ -45,7 +45,11 @@ def test_stacked_triangles(ctx, planes, rays):
     _check(ctx, planes, rays, 1.0)
 
 
-@pytest.mark.parametrize("log2", [-60, -20, 20, 30, 45])
+# the triangle test's FP32 products are cubic in the lengths: they vanish at 2^-60 and overflow at 2^45
+_range = pytest.mark.xfail(strict=True, reason="cubic products leave the FP32 range")
+
+
+@pytest.mark.parametrize("log2", [pytest.param(-60, marks=_range), -20, 20, 30, pytest.param(45, marks=_range)])
 def test_stacked_triangles_at_other_scales(ctx, log2):
     """Powers of two, exact again; rays along an axis in a large scene overflow the node test's scaled slopes."""
     _check(ctx, 9, 513, 2.0 ** log2)

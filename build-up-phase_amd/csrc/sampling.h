@@ -50,7 +50,9 @@ __device__ inline void cosine_dir(const float* n, float u1, float u2, float* d) 
     onb(n, t, b);
     const float r = sqrtf(u1);
     const float phi = 6.28318530717958647692f * u2;
-    const float lx = r * cosf(phi), ly = r * sinf(phi), lz = sqrtf(fmaxf(0.0f, 1.0f - u1));
+    float sn, cs;
+    sincosf(phi, &sn, &cs);  // one argument reduction for both; the bits of sinf and cosf for every 24-bit u2
+    const float lx = r * cs, ly = r * sn, lz = sqrtf(fmaxf(0.0f, 1.0f - u1));
 #pragma unroll
     for (int a = 0; a < 3; ++a) d[a] = lx * t[a] + ly * b[a] + lz * n[a];
 }

@@ -44,8 +44,8 @@ hipError_t nrc_step(NrcState& st, const rtx_nrc_sample* samples, uint32_t n, flo
                     hipStream_t stream);
 // Adam steps over a device-resident sample count: batch b of ceil(count / batch_size) interleaved batches takes
 // samples b, b + nb, b + 2 nb, ...; steps b >= nb return at once.  The enqueued work does not depend on the count,
-// so a frame needs no host round trip (and can be captured).  Launches max_batches steps, then advances the step
-// counter by nb.
+// so a frame needs no host round trip (and can be captured).  Launches max_batches steps, each of which
+// that runs advances the step counter.
 hipError_t nrc_steps_device(NrcState& st, const rtx_nrc_sample* samples, const uint32_t* count_dev,
                             uint32_t max_batches, hipStream_t stream);
 

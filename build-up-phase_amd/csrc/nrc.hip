@@ -12,12 +12,14 @@
 // and pre-permute the next layer's weight columns the same way (fragment packing below).  Activations never
 // leave registers between layers.
 //
-// Training: one 256-thread block = 4 waves x 16 samples.  Forward activations are also written to LDS as
+// Training: one block = 64 samples, 16 each for its first four waves.  Forward activations are also written to LDS as
 // A^T[unit][64 samples] (bf16); the backward data gradient uses W^T as the A operand (same trick); the weight
-// gradient dW = G^T (out x 64) * A (64 x in) is an MFMA GEMM over the 64 samples of the block whose A operand
-// (G^T rows) and B operand (A^T rows) are 16-byte LDS reads.  Each block writes its partial gradient and loss; a
-// second kernel sums the partials in block order (deterministic), applies Adam and writes the updated weights'
-// BF16 fragments.
+// gradient dW = G^T (out x 64) * A (64 x in) is an MFMA GEMM over the 64 samples of the block whose operands (G^T
+// rows, A^T rows) are 16-byte LDS reads.  It falls to four further waves, a layer behind the data gradients of the
+// first four (two G^T buffers).  Bound by latency (a block per CU at 16,384 samples: forward 5 us) and by writing 24 MB
+// of partial gradients: 16.0 us with four waves doing both, now 12.7 us (a step after another one 19.7 and 18.7 us).
+// Each block writes its partial gradient and loss; a second kernel sums the partials in block order (deterministic),
+// applies Adam and writes the updated weights' BF16 fragments.
 #include <cmath>
 
 #include "nrc.h"
@@ -96,50 +98,96 @@ __device__ __forceinline__ void load_query(const rtx_nrc_query* src, rtx_nrc_que
     q.albedo[0] = c.y; q.albedo[1] = c.z; q.albedo[2] = c.w;
 }
 
-// B fragments of the input layer for the lane's sample: k = 32s + 8g + j, i.e. the lane fills the 8-feature chunk
-// c = 4s + g at step s.  Chunks 0..8 are frequency chunks (axis c / 3, frequencies 4(c % 3) .. 4(c % 3) + 3, sin
-// and cos interleaved), so each lane evaluates one sin/cos pair and three angle doublings per step; chunk 9
-// holds normal, direction and albedo[0..1], chunk 10 albedo[2], chunk 11 zeros.
+// Input features: 12 chunks of 8.  Chunks 0..8 are frequency chunks (axis c / 3, frequencies 4(c % 3) ..
+// 4(c % 3) + 3, sin and cos interleaved): one sin/cos pair and three angle doublings.  Chunk 9 holds normal, direction
+// and albedo[0..1], chunk 10 albedo[2], chunk 11 zeros.
+__device__ __forceinline__ u32x4 pack_features(const float* v) {
+    u32x4 w;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const f32x2 f = {v[2 * j], v[2 * j + 1]};
+        w[j] = __builtin_bit_cast(unsigned, __builtin_convertvector(f, bf16x2));
+    }
+    return w;
+}
+
+__device__ __forceinline__ u32x4 frequency_chunk(const float* pn, int c) {
+    const int a = c / 3, k0 = 4 * (c - 3 * a);
+    const float p = a == 0 ? pn[0] : (a == 1 ? pn[1] : pn[2]);
+    // sin / cos of 2^k0 pi p, then three angle doublings: sin 2x = 2 sin x cos x, cos 2x = (cos x - sin x)
+    // (cos x + sin x); each doubling at most doubles the absolute error (a few FP32 ulps after three, far
+    // below the BF16 rounding of the features)
+    float v[8];
+    float sn, cs;
+    sincospif(ldexpf(p, k0), &sn, &cs);
+    v[0] = sn;
+    v[1] = cs;
+#pragma unroll
+    for (int i = 1; i < 4; ++i) {
+        const float s2 = 2.0f * sn * cs;
+        const float c2 = (cs - sn) * (cs + sn);
+        sn = s2;
+        cs = c2;
+        v[2 * i] = sn;
+        v[2 * i + 1] = cs;
+    }
+    return pack_features(v);
+}
+
+__device__ __forceinline__ u32x4 other_chunk(const rtx_nrc_query& q, int c) {
+    const float c9[8] = {q.normal[0],    q.normal[1],    q.normal[2], q.direction[0],
+                         q.direction[1], q.direction[2], q.albedo[0], q.albedo[1]};
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = c == 9 ? c9[j] : (c == 10 && j == 0 ? q.albedo[2] : 0.0f);
+    return pack_features(v);
+}
+
+__device__ __forceinline__ void box_position(const rtx_nrc_query& q, const Norm& nm, float* pn) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) pn[a] = (q.position[a] - nm.lo[a]) * nm.inv[a];
+}
+
+// B fragments of the input layer for the lane's sample: k = 32s + 8g + j, i.e. the lane fills chunk c = 4s + g at step
+// s.  Lanes without a sample get zeros (their activations meet zero gradients).
 __device__ __forceinline__ void encode(const rtx_nrc_query& q, const Norm& nm, int g, bool valid, bf16x8* in0,
                                        __bf16* at0, int col) {
     float pn[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) pn[a] = (q.position[a] - nm.lo[a]) * nm.inv[a];
+    box_position(q, nm, pn);
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
         const int c = 4 * s + g;
-        float v[8];
-        if (c < 9) {
-            const int a = c / 3, k0 = 4 * (c - 3 * a);
-            const float p = a == 0 ? pn[0] : (a == 1 ? pn[1] : pn[2]);
-            // sin / cos of 2^k0 pi p, then three angle doublings: sin 2x = 2 sin x cos x, cos 2x = (cos x - sin x)
-            // (cos x + sin x); each doubling at most doubles the absolute error (a few FP32 ulps after three, far
-            // below the BF16 rounding of the features)
-            float sn, cs;
-            sincospif(ldexpf(p, k0), &sn, &cs);
-            v[0] = sn;
-            v[1] = cs;
+        u32x4 w = c < 9 ? frequency_chunk(pn, c) : other_chunk(q, c);
+        if (!valid) w = u32x4{0u, 0u, 0u, 0u};
+        in0[s] = __builtin_bit_cast(bf16x8, w);
 #pragma unroll
-            for (int i = 1; i < 4; ++i) {
-                const float s2 = 2.0f * sn * cs;
-                const float c2 = (cs - sn) * (cs + sn);
-                sn = s2;
-                cs = c2;
-                v[2 * i] = sn;
-                v[2 * i + 1] = cs;
-            }
-        } else {
-            const float c9[8] = {q.normal[0],    q.normal[1],    q.normal[2], q.direction[0],
-                                 q.direction[1], q.direction[2], q.albedo[0], q.albedo[1]};
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = c == 9 ? c9[j] : (c == 10 && j == 0 ? q.albedo[2] : 0.0f);
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            in0[s][j] = (__bf16)(valid ? v[j] : 0.0f);
-            if (at0) at0[lds_idx(8 * c + j, col)] = in0[s][j];
-        }
+        for (int j = 0; j < 8; ++j) at0[lds_idx(8 * c + j, col)] = in0[s][j];
     }
+}
+
+// The same for the two queries of a pair of tiles, lanes without a query included (inference drops their outputs).  In
+// step 2 only k-group 0 has a frequency chunk, so k-group 1 computes it for the second query.
+__device__ __forceinline__ void encode_pair(const rtx_nrc_query& qa, const rtx_nrc_query& qb, const Norm& nm, int g,
+                                            bf16x8* ina, bf16x8* inb) {
+    float pa[3], pb[3];
+    box_position(qa, nm, pa);
+    box_position(qb, nm, pb);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        ina[s] = __builtin_bit_cast(bf16x8, frequency_chunk(pa, 4 * s + g));
+        inb[s] = __builtin_bit_cast(bf16x8, frequency_chunk(pb, 4 * s + g));
+    }
+    const float pz[3] = {0.0f, 0.0f, g == 0 ? pa[2] : pb[2]};
+    const u32x4 last = frequency_chunk(pz, 8);
+    u32x4 wa = other_chunk(qa, 8 + g), wb = other_chunk(qb, 8 + g);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const unsigned from = (unsigned)__shfl_down((int)last[j], 16);
+        wa[j] = g == 0 ? last[j] : wa[j];
+        wb[j] = g == 0 ? from : wb[j];
+    }
+    ina[2] = __builtin_bit_cast(bf16x8, wa);
+    inb[2] = __builtin_bit_cast(bf16x8, wb);
 }
 
 // ReLU and repack 4 output tiles into the 2 B fragments of the next layer (k order kperm).  The values are
@@ -169,13 +217,18 @@ __device__ __forceinline__ void store_act(const bf16x8* in, __bf16* at, int g, i
         for (int j = 0; j < 8; ++j) at[lds_idx(kperm(s, g, j), col)] = in[s][j];
 }
 
-// Inference, LDS-staged: a persistent block copies the 46 forward fragments (46 KB) into LDS once, then each wave
-// runs two 16-query tiles per pass so that every fragment read from LDS feeds two MFMAs (weights are the A operand,
-// queries the N dimension).  Each tile sees exactly the operations of the training kernel's forward pass.
+// Inference, LDS-staged: a persistent block copies the 46 forward fragments (46 KB) and the biases into LDS once, then
+// each wave runs two 16-query tiles per pass so that every fragment read from LDS feeds two MFMAs (weights are the A
+// operand, queries the N dimension).  Each tile sees exactly the operations of the training kernel's forward pass.
+// Bound by instruction issue: 590 vector instructions (five sin/cos pairs with their doublings, the packing) and 92
+// MFMAs a pass, whose times add up.  512 threads share the fragments, so that 24 waves fit a CU: 2.07M queries
+// 115 us, 150 us with 256 threads (12 waves), global bias reads and six sin/cos pairs.  Four tiles a pass halve the
+// LDS reads and change nothing.
 constexpr int kInferLdsFrags = kFwdFrags * 64;  // bf16x8 entries
+constexpr int kInferThreads = 512;
 
 template <int L>
-__device__ __forceinline__ void layer_forward2(const bf16x8* __restrict__ frag, const float* __restrict__ params,
+__device__ __forceinline__ void layer_forward2(const bf16x8* frag, const f32x4* bias,
                                                const bf16x8* inA, const bf16x8* inB, f32x4* accA, f32x4* accB,
                                                int lane) {
     constexpr int T = out_dim(L) / 16, S = in_dim(L) / 32;
@@ -183,9 +236,7 @@ __device__ __forceinline__ void layer_forward2(const bf16x8* __restrict__ frag, 
 #pragma unroll
     for (int t = 0; t < T; ++t) {
         // the bias is the accumulator's initial value (no separate adds after the products)
-        f32x4 cA, cB;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) cA[i] = cB[i] = params[b_off(L) + 16 * t + 4 * g + i];
+        f32x4 cA = bias[16 * L + 4 * t + g], cB = cA;
 #pragma unroll
         for (int s = 0; s < S; ++s) {
             const bf16x8 a = frag[(fwd_base(L) + t * S + s) * 64 + lane];
@@ -197,13 +248,15 @@ __device__ __forceinline__ void layer_forward2(const bf16x8* __restrict__ frag, 
     }
 }
 
-__global__ __launch_bounds__(256) void nrc_infer_lds_kernel(const bf16x8* __restrict__ fwd,
+__global__ __launch_bounds__(kInferThreads) __attribute__((amdgpu_waves_per_eu(6))) void nrc_infer_lds_kernel(const bf16x8* __restrict__ fwd,
                                                             const float* __restrict__ params,
                                                             const rtx_nrc_query* __restrict__ queries, uint32_t n,
                                                             const uint32_t* __restrict__ n_dev, Norm nm,
                                                             float* __restrict__ out_rgb, InferGather gt) {
     __shared__ bf16x8 frag[kInferLdsFrags];
     for (int i = threadIdx.x; i < kInferLdsFrags; i += blockDim.x) frag[i] = fwd[i];
+    __shared__ f32x4 bias[(5 * 64 + 16) / 4];  // layer L's at 16 L
+    for (int i = threadIdx.x; i < 5 * 64 + 16; i += blockDim.x) ((float*)bias)[i] = params[b_off(i >> 6) + (i & 63)];
     __syncthreads();
     if (n_dev) n = min(n, *n_dev);
     const int lane = threadIdx.x & 63;
@@ -221,26 +274,25 @@ __global__ __launch_bounds__(256) void nrc_infer_lds_kernel(const bf16x8* __rest
         if (vA) load_query(queries + iA, qA);
         if (vB) load_query(queries + iB, qB);
         bf16x8 inA[3], inB[3];
-        encode(qA, nm, g, vA, inA, nullptr, 0);
-        encode(qB, nm, g, vB, inB, nullptr, 0);
+        encode_pair(qA, qB, nm, g, inA, inB);
         bf16x8 aA[2], aB[2];
         f32x4 accA[4], accB[4];
-        layer_forward2<0>(frag, params, inA, inB, accA, accB, lane_f);
+        layer_forward2<0>(frag, bias, inA, inB, accA, accB, lane_f);
         relu_pack(accA, aA);
         relu_pack(accB, aB);
-        layer_forward2<1>(frag, params, aA, aB, accA, accB, lane_f);
+        layer_forward2<1>(frag, bias, aA, aB, accA, accB, lane_f);
         relu_pack(accA, aA);
         relu_pack(accB, aB);
-        layer_forward2<2>(frag, params, aA, aB, accA, accB, lane_f);
+        layer_forward2<2>(frag, bias, aA, aB, accA, accB, lane_f);
         relu_pack(accA, aA);
         relu_pack(accB, aB);
-        layer_forward2<3>(frag, params, aA, aB, accA, accB, lane_f);
+        layer_forward2<3>(frag, bias, aA, aB, accA, accB, lane_f);
         relu_pack(accA, aA);
         relu_pack(accB, aB);
-        layer_forward2<4>(frag, params, aA, aB, accA, accB, lane_f);
+        layer_forward2<4>(frag, bias, aA, aB, accA, accB, lane_f);
         relu_pack(accA, aA);
         relu_pack(accB, aB);
-        layer_forward2<5>(frag, params, aA, aB, accA, accB, lane_f);
+        layer_forward2<5>(frag, bias, aA, aB, accA, accB, lane_f);
         if (g == 0) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -266,40 +318,40 @@ __global__ __launch_bounds__(256) void nrc_infer_lds_kernel(const bf16x8* __rest
     }
 }
 
-// LDS of the training kernel (64 samples): A^T of the layer inputs and G^T of the current layer.
+// LDS of the training kernel (64 samples): A^T of the layer inputs, G^T of the current layer and of the one before.
 struct TrainLds {
     __bf16 at0[96 * 64];
     __bf16 at[5][64 * 64];
-    __bf16 gt[64 * 64];
-    float red[8];
+    __bf16 gt[2][64 * 64];
+    float red[4];
 };
 
-// Weight gradient of layer L for the block's 64 samples: dW tile (t, u) = G^T rows * A columns.
+// Weight gradient of layer L for the block's 64 samples: dW tile (t, u) = G^T rows * A columns; `wave` of `waves`
+// takes every waves-th tile.
 template <int L>
-__device__ __forceinline__ void weight_grad(TrainLds& sm, const __bf16* at, float* __restrict__ part, int wave,
-                                            int lane) {
+__device__ __forceinline__ void weight_grad(const __bf16* gt, const __bf16* at, float* __restrict__ part, int wave,
+                                            int waves, int lane) {
     constexpr int T = out_dim(L) / 16, U = in_dim(L) / 16, N = T * U;
     const int r = lane & 15, g = lane >> 4;
 #pragma unroll
-    for (int k = wave; k < N; k += 4) {
+    for (int k = wave; k < N; k += waves) {
         const int t = k / U, u = k % U;
         f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
-            const bf16x8 a = *(const bf16x8*)(sm.gt + lds_idx(16 * t + r, 32 * s + 8 * g));
+            const bf16x8 a = *(const bf16x8*)(gt + lds_idx(16 * t + r, 32 * s + 8 * g));
             const bf16x8 b = *(const bf16x8*)(at + lds_idx(16 * u + r, 32 * s + 8 * g));
-            c = mfma(a, b, c);
+            c = mfma(b, a, c);  // transposed: the lane's four results lie in one row of dW
         }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) part[w_off(L) + (16 * t + 4 * g + i) * in_dim(L) + 16 * u + r] = c[i];
+        *(f32x4*)(part + w_off(L) + (16 * t + r) * in_dim(L) + 16 * u + 4 * g) = c;
     }
     // bias gradient: sum over the 64 samples of G^T rows; 4 lanes per row (16 samples each), then a shuffle sum
-    const int row = threadIdx.x >> 2, q = threadIdx.x & 3;
+    const int row = wave * 16 + (lane >> 2), q = lane & 3;
     if (row < out_dim(L)) {
         float sum = 0.0f;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const bf16x8 v = *(const bf16x8*)(sm.gt + lds_idx(row, 16 * q + 8 * h));
+            const bf16x8 v = *(const bf16x8*)(gt + lds_idx(row, 16 * q + 8 * h));
 #pragma unroll
             for (int j = 0; j < 8; ++j) sum += (float)v[j];
         }
@@ -379,23 +431,40 @@ __device__ __forceinline__ void store_grad(const f32x4* gv, int tiles, __bf16* g
         }
 }
 
-__global__ __launch_bounds__(256) void nrc_train_kernel(const bf16x8* __restrict__ fwd, const bf16x8* __restrict__ bwd,
+constexpr int kTrainThreads = 512;
+__global__ __launch_bounds__(kTrainThreads) void nrc_train_kernel(const bf16x8* __restrict__ fwd, const bf16x8* __restrict__ bwd,
                                                         const float* __restrict__ params,
                                                         const rtx_nrc_sample* __restrict__ samples, StepShape shape,
                                                         Norm nm, float* __restrict__ partials,
-                                                        float* __restrict__ loss_part) {
+                                                        float* __restrict__ loss_part, uint32_t* __restrict__ steps) {
     __shared__ TrainLds sm;
     uint32_t n, stride, offset;
     // a step that does not run, and blocks past the step's samples, leave at once (the whole block alike)
     if (!step_samples(shape, n, stride, offset) || blockIdx.x * 64u >= n) return;
+    if (steps && blockIdx.x == 0 && threadIdx.x == 0) ++*steps;  // the Adam kernel that follows takes this step
     const float inv_n = 1.0f / (float)n;
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, g = lane >> 4;
+    float* part = partials + (uint64_t)blockIdx.x * RTX_NRC_PARAM_COUNT;
+    if (wave >= 4) {  // the weight gradients of a layer, while the first four waves go on to the layer before
+        __syncthreads();
+        weight_grad<5>(sm.gt[0], sm.at[4], part, wave - 4, 4, lane);
+        __syncthreads();
+        weight_grad<4>(sm.gt[1], sm.at[3], part, wave - 4, 4, lane);
+        __syncthreads();
+        weight_grad<3>(sm.gt[0], sm.at[2], part, wave - 4, 4, lane);
+        __syncthreads();
+        weight_grad<2>(sm.gt[1], sm.at[1], part, wave - 4, 4, lane);
+        __syncthreads();
+        weight_grad<1>(sm.gt[0], sm.at[0], part, wave - 4, 4, lane);
+        __syncthreads();
+        weight_grad<0>(sm.gt[1], sm.at0, part, wave, 8, lane);
+        return;
+    }
     const int col = wave * 16 + c;  // sample column within the block
     const uint64_t idx = (uint64_t)blockIdx.x * 64 + col;
     const bool valid = idx < n;
-    float* part = partials + (uint64_t)blockIdx.x * RTX_NRC_PARAM_COUNT;
     bf16x8 fa[12], fb[8];  // fragments of the current and the next layer
     float ba[16], bb[16];
     load_fwd_layer<0>(fwd, params, lane, fa, ba);
@@ -450,46 +519,34 @@ __global__ __launch_bounds__(256) void nrc_train_kernel(const bf16x8* __restrict
         }
     }
     bf16x8 gfrag[2];
-    store_grad(gy, 1, sm.gt, g, col, gfrag);
-    __syncthreads();
-    load_bwd_layer<4>(bwd, lane, fb);
-    weight_grad<5>(sm, sm.at[4], part, wave, lane);
-    f32x4 gv[4];
-    back_data<5>(fa, gfrag, acts[4], gv);
-    __syncthreads();
-    store_grad(gv, 4, sm.gt, g, col, gfrag);
-    __syncthreads();
-    load_bwd_layer<3>(bwd, lane, fa);
-    weight_grad<4>(sm, sm.at[3], part, wave, lane);
-    back_data<4>(fb, gfrag, acts[3], gv);
-    __syncthreads();
-    store_grad(gv, 4, sm.gt, g, col, gfrag);
-    __syncthreads();
-    load_bwd_layer<2>(bwd, lane, fb);
-    weight_grad<3>(sm, sm.at[2], part, wave, lane);
-    back_data<3>(fa, gfrag, acts[2], gv);
-    __syncthreads();
-    store_grad(gv, 4, sm.gt, g, col, gfrag);
-    __syncthreads();
-    load_bwd_layer<1>(bwd, lane, fa);
-    weight_grad<2>(sm, sm.at[1], part, wave, lane);
-    back_data<2>(fb, gfrag, acts[1], gv);
-    __syncthreads();
-    store_grad(gv, 4, sm.gt, g, col, gfrag);
-    __syncthreads();
-    weight_grad<1>(sm, sm.at[0], part, wave, lane);
-    back_data<1>(fa, gfrag, acts[0], gv);
-    __syncthreads();
-    store_grad(gv, 4, sm.gt, g, col, gfrag);
-    __syncthreads();
-    weight_grad<0>(sm, sm.at0, part, wave, lane);
-
+    store_grad(gy, 1, sm.gt[0], g, col, gfrag);
     // block loss
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
     if (lane == 0) sm.red[wave] = loss;
     __syncthreads();
     if (threadIdx.x == 0) loss_part[blockIdx.x] = (sm.red[0] + sm.red[1] + sm.red[2] + sm.red[3]) * inv_n;
+    f32x4 gv[4];
+    load_bwd_layer<4>(bwd, lane, fb);
+    back_data<5>(fa, gfrag, acts[4], gv);
+    store_grad(gv, 4, sm.gt[1], g, col, gfrag);
+    __syncthreads();
+    load_bwd_layer<3>(bwd, lane, fa);
+    back_data<4>(fb, gfrag, acts[3], gv);
+    store_grad(gv, 4, sm.gt[0], g, col, gfrag);
+    __syncthreads();
+    load_bwd_layer<2>(bwd, lane, fb);
+    back_data<3>(fa, gfrag, acts[2], gv);
+    store_grad(gv, 4, sm.gt[1], g, col, gfrag);
+    __syncthreads();
+    load_bwd_layer<1>(bwd, lane, fa);
+    back_data<2>(fb, gfrag, acts[1], gv);
+    store_grad(gv, 4, sm.gt[0], g, col, gfrag);
+    __syncthreads();
+    back_data<1>(fa, gfrag, acts[0], gv);
+    store_grad(gv, 4, sm.gt[1], g, col, gfrag);
+    __syncthreads();
+    weight_grad<0>(sm.gt[1], sm.at0, part, wave, 8, lane);
 }
 
 // BF16 copy of weight p into its forward fragment slot and, for layers 1..5, its backward fragment slot: the
@@ -515,25 +572,31 @@ __device__ __forceinline__ void scatter_weight(int p, float w, __bf16* __restric
 }
 
 // Sum the block partials and take one Adam step (writing the BF16 fragments of the updated weights), or only
-// write the gradient.  A block covers 16 parameters with 16 threads each; thread k sums partials k, k + 16, ...
-// and a fixed LDS tree adds the 16 slices (deterministic).  The extra last block sums the per-block losses the
-// same way.
-__global__ __launch_bounds__(256) void nrc_adam_kernel(const float* __restrict__ partials, StepShape shape,
+// write the gradient.  A block covers 64 parameters: thread (k, q) sums partials k, k + 16, ... of four of them and a
+// fixed LDS tree adds the 16 slices (deterministic); its fifth wave computes the bias corrections meanwhile.  The extra
+// last block sums the per-block losses the same way.  Bound by reading the partials (256 blocks: 24 MB): 16-byte
+// reads of 256-byte row pieces, all of a thread's in flight; with 4-byte reads of 64-byte pieces and the corrections
+// after the sums 11.2 us, now 7.0 us.
+constexpr uint32_t kAdamParams = 64;
+static_assert(RTX_NRC_PARAM_COUNT % 4 == 0, "a thread's four parameters");
+__global__ __launch_bounds__(320) void nrc_adam_kernel(const float* __restrict__ partials, StepShape shape,
                                                        float* __restrict__ params, float* __restrict__ m,
                                                        float* __restrict__ v, float lr, float b1, float b2, float eps,
                                                        const uint32_t* __restrict__ steps, float* __restrict__ grad_out,
                                                        __bf16* __restrict__ fwd, __bf16* __restrict__ bwd,
                                                        const float* __restrict__ loss_part,
                                                        float* __restrict__ loss_out) {
-    __shared__ float s[16][17];
+    __shared__ f32x4 s[16][17];
+    __shared__ float corr[2];
     uint32_t n, stride, offset;
     if (!step_samples(shape, n, stride, offset)) return;
     const uint32_t nblk = (n + 63) / 64;
     if (blockIdx.x == gridDim.x - 1) {
         __shared__ float ls[256];
         float a = 0.0f;
-        for (uint32_t b = threadIdx.x; b < nblk; b += 256) a += loss_part[b];
-        ls[threadIdx.x] = a;
+        if (threadIdx.x < 256)
+            for (uint32_t b = threadIdx.x; b < nblk; b += 256) a += loss_part[b];
+        if (threadIdx.x < 256) ls[threadIdx.x] = a;
         __syncthreads();
         for (uint32_t h = 128; h > 0; h >>= 1) {
             if (threadIdx.x < h) ls[threadIdx.x] += ls[threadIdx.x + h];
@@ -542,32 +605,38 @@ __global__ __launch_bounds__(256) void nrc_adam_kernel(const float* __restrict__
         if (threadIdx.x == 0) *loss_out = ls[0];
         return;
     }
-    const uint32_t pi = threadIdx.x & 15u, k = threadIdx.x >> 4;
-    const uint32_t p = blockIdx.x * 16u + pi;
-    float acc = 0.0f;
-    if (p < RTX_NRC_PARAM_COUNT)
-        for (uint32_t b = k; b < nblk; b += 16) acc += partials[(uint64_t)b * RTX_NRC_PARAM_COUNT + p];
-    s[k][pi] = acc;
+    const uint32_t q = threadIdx.x & 15u, k = threadIdx.x >> 4;
+    const uint32_t p4 = blockIdx.x * kAdamParams + 4u * q;
+    if (k < 16) {
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (p4 < RTX_NRC_PARAM_COUNT) {
+            const float* src = partials + p4;
+#pragma unroll 16
+            for (uint32_t b = k; b < nblk; b += 16) acc += *(const f32x4*)(src + (uint64_t)b * RTX_NRC_PARAM_COUNT);
+        }
+        s[k][q] = acc;
+    } else if (threadIdx.x < 258 && !grad_out) {
+        // bias corrections of step t, 1 / (1 - beta^t), in FP64, rounded
+        const double t = (double)*steps;
+        corr[threadIdx.x - 256] = (float)(1.0 / (1.0 - pow((double)(threadIdx.x == 256 ? b1 : b2), t)));
+    }
     __syncthreads();
     for (uint32_t h = 8; h > 0; h >>= 1) {
-        if (k < h) s[k][pi] += s[k + h][pi];
+        if (k < h) s[k][q] += s[k + h][q];
         __syncthreads();
     }
-    if (k != 0 || p >= RTX_NRC_PARAM_COUNT) return;
-    const float gsum = s[0][pi];
+    const uint32_t p = blockIdx.x * kAdamParams + threadIdx.x;
+    if (threadIdx.x >= kAdamParams || p >= RTX_NRC_PARAM_COUNT) return;
+    const float gsum = ((const float*)s[0])[threadIdx.x];
     if (grad_out) {
         grad_out[p] = gsum;
         return;
     }
-    // bias corrections of step t = steps taken + this batch's index + 1 (FP64, rounded)
-    const double t = (double)(*steps + shape.batch + 1u);
-    const float c1 = (float)(1.0 / (1.0 - pow((double)b1, t)));
-    const float c2 = (float)(1.0 / (1.0 - pow((double)b2, t)));
     const float mm = b1 * m[p] + (1.0f - b1) * gsum;
     const float vv = b2 * v[p] + (1.0f - b2) * gsum * gsum;
     m[p] = mm;
     v[p] = vv;
-    const float w = params[p] - lr * (mm * c1) / (sqrtf(vv * c2) + eps);
+    const float w = params[p] - lr * (mm * corr[0]) / (sqrtf(vv * corr[1]) + eps);
     params[p] = w;
     scatter_weight((int)p, w, fwd, bwd);
 }
@@ -630,36 +699,31 @@ static Norm make_norm(const NrcState& st) {
 hipError_t nrc_infer(const NrcState& st, const rtx_nrc_query* q, uint32_t n, float* out, hipStream_t s,
                      const uint32_t* n_dev, const InferGather* gather) {
     if (n == 0) return hipSuccess;
-    // persistent LDS-staged kernel: up to 3 blocks per CU (46 KB of fragments each), each wave looping over pairs
-    // of 16-query tiles
+    // persistent LDS-staged kernel: up to 3 blocks per CU (47 KB of fragments and biases each), each wave looping over
+    // pairs of 16-query tiles
     const uint64_t pairs = ((uint64_t)n + 31) / 32;
-    const uint64_t want = (pairs + 3) / 4;
+    const uint64_t want = (pairs + kInferThreads / 64 - 1) / (kInferThreads / 64);
     const unsigned blocks = (unsigned)std::min<uint64_t>(want, (uint64_t)st.cu_count * 3);
-    nrc_infer_lds_kernel<<<blocks, 256, 0, s>>>((const bf16x8*)st.fwd, st.params, q, n, n_dev, make_norm(st), out,
+    nrc_infer_lds_kernel<<<blocks, kInferThreads, 0, s>>>((const bf16x8*)st.fwd, st.params, q, n, n_dev, make_norm(st), out,
                                                  gather ? *gather : InferGather{});
     return hipGetLastError();
-}
-
-// Adds the steps just taken to the step counter: one (host-sized step) or ceil(count / batch_size).
-__global__ void nrc_advance_kernel(uint32_t* steps, const uint32_t* count_dev, uint32_t batch_size) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    *steps += count_dev ? (*count_dev + batch_size - 1) / batch_size : 1u;
 }
 
 // One training step (gradient kernel + Adam kernel) of the given shape; the grid covers the largest batch.
 static hipError_t launch_step(NrcState& st, const rtx_nrc_sample* samples, const StepShape& shape, uint32_t nblk,
                               float* grad_out, float* loss_out, hipStream_t s) {
     float* loss = loss_out ? loss_out : st.loss;
-    nrc_train_kernel<<<nblk, 256, 0, s>>>((const bf16x8*)st.fwd, (const bf16x8*)st.bwd, st.params, samples, shape,
-                                          make_norm(st), st.partials, st.loss_part);
-    // one block per 16 parameters + the loss block
-    const unsigned pb = (RTX_NRC_PARAM_COUNT + 15) / 16 + 1;
+    nrc_train_kernel<<<nblk, kTrainThreads, 0, s>>>((const bf16x8*)st.fwd, (const bf16x8*)st.bwd, st.params, samples, shape,
+                                          make_norm(st), st.partials, st.loss_part,
+                                          grad_out ? nullptr : st.steps_dev);
+    // the parameters' blocks + the loss block
+    const unsigned pb = (RTX_NRC_PARAM_COUNT + kAdamParams - 1) / kAdamParams + 1;
     if (grad_out) {
-        nrc_adam_kernel<<<pb, 256, 0, s>>>(st.partials, shape, st.params, st.m, st.v, 0, 0, 0, 0, st.steps_dev,
+        nrc_adam_kernel<<<pb, 320, 0, s>>>(st.partials, shape, st.params, st.m, st.v, 0, 0, 0, 0, st.steps_dev,
                                            grad_out, nullptr, nullptr, st.loss_part, loss);
         return hipGetLastError();
     }
-    nrc_adam_kernel<<<pb, 256, 0, s>>>(st.partials, shape, st.params, st.m, st.v, st.lr, st.beta1, st.beta2, st.eps,
+    nrc_adam_kernel<<<pb, 320, 0, s>>>(st.partials, shape, st.params, st.m, st.v, st.lr, st.beta1, st.beta2, st.eps,
                                        st.steps_dev, nullptr, (__bf16*)st.fwd, (__bf16*)st.bwd, st.loss_part, loss);
     return hipGetLastError();
 }
@@ -669,10 +733,7 @@ hipError_t nrc_step(NrcState& st, const rtx_nrc_sample* samples, uint32_t n, flo
     if (n == 0) return hipSuccess;
     const uint32_t nblk = (n + 63) / 64;
     if (nblk > st.max_blocks) return hipErrorInvalidValue;
-    hipError_t e = launch_step(st, samples, StepShape{nullptr, n, 0u, st.batch_size}, nblk, grad_out, loss_out, s);
-    if (e || grad_out) return e;
-    nrc_advance_kernel<<<1, 64, 0, s>>>(st.steps_dev, nullptr, st.batch_size);
-    return hipGetLastError();
+    return launch_step(st, samples, StepShape{nullptr, n, 0u, st.batch_size}, nblk, grad_out, loss_out, s);
 }
 
 hipError_t nrc_steps_device(NrcState& st, const rtx_nrc_sample* samples, const uint32_t* count_dev,
@@ -682,8 +743,7 @@ hipError_t nrc_steps_device(NrcState& st, const rtx_nrc_sample* samples, const u
                                    nullptr, s);
         if (e) return e;
     }
-    nrc_advance_kernel<<<1, 64, 0, s>>>(st.steps_dev, count_dev, st.batch_size);
-    return hipGetLastError();
+    return hipSuccess;
 }
 
 }  // namespace rtx

@@ -1002,6 +1002,7 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
 
         int iter = 0;
         bool go = true;
+        uint32_t busy_lanes = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(active));
         while (go) {
             bool done = false;
             uint32_t fault = 0;
@@ -1009,14 +1010,18 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
             // of triangles, the instance step (BLAS entry in FP64) once as many hold one of instances, and both when
             // no lane can traverse; until then lanes with a pending leaf keep traversing their node group, or wait.
             // (Lanes without a ray hold no group.)  Each has its own threshold, because an instance step costs twice a
-            // triangle step: with one for both 16.7M incoherent rays took 2.59 ms, now 2.41 ms.
+            // triangle step: with one for both 16.7M incoherent rays took 2.59 ms, now 2.41 ms.  leaf_lanes is for a
+            // full wave and shrinks with the rays that it still traces: half of a short launch is the tail of its
+            // longest rays (250 to 600 steps), which must not wait for each other (1080p film of dense alpha-tested
+            // geometry 1.15 -> 1.06 ms, 1277x719 film of 64 dense meshes 580 -> 515 us).
             const bool has_leaf = (lg_bits & 255u) != 0u;
             const bool enter = has_leaf && !in_blas;
             const uint32_t inst_lanes = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(enter));
             const uint64_t tri_lanes = __builtin_amdgcn_ballot_w64(has_leaf && in_blas);
             const bool no_node =
                 __builtin_amdgcn_ballot_w64((ng_bits & 255u) || (active && !(lg_bits & 255u))) == 0ull;
-            if (tri_lanes && ((uint32_t)__popcll(tri_lanes) >= args.leaf_lanes || no_node)) {
+            const uint32_t leaf_at = (busy_lanes * args.leaf_lanes + 63u) >> 6;
+            if (tri_lanes && ((uint32_t)__popcll(tri_lanes) >= leaf_at || no_node)) {
                 // The next two triangles of each leaf group, one per lane of the wave: 4 to 12 lanes hold a leaf
                 // group when the leaf step runs, most of them two triangles, so the owners hand theirs out and
                 // one pass of the whole wave tests them (two passes of the owners alone took 6,000 to 10,000
@@ -1139,7 +1144,7 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
                     }
                 }
             }
-            if ((inst_lanes >= args.leaf_lanes || no_node) && enter) {
+            if ((inst_lanes >= leaf_at || no_node) && enter) {
                 // instance leaf: enter its BLAS
                 const uint32_t m = lg_bits & 255u;
                 const uint32_t k = (uint32_t)(__ffs(m) - 1);
@@ -1308,8 +1313,8 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
                 ng_bits = 0;
                 sp = 0;
             }
-            const uint64_t busy = __builtin_amdgcn_ballot_w64(active);
-            go = busy != 0ull;
+            busy_lanes = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(active));
+            go = busy_lanes != 0u;
             if (++iter >= (int)args.refill_interval) {
                 iter = 0;
                 steps += args.refill_interval;
@@ -1319,8 +1324,7 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
                     ng_bits = 0;
                     sp = 0;
                 }
-                const uint32_t lanes = (uint32_t)__popcll(busy);
-                go = go && (kTrain ? lanes > train_floor : (wave_exhausted || lanes >= args.refill_lanes));
+                go = go && (kTrain ? busy_lanes > train_floor : (wave_exhausted || busy_lanes >= args.refill_lanes));
             }
         }
     }

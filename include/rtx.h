@@ -414,8 +414,9 @@ typedef struct rtx_trace_config {
                                  rays when every wave gets >= 8 chunks) */
     uint32_t refill_lanes;    /* a wave fetches new rays once fewer than this many of its 64 lanes are busy */
     uint32_t refill_interval; /* traversal steps between two refill checks (1..64) */
-    uint32_t leaf_lanes;      /* postponed leaves: a wave runs its leaf step (BLAS entry, triangle tests) once this
-                                 many lanes hold a pending leaf group or no lane can traverse (1..64; 1 = at once) */
+    uint32_t leaf_lanes;      /* postponed leaves: a wave enters BLASes, or tests triangles, once this many of 64 lanes
+                                 (proportionally fewer while it traces fewer rays) wait for that, or no lane can
+                                 traverse (1..64; 1 = at once) */
     uint32_t stack_limit;     /* traversal stack entries per lane, LDS and global spill together: 0 (default) sizes the
                                  stack from the traced TLAS's depth (2 entries per BVH level + 4, enough for every
                                  ray); with a smaller value a ray that needs more ends there (reporting the closest

@@ -2238,7 +2238,10 @@ Layout make_layout(uint32_t n, int key_bytes, uint32_t ngeom, uint32_t nbatch = 
     L.boxes = take(nn * 24);
     L.keys = take(nn * key_bytes);
     L.vals = take(nn * 4);
-    L.sort = take(sort_scratch_bytes(n, key_bytes));
+    // The bounds, read by the Morton codes alone, lie where the sort will; its look-back words of small tiles (up to 6 B
+    // a primitive and 24 KB, only between 4,097 and 131,071 primitives) reach into the links (16 B), written after it.
+    L.sort = take(sort_scratch_bytes(n, key_bytes) - sort_small_tile_bytes(n, key_bytes));
+    L.cbounds = L.sort;
     L.left = take(nn * 4);
     L.right = take(nn * 4);
     L.parent = take(2 * nn * 4);
@@ -2249,10 +2252,10 @@ Layout make_layout(uint32_t n, int key_bytes, uint32_t ngeom, uint32_t nbatch = 
     L.hgt = take(nn * 4);
     L.wcost = take(nn * 32);
     L.wdec = take(nn * 4);
-    L.subs = take(nn * 8 + 16ull * (nbatch ? nbatch : 1));  // subtree tasks: of two primitives or more, or a whole BLAS
+    // subtree tasks: of two primitives or more, or a whole BLAS
+    L.subs = take(16 * std::min<uint64_t>(nn, nn / 2 + (nbatch ? nbatch : 1)));
     L.queue = take(nn * 8);
     L.queue_words = take(sizeof(CollapseQueue));
-    L.cbounds = take(kBoundSlots * kBoundStride * 4);
     L.misc = take(64);
     L.geoms = take((uint64_t)(ngeom ? ngeom : 1) * sizeof(GeomDesc));
     if (nbatch) {

@@ -289,6 +289,12 @@ uint64_t sort_scratch_bytes(uint32_t n, int key_bytes) {
     return b;
 }
 
+uint64_t sort_small_tile_bytes(uint32_t n, int key_bytes) {
+    constexpr uint64_t large = (uint64_t)kSortBlock * kItemsLarge;
+    const uint64_t tiles = ((uint64_t)n + tile_keys(n) - 1) / tile_keys(n), least = (n + large - 1) / large;
+    return (uint64_t)key_bytes * (tiles - least) * kRadix * 4;
+}
+
 template <typename K>
 static hipError_t sort_pairs_impl(K* keys, uint32_t* vals, uint32_t n, int passes, void* scratch,
                                   uint32_t* err_flags, hipStream_t stream) {

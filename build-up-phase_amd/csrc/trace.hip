@@ -12,6 +12,7 @@
 //     happens on coordinates of the size of the BLAS box, not of the distance to the camera;
 //   * triangles: watertight test (Woop, Benthin & Wald 2013) with the shear written as three row vectors, so
 //     no per-lane component selection is needed per triangle; exact-zero edge functions are recomputed in FP64;
+//     the wave's lanes test the triangles of the lanes that hold a leaf group, two of each at a time;
 //   * traversal order: children are stored by octant; the group mask is permuted by the ray's sign octant so
 //     that lowest-bit-first visits near children first (Ylitie, Karras & Laine 2017 node groups);
 //   * stack: per-lane entries (slot base, child mask, valid mask, flags) in LDS, spilling to a global

@@ -520,9 +520,9 @@ __device__ __forceinline__ bool candidate_accepted(const TraceArgs& args, uint32
 
 // Ray ids per chunk of a launch of n rays on `waves` waves.  Automatic: at most one ray per lane is spread over all
 // waves (a wave of few rays diverges less, and the launch lasts as long as its slowest wave) where they all run at
-// once; otherwise 64, or for single rays 256 when every wave gets at least 8 chunks (neighbouring rays in one wave:
-// 16.7M camera rays 1.72 ms, 1.81 ms with 64; whole paths are too uneven for that: 4 samples of the 1080p Cornell
-// box 19.6 ms with 256, 18.8 ms with 64).
+// once; otherwise 64, or for single rays 256 when every wave gets at least 8 chunks (16.7M camera or incoherent rays
+// 1.3% faster than with 64, 3M any-hit rays 1% slower; whole paths are too uneven for that: 4 samples of the 1080p
+// Cornell box 13.6 ms with 256, 13.0 ms with 64).
 __host__ __device__ __forceinline__ uint32_t rays_per_chunk(uint32_t configured, uint32_t n, uint32_t waves,
                                                             uint32_t first_chunks, bool paths) {
     if (configured >= 64u) return configured;
@@ -995,8 +995,8 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
         const bool wave_exhausted = !more && pool_next >= pool_end;
         // Whole paths: back to the refill point (where ended rays continue their paths) once half of the lanes that
         // start this round (64 - refill_lanes of 32) have ended their rays, at least one.  Shading costs as much as
-        // five traversal steps, however few lanes shade: 4 samples of the 1080p Cornell box 15.0 ms with half of the
-        // lanes, 17.2 ms with a quarter, 15.8 ms with three quarters.
+        // five traversal steps, however few lanes shade: 4 samples of the 1080p Cornell box 13.0 ms with half of the
+        // lanes, 14.0 ms with a quarter, 13.8 ms with three quarters.
         uint32_t train_floor = 0;
         if (kTrain) {
             const uint32_t n0 = (uint32_t)__popcll(__ballot(active));

@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include "rtx_internal.h"
+#include "trace_rules.h"
 
 namespace rtx {
 

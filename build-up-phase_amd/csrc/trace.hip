@@ -1231,7 +1231,7 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
             // a lane without pending work pops its next group; a node group is taken on in this same step, also by the
             // lanes that have just tested their last triangles (popping at the start of a step: 4% slower)
             if (active && !done && !((lg_bits | ng_bits) & 255u)) {
-                if (sp > 0) {
+                if (pops_entry(sp, D + GD)) {
                     --sp;
                     const uint2 e = stacked(sp);
                     if ((e.y & kEntryTlas) && in_blas) {
@@ -1267,7 +1267,7 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
                         ng_bits = e.y & 0xFFFFu;
                     }
                 } else {
-                    done = true;
+                    done = true;  // no work left, or this step's pushes went past the end (an overflow, below)
                 }
             }
             if (!done && (ng_bits & 255u)) {

@@ -70,9 +70,11 @@ __device__ __forceinline__ uint4 load_words(SlotPtr p, int k) {
 }
 
 // Hit masks in traversal order, by octant and mask: child position k goes to bit k ^ octant.
-struct OctTable {
+struct alignas(16) OctTable {
     uint8_t row[8][256];
 };
+static_assert(alignof(OctTable) >= alignof(uint64_t) && sizeof(OctTable) % sizeof(uint64_t) == 0,
+              "blocks copy the table in 8-byte words");
 constexpr OctTable make_oct_table() {
     OctTable t{};
     for (uint32_t oct = 0; oct < 8; ++oct)

@@ -26,6 +26,7 @@
 //     with its next ray, so one launch traces whole paths.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "pt_shade.h"
 #include "rtx_internal.h"
@@ -75,6 +76,7 @@ struct alignas(16) OctTable {
 };
 static_assert(alignof(OctTable) >= alignof(uint64_t) && sizeof(OctTable) % sizeof(uint64_t) == 0,
               "blocks copy the table in 8-byte words");
+static_assert(sizeof(OctTable) == kOctTableBytes, "the launch rules' size");
 constexpr OctTable make_oct_table() {
     OctTable t{};
     for (uint32_t oct = 0; oct < 8; ++oct)
@@ -86,6 +88,13 @@ constexpr OctTable make_oct_table() {
     return t;
 }
 __constant__ OctTable kOctTable = make_oct_table();
+// The same computed: 16 vector instructions a node step, where the table in LDS would cost blocks.
+__device__ __forceinline__ uint32_t oct_permute(uint32_t m, uint32_t oct) {
+    if (oct & 1u) m = ((m & 0x55u) << 1) | ((m >> 1) & 0x55u);
+    if (oct & 2u) m = ((m & 0x33u) << 2) | ((m >> 2) & 0x33u);
+    if (oct & 4u) m = ((m & 0x0Fu) << 4) | ((m >> 4) & 0x0Fu);
+    return m;
+}
 
 // 1/d for the slab tests, |d| clamped to at least 2^-80.  v_rcp_f32 (1 ulp) on d * 2^-32 keeps the operand and
 // the result in the normal range for every |d| in [2^-80, 2^128); the node test's error margin (2^-20 relative
@@ -284,7 +293,7 @@ struct TraceArgs {
     uint32_t gdepth;
     uint32_t ray_chunk;        // ray ids per queue fetch (< 64: automatic)
     uint32_t guard;            // 1 / 2: the launch traces only if guard_passes
-    uint32_t first_chunks;     // 1: every wave's first chunk is its own, 0: all chunks come from the queues
+    uint32_t first_waves;      // waves whose first chunk is their own; the others take all chunks from the queues
     uint32_t refill_lanes;     // refill a wave once fewer lanes than this are busy
     uint32_t refill_interval;  // steps between refill checks
     uint32_t leaf_lanes;       // pending leaf groups needed before a leaf step runs
@@ -520,17 +529,6 @@ __device__ __forceinline__ bool candidate_accepted(const TraceArgs& args, uint32
     return any_hit_accepts(args, table + (cur_inst & kInstIdMask), geom, u, v);
 }
 
-// Ray ids per chunk of a launch of n rays on `waves` waves.  Automatic: at most one ray per lane is spread over all
-// waves (a wave of few rays diverges less, and the launch lasts as long as its slowest wave) where they all run at
-// once; otherwise 64, or for single rays 256 when every wave gets at least 8 chunks (16.7M camera or incoherent rays
-// 1.3% faster than with 64, 3M any-hit rays 1% slower; whole paths are too uneven for that: 4 samples of the 1080p
-// Cornell box 13.6 ms with 256, 13.0 ms with 64).
-__host__ __device__ __forceinline__ uint32_t rays_per_chunk(uint32_t configured, uint32_t n, uint32_t waves,
-                                                            uint32_t first_chunks, bool paths) {
-    if (configured >= 64u) return configured;
-    if (first_chunks && (uint64_t)n <= (uint64_t)waves * 64u) return n ? (n + waves - 1u) / waves : 1u;
-    return !paths && (uint64_t)n >= (uint64_t)waves * 64u * 8u ? 256u : 64u;
-}
 // Queues that a wave tries before it takes no more chunks.
 constexpr uint32_t kQueueHops = 3u;
 
@@ -543,7 +541,8 @@ __device__ __forceinline__ const void* reread_kernel_arguments() {
     return (const void*)(const __attribute__((address_space(4))) void*)p;
 }
 
-template <int MODE, bool STATS, bool FLAGS>
+// LEAN: no LDS but the stack and the world rays (plan_trace chooses).
+template <int MODE, bool STATS, bool FLAGS, bool LEAN>
 __device__ __forceinline__ void trace_body(const TraceArgs& args) {
     const uint32_t ray_flags = FLAGS ? args.ray_flags : 0u;  // the default variant compiles the flags out
     // dynamic LDS: the per-lane stack (lds_depth entries per lane); the FLAGS variant and the path-tracer modes
@@ -553,15 +552,17 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
     constexpr bool kTrain = MODE == kModeTrain || MODE == kModePixelPaths || MODE == kModePixelCache;  // whole paths
     constexpr int kShadeMode = MODE == kModePixelPaths ? (int)kPtPlain : (int)kPtCache;
     constexpr bool kRayLds = FLAGS || MODE == kModePath || MODE == kModeFused || kTrain;
-    extern __shared__ uint2 lds_stack[];
-    __shared__ Words4 task_words[4][32];
-    // the table in LDS: a byte read instead of 16 vector instructions per node step (path tracing 2% faster)
-    __shared__ OctTable oct_lds;
-    for (uint32_t i = threadIdx.x; i < sizeof(OctTable) / 8u; i += blockDim.x)
-        ((uint64_t*)&oct_lds)[i] = ((const uint64_t*)&kOctTable)[i];
-    __syncthreads();
+    // the triangle tasks of the block's waves (32 of 16 B each), the stack, the rays
+    extern __shared__ __attribute__((aligned(16))) uint2 lds_words[];
+    uint2* const lds_stack = lds_words + (LEAN ? 0u : blockDim.x);
     __attribute__((address_space(3))) Words4* const tasks =
-        (__attribute__((address_space(3))) Words4*)task_words[threadIdx.x >> 6];
+        (__attribute__((address_space(3))) Words4*)lds_words + 32u * (threadIdx.x >> 6);
+    __shared__ OctTable oct_lds;
+    if (!LEAN) {
+        for (uint32_t i = threadIdx.x; i < sizeof(OctTable) / 8u; i += blockDim.x)
+            ((uint64_t*)&oct_lds)[i] = ((const uint64_t*)&kOctTable)[i];
+        __syncthreads();
+    }
     float* const lds_ray = (float*)(lds_stack + args.lds_depth * blockDim.x) + threadIdx.x;
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
@@ -672,24 +673,24 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
         tc = r.tmax;
     };
 
-    // Wave-uniform pool of ray ids [pool_next, pool_end).  Chunk w of the launch is wave w's first pool (not where
-    // the grid's later blocks start only as another launch's blocks retire: first_chunks = 0); the chunks after those
-    // come from kRayQueues counters, each shared by the blocks of one residue: queue q's c-th chunk is one
-    // of the c-th group of nq chunks, at a place rotated by a hash of c (with a fixed place, a film whose rows hold a
-    // multiple of nq / 2 chunks gives every queue its own columns: 20% slower).  An atomic on one word shared by all waves costs 10-20 ns in turn, so one counter
-    // bounded short launches by its 4,096 waves' fetches alone: 777 rays 96 us, the 1200x800 reference film 224 us.
+    // Wave-uniform pool of ray ids [pool_next, pool_end).  Chunk w of the launch is wave w's first pool, for the first
+    // first_waves waves; the chunks after those come from kRayQueues counters, each shared by the blocks of one residue:
+    // queue q's c-th chunk is one of the c-th group of nq chunks, at a place rotated by a hash of c (with a fixed place,
+    // a film whose rows hold a multiple of nq / 2 chunks gives every queue its own columns: 20% slower).  An atomic on
+    // one word shared by all waves costs 10-20 ns in turn, so one counter bounded short launches by its 4,096 waves'
+    // fetches alone: 777 rays 96 us, the 1200x800 reference film 224 us.
     const uint32_t waves_block = blockDim.x >> 6;
     const uint32_t waves_total = gridDim.x * waves_block;
     const uint32_t wave =
         (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * waves_block + (threadIdx.x >> 6)));
-    const uint32_t chunk = rays_per_chunk(args.ray_chunk, nrays, waves_total, args.first_chunks, kTrain);
+    const uint32_t chunk = rays_per_chunk(args.ray_chunk, nrays, waves_total, args.first_waves, kTrain);
     const uint32_t nqueues = gridDim.x < kRayQueues ? gridDim.x : kRayQueues;
     uint32_t queue = blockIdx.x % nqueues;
     uint32_t hops = 0;  // queues this wave has found empty
-    const uint32_t own_chunks = args.first_chunks ? waves_total : 0u;
+    const uint32_t own_chunks = args.first_waves;
     bool more = (uint64_t)chunk * own_chunks < nrays;
     uint32_t pool_next = 0, pool_end = 0;
-    if (own_chunks) {
+    if (wave < own_chunks) {
         const uint64_t first = (uint64_t)wave * chunk;
         if (first < nrays) {
             pool_next = (uint32_t)first;
@@ -1050,15 +1051,30 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
                         fault = kErrBadAs;
                         slot0 = slot1 = kNoSlot;
                     }
-                    tasks[rank] = Words4{slot0, slot1, lane, 0u};
                 }
                 const uint32_t ntri = 2u * (uint32_t)__popcll(tri_lanes);
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 uint32_t from = lane, slot = kNoSlot;
-                if (lane < ntri) {
-                    const Words4 w = tasks[lane >> 1];
-                    slot = (lane & 1u) ? w.y : w.x;
-                    from = w.z;
+                if (LEAN) {
+                    // Owner number k sends its triangles and its place to lane 2 k, from where lane 2 k + 1 takes them
+                    // too (quad_perm [0, 0, 2, 2]); lanes that own nothing send to lane 1, whose word nobody reads.
+                    const int to = owner ? (int)(rank << 3) : 4;
+                    const auto pair = [&](uint32_t v) {
+                        return (uint32_t)__builtin_amdgcn_mov_dpp(__builtin_amdgcn_ds_permute(to, (int)v), 0xA0, 0xF,
+                                                                  0xF, true);
+                    };
+                    const uint32_t whose = pair(lane), task0 = pair(slot0), task1 = pair(slot1);
+                    if (lane < ntri) {
+                        slot = (lane & 1u) ? task1 : task0;
+                        from = whose;
+                    }
+                } else {
+                    if (owner) tasks[rank] = Words4{slot0, slot1, lane, 0u};
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    if (lane < ntri) {
+                        const Words4 w = tasks[lane >> 1];
+                        slot = (lane & 1u) ? w.y : w.x;
+                        from = w.z;
+                    }
                 }
                 // the owner's ray
                 const auto pull = [&](float v) {
@@ -1120,22 +1136,32 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
                 }
                 const uint64_t hits = __builtin_amdgcn_ballot_w64(cand);
                 if (hits) {
-                    if (cand) ((__attribute__((address_space(3))) float*)(tasks + (lane >> 1)))[lane & 1u] = th;
-                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    uint32_t t0 = 0, t1 = 0;  // the owner's two distances
+                    if (LEAN) {
+                        t0 = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(rank << 3), (int)__float_as_uint(th));
+                        t1 = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(rank << 3) + 4, (int)__float_as_uint(th));
+                    } else {
+                        if (cand) ((__attribute__((address_space(3))) float*)(tasks + (lane >> 1)))[lane & 1u] = th;
+                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    }
                     const uint32_t own = owner ? (uint32_t)(hits >> (2u * rank)) & 3u : 0u;
                     if (own) {
                         if (MODE == kModeAny || ((MODE == kModeFused || kTrain) && shadow_ray)) {
                             occl = true;
                             done = true;
                         } else {
-                            const Words2 w = *(__attribute__((address_space(3))) Words2*)(tasks + rank);
+                            if (!LEAN) {
+                                const Words2 w = *(__attribute__((address_space(3))) Words2*)(tasks + rank);
+                                t0 = w.x;
+                                t1 = w.y;
+                            }
                             // Exact ties in t go to the smaller (instance, slot), so the closest hit does not
                             // depend on the order in which a lane meets its candidates (which the wave's leaf
                             // scheduling can change).  A ray's first hit may round past its tmax.
                             const uint32_t ci = cur_inst & kInstIdMask;
 #pragma unroll
                             for (int k = 0; k < 2; ++k) {
-                                const float tn = s.toff + __uint_as_float(k ? w.y : w.x);
+                                const float tn = s.toff + __uint_as_float(k ? t1 : t0);
                                 const uint32_t sl = k ? slot1 : slot0;
                                 const bool closer = !(tn >= tc) || hit_inst == kNoHit ||
                                                     (tn == tc && (ci < hit_inst || (ci == hit_inst && sl < hit_slot)));
@@ -1295,7 +1321,7 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
                     const uint32_t imask = (w0.z >> 8) & 255u;
                     const uint32_t vmask = (w0.z >> 16) & 255u;
                     ng_base = w0.w;
-                    ng_bits = oct_lds.row[s.oct][hm & imask] | (vmask << 8);
+                    ng_bits = (LEAN ? oct_permute(hm & imask, s.oct) : oct_lds.row[s.oct][hm & imask]) | (vmask << 8);
                     const uint32_t lg_new = (hm & ~imask) | (vmask << 8);
                     if (!(lg_bits & 255u)) {
                         lg_base = w0.w;
@@ -1344,20 +1370,20 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
     }
 }
 
-// Three occupancy variants of the same traversal: unconstrained registers, at most 128 VGPRs (four waves per
-// SIMD) and at most 96 VGPRs (five waves per SIMD), chosen by the waves per SIMD that the launch shape asks for.
+// Occupancy variants of the same traversal: unconstrained registers (three waves per SIMD at least), at most 128 VGPRs
+// (four waves) and at most 96 VGPRs (five waves, LEAN), chosen by the waves per SIMD that the launch shape asks for.
 template <int MODE, bool STATS, bool FLAGS>
 __global__ __launch_bounds__(256) void trace_kernel(TraceArgs args) {
-    trace_body<MODE, STATS, FLAGS>(args);
+    trace_body<MODE, STATS, FLAGS, false>(args);
 }
-template <int MODE, bool STATS, bool FLAGS>
+template <int MODE, bool STATS, bool FLAGS, bool LEAN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void trace_kernel_w4(TraceArgs args) {
-    trace_body<MODE, STATS, FLAGS>(args);
+    trace_body<MODE, STATS, FLAGS, LEAN>(args);
 }
 
 template <int MODE, bool STATS, bool FLAGS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void trace_kernel_w5(TraceArgs args) {
-    trace_body<MODE, STATS, FLAGS>(args);
+    trace_body<MODE, STATS, FLAGS, true>(args);
 }
 
 __global__ void reset_counter_kernel(DeviceState* st, int clear_stats) {
@@ -1373,18 +1399,15 @@ __global__ void reset_counter_kernel(DeviceState* st, int clear_stats) {
 }
 
 template <int MODE, bool STATS, bool FLAGS>
-hipError_t launch_variant(const TraceArgs& a, const TraceLaunch& L, hipStream_t s) {
-    // the stack, and the lanes' world rays where the kernel keeps them in LDS
-    constexpr bool kRayLds = FLAGS || MODE == kModePath || MODE == kModeFused || MODE == kModeTrain ||
-                             MODE == kModePixelPaths || MODE == kModePixelCache;
-    const size_t lds =
-        (size_t)L.lds_depth * L.block_size * sizeof(uint2) + (kRayLds ? (size_t)L.block_size * 6 * sizeof(float) : 0);
+hipError_t launch_variant(const TraceArgs& a, const TraceLaunch& L, const TracePlan& p, hipStream_t s) {
     if (L.waves >= 5)
-        trace_kernel_w5<MODE, STATS, FLAGS><<<L.grid, L.block_size, lds, s>>>(a);
+        trace_kernel_w5<MODE, STATS, FLAGS><<<p.grid, L.block_size, p.lds, s>>>(a);
+    else if (p.lean)
+        trace_kernel_w4<MODE, STATS, FLAGS, true><<<p.grid, L.block_size, p.lds, s>>>(a);
     else if (L.waves == 4)
-        trace_kernel_w4<MODE, STATS, FLAGS><<<L.grid, L.block_size, lds, s>>>(a);
+        trace_kernel_w4<MODE, STATS, FLAGS, false><<<p.grid, L.block_size, p.lds, s>>>(a);
     else
-        trace_kernel<MODE, STATS, FLAGS><<<L.grid, L.block_size, lds, s>>>(a);
+        trace_kernel<MODE, STATS, FLAGS><<<p.grid, L.block_size, p.lds, s>>>(a);
     return hipGetLastError();
 }
 
@@ -1393,11 +1416,8 @@ constexpr uint32_t kActiveRayFlags = kRayTerminateOnFirstHit | kRaySkipClosestHi
                                      kRayCullOpaque | kRayCullNoOpaque | kRayNoOpaque | kRaySkipTriangles |
                                      kRaySkipAabbs;
 
-template <int MODE, bool STATS>
-hipError_t launch(const TraceArgs& a, const TraceLaunch& L, uint32_t content, hipStream_t s) {
-    if (trace_needs_flags(a.ray_flags, content)) return launch_variant<MODE, STATS, true>(a, L, s);
-    return launch_variant<MODE, STATS, false>(a, L, s);
-}
+template <int M>
+using ModeC = std::integral_constant<int, M>;
 
 }  // namespace
 
@@ -1454,33 +1474,42 @@ hipError_t trace_rays_launch(const TraceRequest& r, const TraceLaunch& L, hipStr
         reset_counter_kernel<<<1, 64, 0, s>>>(r.state, r.stats ? 1 : 0);
         return hipGetLastError();
     }
-    // A host-known ray count: no more waves than rays, and no queue to clear where the first chunks cover the rays.
-    TraceLaunch G = L;
-    bool queues = true;
-    a.first_chunks = r.mode != 5;  // training paths run beside the pixel paths, on blocks that start one by one
-    if (!r.n_ptr && a.first_chunks) {
-        const uint32_t waves_block = L.block_size / 64u;
-        if (L.ray_chunk < 64u) G.grid = std::min(L.grid, (r.n - 1u) / waves_block + 1u);
-        const uint32_t waves = G.grid * waves_block;
-        queues = (uint64_t)rays_per_chunk(L.ray_chunk, r.n, waves, 1u, r.mode >= 5) * waves < r.n;
-    }
     // guard 3: both variants, each guarded by the TLAS content the device reads, so that one of them takes the rays
     const bool both = r.guard == 3u && r.mode <= 2 && !(r.ray_flags & kActiveRayFlags);
     for (uint32_t g = 1; g <= (both ? 2u : 1u); ++g) {
-        const bool clear = r.stats && g == 1;
-        if (queues || clear) reset_counter_kernel<<<1, 64, 0, s>>>(r.state, clear ? 1 : 0);
-        a.guard = both ? g : (r.guard == 1u || r.guard == 2u ? r.guard : 0u);
         const uint32_t c = !both ? r.content : (g == 1 ? 0u : (kContentAabb | kContentNonOpaque));
+        const bool flags = r.mode < 5 && trace_needs_flags(a.ray_flags, c);
+        TraceShape sh;
+        sh.block_size = L.block_size;
+        sh.blocks_per_cu = L.blocks_per_cu;
+        sh.grid = L.grid;
+        sh.waves_per_simd = L.waves >= 5u ? 5u : (L.waves == 4u ? 4u : 3u);
+        sh.lane_bytes = L.lds_depth * (uint32_t)sizeof(uint2) + (flags || r.mode >= 3 ? 6u * (uint32_t)sizeof(float) : 0u);
+        sh.beside = r.mode == 5;  // training paths run beside the pixel paths, on blocks that start one by one
+        const TracePlan p = plan_trace(sh, L.ray_chunk, r.n_ptr ? 0u : r.n, r.mode >= 5);
+        a.first_waves = p.first_waves;
+        a.guard = both ? g : (r.guard == 1u || r.guard == 2u ? r.guard : 0u);
+        const bool clear = r.stats && g == 1;
+        if (p.queues || clear) reset_counter_kernel<<<1, 64, 0, s>>>(r.state, clear ? 1 : 0);
+        const auto launch = [&](auto mode, auto stats) {
+            constexpr int M = decltype(mode)::value;
+            constexpr bool S = decltype(stats)::value;
+            if constexpr (M < kModeTrain)
+                if (flags) return launch_variant<M, S, true>(a, L, p, s);
+            return launch_variant<M, S, false>(a, L, p, s);
+        };
+        const std::true_type on;
+        const std::false_type off;
         hipError_t e;
         switch (r.mode) {
-            case 0: e = r.stats ? launch<kModeClosest, true>(a, G, c, s) : launch<kModeClosest, false>(a, G, c, s); break;
-            case 1: e = r.stats ? launch<kModeAny, true>(a, G, c, s) : launch<kModeAny, false>(a, G, c, s); break;
-            case 3: e = launch<kModePath, false>(a, G, c, s); break;
-            case 4: e = launch<kModeFused, false>(a, G, c, s); break;
-            case 5: e = launch_variant<kModeTrain, false, false>(a, G, s); break;
-            case 6: e = launch_variant<kModePixelPaths, false, false>(a, G, s); break;
-            case 7: e = launch_variant<kModePixelCache, false, false>(a, G, s); break;
-            default: e = r.stats ? launch<kModeRaygen, true>(a, G, c, s) : launch<kModeRaygen, false>(a, G, c, s);
+            case 0: e = r.stats ? launch(ModeC<kModeClosest>(), on) : launch(ModeC<kModeClosest>(), off); break;
+            case 1: e = r.stats ? launch(ModeC<kModeAny>(), on) : launch(ModeC<kModeAny>(), off); break;
+            case 3: e = launch(ModeC<kModePath>(), off); break;
+            case 4: e = launch(ModeC<kModeFused>(), off); break;
+            case 5: e = launch(ModeC<kModeTrain>(), off); break;
+            case 6: e = launch(ModeC<kModePixelPaths>(), off); break;
+            case 7: e = launch(ModeC<kModePixelCache>(), off); break;
+            default: e = r.stats ? launch(ModeC<kModeRaygen>(), on) : launch(ModeC<kModeRaygen>(), off);
         }
         if (e) return e;
     }

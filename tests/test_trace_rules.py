@@ -1,6 +1,9 @@
-"""The traversal's rules that are plain functions of sizes (csrc/trace_rules.h), compiled for the CPU."""
+"""The traversal's rules that are plain functions of sizes (csrc/trace_rules.h), compiled for the CPU, and the LDS that
+the built kernels take by themselves."""
 import ctypes
 import os
+import re
+import shutil
 import subprocess
 
 import pytest
@@ -11,6 +14,16 @@ SOURCE = r"""
 #include "trace_rules.h"
 extern "C" {
 int pops_entry(uint32_t sp, uint32_t entries) { return rtx::pops_entry(sp, entries); }
+// out: grid, lds, first_waves, lean, queues, resident blocks per CU, rays per chunk
+void plan(uint32_t block, uint32_t per_cu, uint32_t cus, uint32_t simd, uint32_t lane_bytes, uint32_t beside,
+          uint32_t chunk, uint32_t n, uint32_t paths, uint32_t* out) {
+    const rtx::TraceShape s = {block, per_cu, cus * per_cu, simd, lane_bytes, beside != 0};
+    const rtx::TracePlan p = rtx::plan_trace(s, chunk, n, paths != 0);
+    const uint32_t fixed = p.lean ? 0u : rtx::kOctTableBytes;
+    const uint32_t v[] = {p.grid, p.lds, p.first_waves, p.lean, p.queues, rtx::resident_blocks(s, p.lds + fixed),
+                          rtx::rays_per_chunk(chunk, n, p.grid * (block / 64), p.first_waves, paths != 0)};
+    for (int i = 0; i < 7; ++i) out[i] = v[i];
+}
 }
 """
 
@@ -23,6 +36,65 @@ def rules(tmp_path_factory):
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-Wall", "-I", os.path.join(PKG, "csrc"), str(src),
                     "-o", str(lib)], check=True)
     return ctypes.CDLL(str(lib))
+
+
+def _plan(rules, block, per_cu, cus=256, depth=12, ray=True, beside=False, chunk=1, n=0, paths=False):
+    waves = block // 64 * per_cu // 4
+    out = (ctypes.c_uint32 * 7)()
+    rules.plan(block, per_cu, cus, 5 if waves >= 5 else 4 if waves == 4 else 3, 8 * depth + (24 if ray else 0),
+               int(beside), chunk, n, int(paths), out)
+    return dict(zip(("grid", "lds", "first_waves", "lean", "queues", "resident", "chunk"), out))
+
+
+def _units(b):  # LDS of a CU is given out in 128 units of 1,280 B
+    return -(-b // 1280)
+
+
+def test_the_tables_and_tasks_take_no_block_from_a_cu(rules):
+    """Over every configuration that the library accepts: as many blocks of a launch fit a CU's LDS as would with the
+    stack and the world rays alone, and the default launch keeps its table and tasks."""
+    for block in (64, 128, 192, 256):
+        for per_cu in range(1, 33):
+            for depth in range(1, 4097):
+                if (8 * depth + 24) * block > 64 * 1024:
+                    break
+                for ray in (False, True):
+                    p = _plan(rules, block, per_cu, depth=depth, ray=ray)
+                    waves = block // 64 * per_cu // 4
+                    alone = 128 // _units((8 * depth + 24 * ray) * block)
+                    want = min(per_cu, 4 * (5 if waves >= 5 else 4 if waves == 4 else 3) // (block // 64), alone)
+                    assert p["resident"] == want, (block, per_cu, depth, ray, p)
+                    extra = 0 if p["lean"] else 8 * block
+                    assert p["lds"] == (8 * depth + 24 * ray) * block + extra
+    assert not _plan(rules, 256, 4)["lean"] and not _plan(rules, 64, 16)["lean"]
+    assert _plan(rules, 64, 20)["lean"] and _plan(rules, 64, 16, depth=16)["lean"]
+
+
+READELF = "/opt/rocm/llvm/bin/llvm-readelf"
+BUNDLER = "/opt/rocm/llvm/bin/clang-offload-bundler"
+OBJECT = os.path.join(PKG, "_build", "trace.o")
+
+
+@pytest.mark.skipif(not (os.path.exists(OBJECT) and os.path.exists(READELF) and shutil.which("objcopy")),
+                    reason="needs the object file of the build and the ROCm binary tools")
+def test_static_lds_of_the_traversal_kernels(tmp_path):
+    """What the launch rules count is what the kernels take: the octant table, and nothing in the lean form (five waves
+    per SIMD, and the LEAN = true instances of four)."""
+    fat, code = str(tmp_path / "fat"), str(tmp_path / "code")
+    subprocess.run(["objcopy", "-O", "binary", "--only-section=.hip_fatbin", OBJECT, fat], check=True)
+    subprocess.run([BUNDLER, "--unbundle", "--type=o", f"--input={fat}", f"--output={code}",
+                    "--targets=hipv4-amdgcn-amd-amdhsa--gfx950"], check=True)
+    notes = subprocess.run([READELF, "--notes", code], check=True, capture_output=True, text=True).stdout
+    seen = {"lean": 0, "full": 0}
+    for part in notes.split(".group_segment_fixed_size:")[1:]:
+        lds, name = int(part.split()[0]), re.search(r"\.name:\s+(\S+)", part).group(1)
+        m = re.search(r"trace_kernel(_w[45])?ILi\dE((?:Lb[01]E)+)", name)
+        if not m:
+            continue
+        lean = m.group(1) == "_w5" or (m.group(1) == "_w4" and m.group(2).endswith("Lb1E"))
+        assert lds == (0 if lean else 2048), name
+        seen["lean" if lean else "full"] += 1
+    assert seen["lean"] > 10 and seen["full"] > 10, seen
 
 
 @pytest.mark.parametrize("entries", [1, 2, 12, 76, 4096])

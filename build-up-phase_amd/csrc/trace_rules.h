@@ -71,18 +71,23 @@ struct TracePlan {
 //                wave per CU (12 or 13 of them fitted) and 7.9 ms on 16 with 16 stack entries each; lean 7.2 and
 //                6.3 ms.  Where they fit (256 x 4), the table's byte read instead of 16 vector instructions per node
 //                step and the tasks through LDS instead of five permutes are 2% and 1% faster
-//   first_waves  all, but none where the chip is shared: blocks that start as the other launch's retire come too late
+//   first_waves  only waves that start at once own rays.  The blocks beyond start as others retire, when the queues have
+//                run dry, and would only then begin with theirs: on 32 blocks of 256 per CU, of which 4 or 5 start, 4M
+//                incoherent rays took 1.83 ms and 720p path tracing 9.3 ms, now 1.22 and 7.2 ms.  None where the chip is
+//                shared: which blocks start at once is not known then
 //   grid         no more waves than rays
 RTX_RULE TracePlan plan_trace(const TraceShape& s, uint32_t ray_chunk, uint32_t n, bool paths) {
     TracePlan p;
     const uint32_t waves_block = s.block_size / 64u;
     p.lds = s.lane_bytes * s.block_size;
     const uint32_t tasks = kTaskLaneBytes * s.block_size;
-    p.lean = s.waves_per_simd >= 5u || resident_blocks(s, p.lds + tasks + kOctTableBytes) < resident_blocks(s, p.lds);
+    uint32_t resident = resident_blocks(s, p.lds);
+    p.lean = s.waves_per_simd >= 5u || resident_blocks(s, p.lds + tasks + kOctTableBytes) < resident;
     if (!p.lean) p.lds += tasks;
     p.grid = s.grid;
     if (n && !s.beside && ray_chunk < 64u && (n - 1u) / waves_block < p.grid) p.grid = (n - 1u) / waves_block + 1u;
-    p.first_waves = s.beside ? 0u : p.grid * waves_block;
+    const uint32_t at_once = s.grid / s.blocks_per_cu * resident;
+    p.first_waves = s.beside ? 0u : (at_once < p.grid ? at_once : p.grid) * waves_block;
     p.queues = !n || (uint64_t)rays_per_chunk(ray_chunk, n, p.grid * waves_block, p.first_waves, paths) * p.first_waves < n;
     return p;
 }

@@ -70,6 +70,28 @@ def test_the_tables_and_tasks_take_no_block_from_a_cu(rules):
     assert _plan(rules, 64, 20)["lean"] and _plan(rules, 64, 16, depth=16)["lean"]
 
 
+@pytest.mark.parametrize("chunk", [1, 64, 128, 4096])
+@pytest.mark.parametrize("shape", [(64, 1), (64, 13), (64, 20), (64, 32), (128, 10), (192, 3), (256, 4), (256, 5), (256, 32)])
+def test_first_chunks_belong_to_waves_that_start_at_once(rules, shape, chunk):
+    """Waves own a first chunk only among the blocks that the chip holds at once, and not beside another launch; the
+    first chunks and the queues' chunks cover the rays, and the queues are used exactly where rays are left for them."""
+    block, per_cu = shape
+    cus, wb = 4, block // 64
+    for ray in (False, True):
+        full = _plan(rules, block, per_cu, cus, ray=ray)
+        for n in [1, 2, 63, 64, 65, 777, 64 * cus * per_cu * wb - 1, 64 * cus * per_cu * wb, 64 * cus * per_cu * wb + 1,
+                  512 * cus * per_cu * wb, 2 ** 28, 2 ** 32 - 1]:
+            for paths in (False, True):
+                p = _plan(rules, block, per_cu, cus, ray=ray, chunk=chunk, n=n, paths=paths)
+                assert p["first_waves"] <= full["resident"] * cus * wb, (n, p)
+                assert 1 <= p["grid"] <= cus * per_cu and p["first_waves"] <= p["grid"] * wb
+                assert p["chunk"] >= 1 and bool(p["queues"]) == (p["chunk"] * p["first_waves"] < n)
+                b = _plan(rules, block, per_cu, cus, ray=ray, chunk=chunk, n=n, paths=paths, beside=True)
+                assert b["first_waves"] == 0 and b["queues"] and b["grid"] == cus * per_cu
+        d = _plan(rules, block, per_cu, cus, ray=ray, chunk=chunk, n=0)  # a count that only the device knows
+        assert d["queues"] and d["grid"] == cus * per_cu
+
+
 READELF = "/opt/rocm/llvm/bin/llvm-readelf"
 BUNDLER = "/opt/rocm/llvm/bin/clang-offload-bundler"
 OBJECT = os.path.join(PKG, "_build", "trace.o")

@@ -642,6 +642,8 @@ hipError_t pt_render_nrc(PtArgs a, const TraceLaunch& L, const SideChain& side, 
         // while the host enqueues the training wavefront's many short ones)
         if (!train_only && (e = render_cache_sample(a, L, sample_offset + si, s))) return e;
         fill_words_kernel<<<1024, 256, 0, side.stream>>>((uint32_t*)a.rec, nrec * 20, 0u);
+        TraceLaunch tl = side.launch;
+        if (train_only) tl.beside = 0u;  // no pixel paths: the training paths have the chip to themselves
         if (!t.tail && pt_whole_paths(t)) {
             // the whole training wavefront in one traversal launch (each lane shades and continues its own path)
             TraceRequest tr{};
@@ -658,8 +660,8 @@ hipError_t pt_render_nrc(PtArgs a, const TraceLaunch& L, const SideChain& side, 
             tr.pt = &t;
             tr.pt_sample = sample_offset + si;
             tr.content = t.content;
-            if ((e = trace_rays_launch(tr, side.launch, side.stream))) return e;
-        } else if ((e = run_pass(t, side.launch, sample_offset + si, t.train_end, side.stream))) {
+            if ((e = trace_rays_launch(tr, tl, side.stream))) return e;
+        } else if ((e = run_pass(t, tl, sample_offset + si, t.train_end, side.stream))) {
             return e;
         }
         // training tails (self-training) are predicted with the cache before this frame's Adam steps

@@ -1485,7 +1485,7 @@ hipError_t trace_rays_launch(const TraceRequest& r, const TraceLaunch& L, hipStr
         sh.grid = L.grid;
         sh.waves_per_simd = L.waves >= 5u ? 5u : (L.waves == 4u ? 4u : 3u);
         sh.lane_bytes = L.lds_depth * (uint32_t)sizeof(uint2) + (flags || r.mode >= 3 ? 6u * (uint32_t)sizeof(float) : 0u);
-        sh.beside = r.mode == 5;  // training paths run beside the pixel paths, on blocks that start one by one
+        sh.beside = L.beside != 0;
         const TracePlan p = plan_trace(sh, L.ray_chunk, r.n_ptr ? 0u : r.n, r.mode >= 5);
         a.first_waves = p.first_waves;
         a.guard = both ? g : (r.guard == 1u || r.guard == 2u ? r.guard : 0u);

@@ -1485,7 +1485,8 @@ int rtx_set_trace_config(rtx_context ctx, const rtx_trace_config* cfg) {
         return fail(ctx, RTX_ERROR_INVALID_ARGUMENT, "block_size must be 64, 128, 192 or 256");
     if (c.blocks_per_cu < 1 || c.blocks_per_cu > 32)
         return fail(ctx, RTX_ERROR_INVALID_ARGUMENT, "blocks_per_cu must be in [1, 32]");
-    // per lane: the stack entries (8 B each) and the world ray (24 B)
+    // per lane: the stack entries (8 B each) and the world ray (24 B); the kernels' own LDS comes on top where it costs no
+    // block (plan_trace)
     if (c.lds_stack_depth < 1 || ((uint64_t)c.lds_stack_depth * 8 + 24) * c.block_size > 64 * 1024)
         return fail(ctx, RTX_ERROR_INVALID_ARGUMENT, "LDS stack above 64 KiB per block");
     ctx->cfg = c;

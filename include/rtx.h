@@ -408,7 +408,9 @@ typedef struct rtx_trace_config {
     uint32_t block_size;      /* threads per block: 64, 128, 192 or 256 */
     uint32_t blocks_per_cu;   /* persistent blocks per compute unit (1..32) */
     uint32_t lds_stack_depth; /* stack entries held in LDS per lane before spilling to global memory; with the
-                                 lane's world ray (24 B) at most 64 KiB of LDS per block: (8 depth + 24) block */
+                                 lane's world ray (24 B) at most 64 KiB of LDS per block: (8 depth + 24) block.
+                                 Launches take 8 B per lane and 2 KiB per block more where that costs no block of
+                                 a compute unit's 160 KiB (not with five or more waves per SIMD) */
     uint32_t ray_chunk;       /* ray ids a wave takes from a queue per fetch: a multiple of 64 up to
                                  4096, or RTX_TRACE_RAY_CHUNK_AUTO (up to 64, or 256 for single
                                  rays when every wave gets >= 8 chunks) */
@@ -420,8 +422,9 @@ typedef struct rtx_trace_config {
     uint32_t stack_limit;     /* traversal stack entries per lane, LDS and global spill together: 0 (default) sizes the
                                  stack from the traced TLAS's depth (2 entries per BVH level + 4, enough for every
                                  ray); with a smaller value a ray that needs more ends there (reporting the closest
-                                 hit found so far, or a miss) and rtx_sync reports RTX_ERROR_STACK_OVERFLOW.  Not an autotuner knob; rtx_set_trace_config keeps it
-                                 when the field is 0, so RTX_TRACE_STACK_LIMIT_DERIVED restores the default. */
+                                 hit found so far, or a miss) and rtx_sync reports RTX_ERROR_STACK_OVERFLOW.  Not an
+                                 autotuner knob; rtx_set_trace_config keeps it when the field is 0, so
+                                 RTX_TRACE_STACK_LIMIT_DERIVED restores the default. */
 } rtx_trace_config;
 #define RTX_TRACE_STACK_LIMIT_DERIVED 0xFFFFFFFFu
 #define RTX_TRACE_RAY_CHUNK_AUTO 1u

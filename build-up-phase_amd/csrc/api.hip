@@ -493,15 +493,10 @@ int rtx_sync(rtx_context ctx) {
             flags |= nf;
         }
     }
-    if (flags) {
-        if (flags & rtx::kErrStackOverflow)
-            return fail(ctx, RTX_ERROR_STACK_OVERFLOW, "traversal stack overflow (more than %u entries per lane)",
-                        ctx->last_stack);
-        if (flags & rtx::kErrSortTimeout) return fail(ctx, RTX_ERROR_DEVICE_LOST, "radix sort look-back timed out");
-        if (flags & rtx::kErrBuildDepth)
-            return fail(ctx, RTX_ERROR_INVALID_AS, "BVH deeper than the builder's collapse level bound");
-        return fail(ctx, RTX_ERROR_INVALID_AS, "device reported an invalid acceleration structure");
-    }
+    const rtx::DeviceError err = rtx::device_error(flags);
+    if (err.code == RTX_ERROR_STACK_OVERFLOW)
+        return fail(ctx, err.code, "%s (more than %u entries per lane)", err.text, ctx->last_stack);
+    if (err.code) return fail(ctx, err.code, "%s", err.text);
     return RTX_SUCCESS;
 }
 

@@ -1925,7 +1925,10 @@ __global__ __launch_bounds__(64) void collapse_top_kernel(CollapseArgs a) {
         if (!onm) {
             if (__shfl(open, 0) == 0u) break;
             if (++spins > kQueueSpins) {
-                if (lane == 0) atomicOr(a.err, kErrBuildDepth);
+                if (lane == 0) {
+                    atomicOr(a.err, kErrCollapseTimeout);
+                    if (!BATCHED) a.h->build_error = 1u;
+                }
                 break;
             }
             __builtin_amdgcn_s_sleep(4);

@@ -22,6 +22,7 @@
 #include <stdint.h>
 
 #include "../../include/rtx.h"
+#include "device_errors.h"
 
 namespace rtx {
 
@@ -150,7 +151,7 @@ constexpr uint32_t kRayQueues = 32;
 // Context-owned device state.
 struct DeviceState {
     RayQueue queue[kRayQueues];
-    uint32_t error_flags;  // bit 0: stack overflow, bit 1: sort look-back timeout, bit 2: bad AS
+    uint32_t error_flags;  // kErr* bits (device_errors.h)
     uint32_t pad[3];
     unsigned long long stat_nodes;
     unsigned long long stat_tris;
@@ -158,11 +159,6 @@ struct DeviceState {
     unsigned long long stat_rays;
     unsigned long long pt_rays;  // rays traced by the path tracer (extension + shadow)
 };
-
-constexpr uint32_t kErrStackOverflow = 1u;
-constexpr uint32_t kErrSortTimeout = 2u;
-constexpr uint32_t kErrBadAs = 4u;
-constexpr uint32_t kErrBuildDepth = 8u;
 
 // ---- small device helpers ---------------------------------------------------------------------------------
 __device__ __forceinline__ uint32_t float_to_ordered(float f) {

@@ -128,7 +128,8 @@ __device__ void load_bounds(const uint32_t* __restrict__ cb, uint32_t* s) {
 
 // Words that a build starts from: the bounds' slots, and the 16 words of counters (zero).
 __global__ __launch_bounds__(256) void init_build_kernel(uint32_t* __restrict__ cb, uint32_t* __restrict__ misc) {
-    for (uint32_t i = threadIdx.x; i < kBoundSlots * kBoundStride; i += 256u) cb[i] = i % kBoundStride < 3u ? 0xFFFFFFFFu : 0u;
+    for (uint32_t i = threadIdx.x; i < kBoundSlots * kBoundStride; i += 256u)
+        cb[i] = i % kBoundStride < 3u ? 0xFFFFFFFFu : 0u;
     if (threadIdx.x < 16u) misc[threadIdx.x] = 0u;
 }
 
@@ -168,35 +169,36 @@ __global__ __launch_bounds__(256) void prep_tris_kernel(const GeomDesc* __restri
                 for (int k = 0; k < 6; ++k) t.v[k] = src[k];
                 t.v[6] = t.v[7] = t.v[8] = 0.0f;
 #pragma unroll
-                for (int a = 0; a < 3; ++a) valid = valid && isfinite(t.v[a]) && isfinite(t.v[3 + a]) && t.v[a] <= t.v[3 + a];
+                for (int a = 0; a < 3; ++a)
+                    valid = valid && isfinite(t.v[a]) && isfinite(t.v[3 + a]) && t.v[a] <= t.v[3 + a];
             } else {
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                uint32_t vi = g.idx[3 * (uint64_t)p + k];
-                float v[3];
-                if (vi > g.max_vertex) {
-                    valid = false;
-                    v[0] = v[1] = v[2] = 0.0f;
-                } else {
-                    const float* src = (const float*)(g.vtx + (uint64_t)(vi + g.first_vertex) * g.stride);
-                    v[0] = src[0];
-                    v[1] = src[1];
-                    v[2] = src[2];
+                for (int k = 0; k < 3; ++k) {
+                    uint32_t vi = g.idx[3 * (uint64_t)p + k];
+                    float v[3];
+                    if (vi > g.max_vertex) {
+                        valid = false;
+                        v[0] = v[1] = v[2] = 0.0f;
+                    } else {
+                        const float* src = (const float*)(g.vtx + (uint64_t)(vi + g.first_vertex) * g.stride);
+                        v[0] = src[0];
+                        v[1] = src[1];
+                        v[2] = src[2];
+                    }
+                    if (g.xform) {
+                        float o[3];
+                        xform_vertex(g.xform, v, o);
+                        t.v[3 * k] = o[0];
+                        t.v[3 * k + 1] = o[1];
+                        t.v[3 * k + 2] = o[2];
+                    } else {
+                        t.v[3 * k] = v[0];
+                        t.v[3 * k + 1] = v[1];
+                        t.v[3 * k + 2] = v[2];
+                    }
                 }
-                if (g.xform) {
-                    float o[3];
-                    xform_vertex(g.xform, v, o);
-                    t.v[3 * k] = o[0];
-                    t.v[3 * k + 1] = o[1];
-                    t.v[3 * k + 2] = o[2];
-                } else {
-                    t.v[3 * k] = v[0];
-                    t.v[3 * k + 1] = v[1];
-                    t.v[3 * k + 2] = v[2];
-                }
-            }
 #pragma unroll
-            for (int k = 0; k < 9; ++k) valid = valid && isfinite(t.v[k]);
+                for (int k = 0; k < 9; ++k) valid = valid && isfinite(t.v[k]);
             }
             t.prim = p;
             t.geom = g.geom_local;
@@ -594,7 +596,9 @@ __device__ __forceinline__ void store_coherent_u32(uint32_t* p, uint32_t v) {
 __device__ __forceinline__ int32_t load_coherent_i32(const int32_t* p) {
     return (int32_t)load_coherent_u32((const uint32_t*)p);
 }
-__device__ __forceinline__ void store_coherent_i32(int32_t* p, int32_t v) { store_coherent_u32((uint32_t*)p, (uint32_t)v); }
+__device__ __forceinline__ void store_coherent_i32(int32_t* p, int32_t v) {
+    store_coherent_u32((uint32_t*)p, (uint32_t)v);
+}
 
 // ---- bottom-up refit with SAH treelet refinement ------------------------------------------------------------
 //
@@ -611,7 +615,7 @@ __device__ __forceinline__ void store_coherent_i32(int32_t* p, int32_t v) { stor
 //   DP         over the 127 leaf subsets S in order of size: cost(S) = area(S) + min over splits {P, S\P} of
 //              (cost(P) + cost(S\P)), P containing the lowest leaf of S; ties go to the smallest P
 //   rebuild    only on a strict cost decrease and when the treelet height does not grow (so the whole tree
-//              keeps the depth bound the collapse relies on): breadth-first from S = all leaves, internal
+//              keeps the radix tree's depth bound): breadth-first from S = all leaves, internal
 //              nodes reused in formation order.
 // A treelet covers only nodes of its root's finished subtree and is processed after that subtree is final, so
 // the result does not depend on the order in which waves finish.
@@ -959,9 +963,9 @@ __device__ __forceinline__ void treelet_optimize(TreeletLds& T, const SplitRegs&
 //
 // A maximal subtree of at most kSubtree primitives as one wave holds it: internal nodes 0 .. nint - 1 breadth-first
 // from the root, primitives at kSubtree + 0 .. (local ids), each with its code in the binary tree.
-// 112: 9.6 KB of LDS, so that 16 waves share a CU, the four per SIMD that 128 registers allow; the two passes over 15.5M
-// triangles of 64 meshes take 11.0 + 2.5 ms (subtrees + the nodes above), with 96 primitives 11.1 + 3.0 ms, with 128
-// 14.8 + 2.2 ms.
+// 112: 9.6 KB of LDS, so that 16 waves share a CU, the four per SIMD that 128 registers allow.  The two rounds over 15.5M
+// triangles of 64 meshes take 9.5 + 2.4 ms (subtrees + the nodes above); when they took 11.0 + 2.5, it was 11.1 + 3.0
+// with 96 primitives and 14.8 + 2.2 with 128.
 constexpr uint32_t kSubtree = 112;
 struct SubtreeLds {
     int32_t code[2 * kSubtree];
@@ -1089,8 +1093,8 @@ struct RefineArgs {
 
 // Refit and refinement of the listed subtrees, one wave each.  A pass whose every node went through global memory
 // (agent-scope loads that miss the L2, about 16 dependent ones per treelet) took 18.0 and 12.3 ms for the two rounds on
-// 15.5M triangles, 4.4 ms for the first one on 4M; here the links and boxes of a subtree are read once.  What bounds it now:
-// the instructions of the treelets (about 600 VALU and 450 SALU each) at four waves per SIMD.
+// 15.5M triangles, 4.4 ms for the first one on 4M; here the links and boxes of a subtree are read once.  What bounds it
+// now: the instructions of the treelets (about 600 VALU and 450 SALU each) at four waves per SIMD.
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void subtree_refine_kernel(RefineArgs a) {
     __shared__ SubtreeLds U;
     __shared__ float ubox[2 * kSubtree][6];
@@ -1224,7 +1228,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void su
 
 // Treelet refinement rounds: default kTreeletRounds, none under PREFER_FAST_BUILD, RTX_BUILD_TREELET_ROUNDS_*
 // overrides both, NO_TREELET disables; round r restructures nodes with at least kTreeletMinPrims[r] primitives.
-// (Each round costs ~17 ms on 20M triangles and buys 0.5-1.5% of closest-hit speed on the query scenes.)
+// (The two rounds take 12 ms on 15.5M triangles; each buys 0.5-1.5% of closest-hit speed on the query scenes.)
 constexpr int kTreeletRounds = 2;
 constexpr uint32_t kTreeletMinPrims[3] = {7, 14, 28};
 int treelet_rounds(uint32_t flags, uint32_t n) {
@@ -1565,7 +1569,9 @@ struct CollapseQueue {
     uint32_t subs, pad3[31];
 };
 static_assert(sizeof(CollapseQueue) == 512, "the scratch layout's queue words");
-__device__ __forceinline__ uint64_t pack_task(int32_t node, uint32_t slot) { return (uint32_t)node | (uint64_t)slot << 32; }
+__device__ __forceinline__ uint64_t pack_task(int32_t node, uint32_t slot) {
+    return (uint32_t)node | (uint64_t)slot << 32;
+}
 
 // Root of a structure (header fields set, slot 0): its subtree task or its queue task, and what the header says of it.
 __device__ void push_root(AsHeader* h, int32_t root, uint32_t blas, const uint32_t* cnt, const uint32_t* sub,
@@ -1849,7 +1855,8 @@ __device__ __forceinline__ void write_node(WideLds& W, bool on, uint4* slots, ui
     __syncthreads();
 }
 
-__device__ __forceinline__ void copy_leaf(uint4* slots, uint32_t slot, const uint4* __restrict__ leaf_src, uint32_t prim) {
+__device__ __forceinline__ void copy_leaf(uint4* slots, uint32_t slot, const uint4* __restrict__ leaf_src,
+                                          uint32_t prim) {
     const uint4* src = leaf_src + 4 * (uint64_t)prim;
     uint4* dst = slots + 4 * (uint64_t)slot;
     const uint4 w0 = src[0], w1 = src[1], w2 = src[2], w3 = src[3];
@@ -2624,7 +2631,8 @@ hipError_t update_blas(const GeomDesc* geoms_host, uint32_t ngeom, uint32_t n, u
         if ((err = hipMemcpyAsync(sc + L.parent, u + 4ull * (3 * n - 2), 4ull * (2 * n - 1),
                                   hipMemcpyDeviceToDevice, s)))
             return err;
-        refit_passes(n, flags | RTX_BUILD_NO_TREELET_BIT, sc, L, (const float*)(sc + L.boxes), s, nullptr, kLeafCostTri, false);
+        refit_passes(n, flags | RTX_BUILD_NO_TREELET_BIT, sc, L, (const float*)(sc + L.boxes), s, nullptr,
+                     kLeafCostTri, false);
     }
     header_kernel<<<1, 64, 0, s>>>(h, 0, flags, n, ngeom, (const float*)(sc + L.nboxes), (const float*)(sc + L.cost),
                                    2ull * (n ? n : 1) + 1, 0, (const uint32_t*)(sc + L.cnt),
@@ -2648,9 +2656,9 @@ hipError_t build_tlas(const rtx_instance* inst, uint32_t n, uint32_t flags, void
     uint32_t* maxd = (uint32_t*)(sc + L.misc);
     init_build_kernel<<<1, 256, 0, s>>>(cb, maxd);  // misc words 0, 1: deepest BLAS, content bits
     if (n > 0)
-        prep_instances_kernel<<<std::min((n + 3) / 4, 2048u), 256, 0, s>>>(inst, n, (InstSlot*)(sc + L.leaves),
-                                                              (InstanceInfo*)((uint8_t*)dst + table_offset),
-                                                              (float*)(sc + L.boxes), cb, maxd, maxd + 1);
+        prep_instances_kernel<<<std::min((n + 3) / 4, 2048u), 256, 0, s>>>(
+            inst, n, (InstSlot*)(sc + L.leaves), (InstanceInfo*)((uint8_t*)dst + table_offset),
+            (float*)(sc + L.boxes), cb, maxd, maxd + 1);
     hipError_t err;
     if ((err = lbvh_common(n, k64, 1, flags, 0, sc, L, (uint8_t*)dst, table_offset, err_flags, s))) return err;
     finish_tlas_kernel<<<1, 64, 0, s>>>((AsHeader*)dst, maxd);

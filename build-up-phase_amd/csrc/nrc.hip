@@ -248,11 +248,9 @@ __device__ __forceinline__ void layer_forward2(const bf16x8* frag, const f32x4* 
     }
 }
 
-__global__ __launch_bounds__(kInferThreads) __attribute__((amdgpu_waves_per_eu(6))) void nrc_infer_lds_kernel(const bf16x8* __restrict__ fwd,
-                                                            const float* __restrict__ params,
-                                                            const rtx_nrc_query* __restrict__ queries, uint32_t n,
-                                                            const uint32_t* __restrict__ n_dev, Norm nm,
-                                                            float* __restrict__ out_rgb, InferGather gt) {
+__global__ __launch_bounds__(kInferThreads) __attribute__((amdgpu_waves_per_eu(6))) void nrc_infer_lds_kernel(
+    const bf16x8* __restrict__ fwd, const float* __restrict__ params, const rtx_nrc_query* __restrict__ queries,
+    uint32_t n, const uint32_t* __restrict__ n_dev, Norm nm, float* __restrict__ out_rgb, InferGather gt) {
     __shared__ bf16x8 frag[kInferLdsFrags];
     for (int i = threadIdx.x; i < kInferLdsFrags; i += blockDim.x) frag[i] = fwd[i];
     __shared__ f32x4 bias[(5 * 64 + 16) / 4];  // layer L's at 16 L
@@ -432,11 +430,10 @@ __device__ __forceinline__ void store_grad(const f32x4* gv, int tiles, __bf16* g
 }
 
 constexpr int kTrainThreads = 512;
-__global__ __launch_bounds__(kTrainThreads) void nrc_train_kernel(const bf16x8* __restrict__ fwd, const bf16x8* __restrict__ bwd,
-                                                        const float* __restrict__ params,
-                                                        const rtx_nrc_sample* __restrict__ samples, StepShape shape,
-                                                        Norm nm, float* __restrict__ partials,
-                                                        float* __restrict__ loss_part, uint32_t* __restrict__ steps) {
+__global__ __launch_bounds__(kTrainThreads) void nrc_train_kernel(
+    const bf16x8* __restrict__ fwd, const bf16x8* __restrict__ bwd, const float* __restrict__ params,
+    const rtx_nrc_sample* __restrict__ samples, StepShape shape, Norm nm, float* __restrict__ partials,
+    float* __restrict__ loss_part, uint32_t* __restrict__ steps) {
     __shared__ TrainLds sm;
     uint32_t n, stride, offset;
     // a step that does not run, and blocks past the step's samples, leave at once (the whole block alike)
@@ -704,8 +701,8 @@ hipError_t nrc_infer(const NrcState& st, const rtx_nrc_query* q, uint32_t n, flo
     const uint64_t pairs = ((uint64_t)n + 31) / 32;
     const uint64_t want = (pairs + kInferThreads / 64 - 1) / (kInferThreads / 64);
     const unsigned blocks = (unsigned)std::min<uint64_t>(want, (uint64_t)st.cu_count * 3);
-    nrc_infer_lds_kernel<<<blocks, kInferThreads, 0, s>>>((const bf16x8*)st.fwd, st.params, q, n, n_dev, make_norm(st), out,
-                                                 gather ? *gather : InferGather{});
+    nrc_infer_lds_kernel<<<blocks, kInferThreads, 0, s>>>((const bf16x8*)st.fwd, st.params, q, n, n_dev,
+                                                          make_norm(st), out, gather ? *gather : InferGather{});
     return hipGetLastError();
 }
 
@@ -713,9 +710,9 @@ hipError_t nrc_infer(const NrcState& st, const rtx_nrc_query* q, uint32_t n, flo
 static hipError_t launch_step(NrcState& st, const rtx_nrc_sample* samples, const StepShape& shape, uint32_t nblk,
                               float* grad_out, float* loss_out, hipStream_t s) {
     float* loss = loss_out ? loss_out : st.loss;
-    nrc_train_kernel<<<nblk, kTrainThreads, 0, s>>>((const bf16x8*)st.fwd, (const bf16x8*)st.bwd, st.params, samples, shape,
-                                          make_norm(st), st.partials, st.loss_part,
-                                          grad_out ? nullptr : st.steps_dev);
+    nrc_train_kernel<<<nblk, kTrainThreads, 0, s>>>((const bf16x8*)st.fwd, (const bf16x8*)st.bwd, st.params, samples,
+                                                    shape, make_norm(st), st.partials, st.loss_part,
+                                                    grad_out ? nullptr : st.steps_dev);
     // the parameters' blocks + the loss block
     const unsigned pb = (RTX_NRC_PARAM_COUNT + kAdamParams - 1) / kAdamParams + 1;
     if (grad_out) {

@@ -17,8 +17,10 @@ namespace rtx {
 namespace {
 
 constexpr int kSortBlock = 256;
-// Keys per thread: 16 (4,096-key tiles); below kLargeFrom keys 4 (1,024-key tiles), so that more blocks share a pass
-// (655K keys: 20 us a pass with 16, 27 us with 4, whose look-back goes over four times the tiles).
+// Keys per thread: 16 (4,096-key tiles); below kLargeFrom keys 4 (1,024-key tiles), so that more blocks share a pass.
+// A pass with 4 and with 16: 32,768 keys 8.2 and 13 us, 65,536 9.6 and 13.5, 131,072 11.6 and 14.4, 262,144 15.1 and
+// 15.7, 655K 28 and 20 (the look-back of small tiles goes over four times as many).  They cross near 270,000 keys; the
+// line below gives away at most 3 us a pass between.
 constexpr int kItemsLarge = 16, kItemsSmall = 4;
 constexpr uint32_t kLargeFrom = 1u << 17;
 constexpr uint32_t kOneBlock = kSortBlock * kItemsLarge;

@@ -59,7 +59,7 @@ struct TraceLaunch {
     uint32_t refill_lanes;     // refill a wave once fewer lanes than this are busy (1..64)
     uint32_t refill_interval;  // traversal steps between refill checks (1..64)
     uint32_t leaf_lanes;       // pending leaf groups in a wave before the leaf step runs (1..64)
-    uint32_t waves;            // VGPR-bounded kernel variant: 0 (unbounded), 4 (128 VGPRs) or 5 (96 VGPRs) waves per SIMD
+    uint32_t waves;            // VGPR-bounded kernel variant: 0 (unbounded), 4 (128) or 5 (96 VGPRs) waves per SIMD
     uint32_t beside;           // 1: runs beside another launch, which holds part of the chip when this one starts
 };
 

@@ -104,10 +104,6 @@ __device__ __forceinline__ float safe_rcp(float d) {
     return __builtin_amdgcn_rcpf(a * 0x1p-32f) * 0x1p-32f;
 }
 
-__device__ __forceinline__ float byte_f(uint32_t w, int b) {
-    return (float)((w >> (8 * b)) & 255u);
-}
-
 struct Space {
     float ox, oy, oz;
     float dx, dy, dz;
@@ -673,12 +669,12 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
         tc = r.tmax;
     };
 
-    // Wave-uniform pool of ray ids [pool_next, pool_end).  Chunk w of the launch is wave w's first pool, for the first
-    // first_waves waves; the chunks after those come from kRayQueues counters, each shared by the blocks of one residue:
-    // queue q's c-th chunk is one of the c-th group of nq chunks, at a place rotated by a hash of c (with a fixed place,
-    // a film whose rows hold a multiple of nq / 2 chunks gives every queue its own columns: 20% slower).  An atomic on
-    // one word shared by all waves costs 10-20 ns in turn, so one counter bounded short launches by its 4,096 waves'
-    // fetches alone: 777 rays 96 us, the 1200x800 reference film 224 us.
+    // Wave-uniform pool of ray ids [pool_next, pool_end).  Chunk w of the launch is wave w's first pool, for the
+    // first first_waves waves; the chunks after those come from kRayQueues counters, each shared by the blocks of one
+    // residue: queue q's c-th chunk is one of the c-th group of nq chunks, at a place rotated by a hash of c (with a
+    // fixed place, a film whose rows hold a multiple of nq / 2 chunks gives every queue its own columns: 20% slower).
+    // An atomic on one word shared by all waves costs 10-20 ns in turn, so one counter bounded short launches by its
+    // 4,096 waves' fetches alone: 777 rays 96 us, the 1200x800 reference film 224 us.
     const uint32_t waves_block = blockDim.x >> 6;
     const uint32_t waves_total = gridDim.x * waves_block;
     const uint32_t wave =
@@ -1484,7 +1480,8 @@ hipError_t trace_rays_launch(const TraceRequest& r, const TraceLaunch& L, hipStr
         sh.blocks_per_cu = L.blocks_per_cu;
         sh.grid = L.grid;
         sh.waves_per_simd = L.waves >= 5u ? 5u : (L.waves == 4u ? 4u : 3u);
-        sh.lane_bytes = L.lds_depth * (uint32_t)sizeof(uint2) + (flags || r.mode >= 3 ? 6u * (uint32_t)sizeof(float) : 0u);
+        const bool rays = flags || r.mode >= 3;  // as kRayLds in the kernel
+        sh.lane_bytes = L.lds_depth * (uint32_t)sizeof(uint2) + (rays ? 6u * (uint32_t)sizeof(float) : 0u);
         sh.beside = L.beside != 0;
         const TracePlan p = plan_trace(sh, L.ray_chunk, r.n_ptr ? 0u : r.n, r.mode >= 5);
         a.first_waves = p.first_waves;

@@ -48,12 +48,15 @@ RTX_RULE uint32_t resident_blocks(const TraceShape& s, uint32_t lds_bytes) {
 
 // Ray ids per chunk of a launch of n rays on `waves` waves, of which first_waves own their first chunk.  Automatic: at
 // most one ray per lane of those is spread over all of them (a wave of few rays diverges less, and the launch lasts as
-// long as its slowest wave); otherwise 64, or for single rays 256 when every wave gets at least 8 chunks (16.7M camera or
-// incoherent rays 1.3% faster than with 64, 3M any-hit rays 1% slower; whole paths are too uneven for that: 4 samples
-// of the 1080p Cornell box 13.6 ms with 256, 13.0 ms with 64).
+// long as its slowest wave); otherwise 64, or for single rays 256 when every wave gets at least 8 chunks.  Fetches count
+// where rays are cheap: a 7680x4320 film of two quads 437 us with 64, 391 us with 256, 16.7M rays that all miss 239 and
+// 218 us; where they are not, 256 is even (16.7M rays over 20M triangles) or up to 3% slower (3M to 16M any-hit rays
+// 1%, camera rays that all enter small meshes 865 and 893 us).  Whole paths are too uneven for that: 4 samples of the
+// 1080p Cornell box 13.6 ms with 256, 13.0 ms with 64.
 RTX_RULE uint32_t rays_per_chunk(uint32_t configured, uint32_t n, uint32_t waves, uint32_t first_waves, bool paths) {
     if (configured >= 64u) return configured;
-    if (first_waves && (uint64_t)n <= (uint64_t)first_waves * 64u) return n ? (n + first_waves - 1u) / first_waves : 1u;
+    if (first_waves && (uint64_t)n <= (uint64_t)first_waves * 64u)
+        return n ? (n + first_waves - 1u) / first_waves : 1u;
     return !paths && (uint64_t)n >= (uint64_t)waves * 64u * 8u ? 256u : 64u;
 }
 
@@ -66,15 +69,15 @@ struct TracePlan {
 };
 
 // The plan of a launch of n rays (0: the count is on the device).
-//   lean         where the table and the tasks would cost a CU a block, and for five waves per SIMD, whose shapes fill the
-//                LDS with their stacks.  With both in all launches 720p path tracing took 10.1 ms on 20 blocks of one
-//                wave per CU (12 or 13 of them fitted) and 7.9 ms on 16 with 16 stack entries each; lean 7.2 and
+//   lean         where the table and the tasks would cost a CU a block, and for five waves per SIMD, whose shapes fill
+//                the LDS with their stacks.  With both in all launches 720p path tracing took 10.1 ms on 20 blocks of
+//                one wave per CU (12 or 13 of them fitted) and 7.9 ms on 16 with 16 stack entries each; lean 7.2 and
 //                6.3 ms.  Where they fit (256 x 4), the table's byte read instead of 16 vector instructions per node
 //                step and the tasks through LDS instead of five permutes are 2% and 1% faster
-//   first_waves  only waves that start at once own rays.  The blocks beyond start as others retire, when the queues have
-//                run dry, and would only then begin with theirs: on 32 blocks of 256 per CU, of which 4 or 5 start, 4M
-//                incoherent rays took 1.83 ms and 720p path tracing 9.3 ms, now 1.22 and 7.2 ms.  None where the chip is
-//                shared: which blocks start at once is not known then
+//   first_waves  only waves that start at once own rays.  The blocks beyond start as others retire, when the queues
+//                have run dry, and would only then begin with theirs: on 32 blocks of 256 per CU, of which 4 or 5
+//                start, 4M incoherent rays took 1.83 ms and 720p path tracing 9.3 ms, now 1.22 and 7.2 ms.  None where
+//                the chip is shared: which blocks start at once is not known then
 //   grid         no more waves than rays
 RTX_RULE TracePlan plan_trace(const TraceShape& s, uint32_t ray_chunk, uint32_t n, bool paths) {
     TracePlan p;
@@ -88,7 +91,8 @@ RTX_RULE TracePlan plan_trace(const TraceShape& s, uint32_t ray_chunk, uint32_t 
     if (n && !s.beside && ray_chunk < 64u && (n - 1u) / waves_block < p.grid) p.grid = (n - 1u) / waves_block + 1u;
     const uint32_t at_once = s.grid / s.blocks_per_cu * resident;
     p.first_waves = s.beside ? 0u : (at_once < p.grid ? at_once : p.grid) * waves_block;
-    p.queues = !n || (uint64_t)rays_per_chunk(ray_chunk, n, p.grid * waves_block, p.first_waves, paths) * p.first_waves < n;
+    const uint64_t chunk = rays_per_chunk(ray_chunk, n, p.grid * waves_block, p.first_waves, paths);
+    p.queues = !n || chunk * p.first_waves < n;
     return p;
 }
 

@@ -54,7 +54,7 @@ typedef enum rtx_result {
     RTX_ERROR_OUT_OF_HOST_MEMORY = -1,      /* VK_ERROR_OUT_OF_HOST_MEMORY */
     RTX_ERROR_OUT_OF_DEVICE_MEMORY = -2,    /* VK_ERROR_OUT_OF_DEVICE_MEMORY: storage/scratch below the size query */
     RTX_ERROR_INITIALIZATION_FAILED = -3,   /* VK_ERROR_INITIALIZATION_FAILED */
-    RTX_ERROR_DEVICE_LOST = -4,             /* VK_ERROR_DEVICE_LOST: a HIP call failed, or a wait on the device ran out */
+    RTX_ERROR_DEVICE_LOST = -4,             /* VK_ERROR_DEVICE_LOST: a HIP call failed or a device wait ran out */
     RTX_ERROR_INVALID_ARGUMENT = -1000,     /* bad pointer, size, count or flag */
     RTX_ERROR_STACK_OVERFLOW = -1001,       /* traversal stack exceeded the built depth bound */
     RTX_ERROR_INVALID_AS = -1002,           /* address is not an acceleration structure of this library */

@@ -76,7 +76,7 @@ namespace {
 constexpr uint32_t kMaxPrims = (1u << 30) - 1u;
 // NRC training paths: the pixel-path launch leaves kSideReserve 256-thread blocks per CU free for them, and their
 // launch has kSideBlocks 256-thread blocks per CU: the blocks beyond the reserve start as pixel-path blocks retire
-// (a launch beside another hands all paths out from the queues, so late blocks only take what is left).
+// (which own no paths, TraceLaunch::start_blocks, and only take what the queues still hold).
 constexpr uint32_t kSideReserve = 1u;
 constexpr uint32_t kSideBlocks = 2u;
 // Samples per whole-path launch of a plain render: up to 16, and at most 2^25 paths per launch (the per-path state
@@ -374,7 +374,7 @@ int side_chain(rtx_context ctx, const rtx::TraceLaunch& L, rtx::SideChain& side)
     S.blocks_per_cu = kSideBlocks * 256u / L.block_size > 0 ? kSideBlocks * 256u / L.block_size : 1u;
     S.grid = (uint32_t)ctx->cu_count * S.blocks_per_cu;
     S.waves = 4;
-    S.beside = 1;
+    S.start_blocks = kSideReserve * 256u / L.block_size > 0 ? kSideReserve * 256u / L.block_size : 1u;
     uint64_t bytes = ctx->side_gstack_entries * sizeof(uint2);
     const uint64_t per_lane = std::max(S.gdepth, unknown_depth_gdepth(ctx, S));
     const int r = grow_buffer(ctx, (void**)&ctx->side_gstack, &bytes,
@@ -404,7 +404,7 @@ rtx::TraceLaunch launch_shape(rtx_context ctx, uint32_t depth) {
     L.leaf_lanes = ctx->cfg.leaf_lanes;
     const uint32_t waves = (L.block_size / 64u) * L.blocks_per_cu / 4u;  // per SIMD
     L.waves = waves >= 5u ? 5u : (waves == 4u ? 4u : 0u);
-    L.beside = 0u;
+    L.start_blocks = L.blocks_per_cu;
     return L;
 }
 

@@ -60,7 +60,7 @@ struct TraceLaunch {
     uint32_t refill_interval;  // traversal steps between refill checks (1..64)
     uint32_t leaf_lanes;       // pending leaf groups in a wave before the leaf step runs (1..64)
     uint32_t waves;            // VGPR-bounded kernel variant: 0 (unbounded), 4 (128) or 5 (96 VGPRs) waves per SIMD
-    uint32_t beside;           // 1: runs beside another launch, which holds part of the chip when this one starts
+    uint32_t start_blocks;     // blocks per CU that can start at once beside what runs already
 };
 
 hipError_t trace_rays_launch(const TraceRequest& req, const TraceLaunch& launch, hipStream_t stream);

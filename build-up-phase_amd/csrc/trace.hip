@@ -1482,7 +1482,7 @@ hipError_t trace_rays_launch(const TraceRequest& r, const TraceLaunch& L, hipStr
         sh.waves_per_simd = L.waves >= 5u ? 5u : (L.waves == 4u ? 4u : 3u);
         const bool rays = flags || r.mode >= 3;  // as kRayLds in the kernel
         sh.lane_bytes = L.lds_depth * (uint32_t)sizeof(uint2) + (rays ? 6u * (uint32_t)sizeof(float) : 0u);
-        sh.beside = L.beside != 0;
+        sh.start_blocks = L.start_blocks;
         const TracePlan p = plan_trace(sh, L.ray_chunk, r.n_ptr ? 0u : r.n, r.mode >= 5);
         a.first_waves = p.first_waves;
         a.guard = both ? g : (r.guard == 1u || r.guard == 2u ? r.guard : 0u);

@@ -34,7 +34,7 @@ struct TraceShape {
     uint32_t grid;            // blocks: blocks_per_cu on every CU
     uint32_t waves_per_simd;  // that the kernel variant's registers allow at least
     uint32_t lane_bytes;      // LDS of a lane: its stack entries, and its world ray where the kernel keeps it there
-    bool beside;              // another launch holds part of the chip when this one starts
+    uint32_t start_blocks;    // blocks of a CU that can start at once beside what runs already
 };
 
 // Blocks of a launch that a CU holds at once.
@@ -76,8 +76,7 @@ struct TracePlan {
 //                step and the tasks through LDS instead of five permutes are 2% and 1% faster
 //   first_waves  only waves that start at once own rays.  The blocks beyond start as others retire, when the queues
 //                have run dry, and would only then begin with theirs: on 32 blocks of 256 per CU, of which 4 or 5
-//                start, 4M incoherent rays took 1.83 ms and 720p path tracing 9.3 ms, now 1.22 and 7.2 ms.  None where
-//                the chip is shared: which blocks start at once is not known then
+//                start, 4M incoherent rays took 1.83 ms and 720p path tracing 9.3 ms, now 1.22 and 7.2 ms
 //   grid         no more waves than rays
 RTX_RULE TracePlan plan_trace(const TraceShape& s, uint32_t ray_chunk, uint32_t n, bool paths) {
     TracePlan p;
@@ -88,9 +87,10 @@ RTX_RULE TracePlan plan_trace(const TraceShape& s, uint32_t ray_chunk, uint32_t 
     p.lean = s.waves_per_simd >= 5u || resident_blocks(s, p.lds + tasks + kOctTableBytes) < resident;
     if (!p.lean) p.lds += tasks;
     p.grid = s.grid;
-    if (n && !s.beside && ray_chunk < 64u && (n - 1u) / waves_block < p.grid) p.grid = (n - 1u) / waves_block + 1u;
+    if (n && ray_chunk < 64u && (n - 1u) / waves_block < p.grid) p.grid = (n - 1u) / waves_block + 1u;
+    if (s.start_blocks < resident) resident = s.start_blocks;
     const uint32_t at_once = s.grid / s.blocks_per_cu * resident;
-    p.first_waves = s.beside ? 0u : (at_once < p.grid ? at_once : p.grid) * waves_block;
+    p.first_waves = (at_once < p.grid ? at_once : p.grid) * waves_block;
     const uint64_t chunk = rays_per_chunk(ray_chunk, n, p.grid * waves_block, p.first_waves, paths);
     p.queues = !n || chunk * p.first_waves < n;
     return p;

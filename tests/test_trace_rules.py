@@ -15,9 +15,9 @@ SOURCE = r"""
 extern "C" {
 int pops_entry(uint32_t sp, uint32_t entries) { return rtx::pops_entry(sp, entries); }
 // out: grid, lds, first_waves, lean, queues, resident blocks per CU, rays per chunk
-void plan(uint32_t block, uint32_t per_cu, uint32_t cus, uint32_t simd, uint32_t lane_bytes, uint32_t beside,
+void plan(uint32_t block, uint32_t per_cu, uint32_t cus, uint32_t simd, uint32_t lane_bytes, uint32_t start,
           uint32_t chunk, uint32_t n, uint32_t paths, uint32_t* out) {
-    const rtx::TraceShape s = {block, per_cu, cus * per_cu, simd, lane_bytes, beside != 0};
+    const rtx::TraceShape s = {block, per_cu, cus * per_cu, simd, lane_bytes, start};
     const rtx::TracePlan p = rtx::plan_trace(s, chunk, n, paths != 0);
     const uint32_t fixed = p.lean ? 0u : rtx::kOctTableBytes;
     const uint32_t v[] = {p.grid, p.lds, p.first_waves, p.lean, p.queues, rtx::resident_blocks(s, p.lds + fixed),
@@ -38,11 +38,11 @@ def rules(tmp_path_factory):
     return ctypes.CDLL(str(lib))
 
 
-def _plan(rules, block, per_cu, cus=256, depth=12, ray=True, beside=False, chunk=1, n=0, paths=False):
+def _plan(rules, block, per_cu, cus=256, depth=12, ray=True, start=None, chunk=1, n=0, paths=False):
     waves = block // 64 * per_cu // 4
     out = (ctypes.c_uint32 * 7)()
     rules.plan(block, per_cu, cus, 5 if waves >= 5 else 4 if waves == 4 else 3, 8 * depth + (24 if ray else 0),
-               int(beside), chunk, n, int(paths), out)
+               per_cu if start is None else start, chunk, n, int(paths), out)
     return dict(zip(("grid", "lds", "first_waves", "lean", "queues", "resident", "chunk"), out))
 
 
@@ -73,8 +73,9 @@ def test_the_tables_and_tasks_take_no_block_from_a_cu(rules):
 @pytest.mark.parametrize("chunk", [1, 64, 128, 4096])
 @pytest.mark.parametrize("shape", [(64, 1), (64, 13), (64, 20), (64, 32), (128, 10), (192, 3), (256, 4), (256, 5), (256, 32)])
 def test_first_chunks_belong_to_waves_that_start_at_once(rules, shape, chunk):
-    """Waves own a first chunk only among the blocks that the chip holds at once, and not beside another launch; the
-    first chunks and the queues' chunks cover the rays, and the queues are used exactly where rays are left for them."""
+    """Waves own a first chunk only among the blocks that start at once, by what the chip holds and beside what runs
+    already; the first chunks and the queues' chunks cover the rays, and the queues are used exactly where rays are left
+    for them."""
     block, per_cu = shape
     cus, wb = 4, block // 64
     for ray in (False, True):
@@ -86,8 +87,10 @@ def test_first_chunks_belong_to_waves_that_start_at_once(rules, shape, chunk):
                 assert p["first_waves"] <= full["resident"] * cus * wb, (n, p)
                 assert 1 <= p["grid"] <= cus * per_cu and p["first_waves"] <= p["grid"] * wb
                 assert p["chunk"] >= 1 and bool(p["queues"]) == (p["chunk"] * p["first_waves"] < n)
-                b = _plan(rules, block, per_cu, cus, ray=ray, chunk=chunk, n=n, paths=paths, beside=True)
-                assert b["first_waves"] == 0 and b["queues"] and b["grid"] == cus * per_cu
+                for start in (0, 1, per_cu // 2):
+                    b = _plan(rules, block, per_cu, cus, ray=ray, chunk=chunk, n=n, paths=paths, start=start)
+                    assert b["first_waves"] == min(min(start, full["resident"]) * cus, b["grid"]) * wb
+                    assert bool(b["queues"]) == (b["chunk"] * b["first_waves"] < n) and b["lds"] == p["lds"]
         d = _plan(rules, block, per_cu, cus, ray=ray, chunk=chunk, n=0)  # a count that only the device knows
         assert d["queues"] and d["grid"] == cus * per_cu
 

@@ -548,11 +548,11 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
     constexpr bool kTrain = MODE == kModeTrain || MODE == kModePixelPaths || MODE == kModePixelCache;  // whole paths
     constexpr int kShadeMode = MODE == kModePixelPaths ? (int)kPtPlain : (int)kPtCache;
     constexpr bool kRayLds = FLAGS || MODE == kModePath || MODE == kModeFused || kTrain;
-    // the triangle tasks of the block's waves (32 of 16 B each), the stack, the rays
-    extern __shared__ __attribute__((aligned(16))) uint2 lds_words[];
-    uint2* const lds_stack = lds_words + (LEAN ? 0u : blockDim.x);
+    // the stack, the rays, the triangle tasks of the block's waves (32 of 16 B each)
+    extern __shared__ __attribute__((aligned(16))) uint2 lds_stack[];
     __attribute__((address_space(3))) Words4* const tasks =
-        (__attribute__((address_space(3))) Words4*)lds_words + 32u * (threadIdx.x >> 6);
+        (__attribute__((address_space(3))) Words4*)(lds_stack + (args.lds_depth + (kRayLds ? 3u : 0u)) * blockDim.x) +
+        32u * (threadIdx.x >> 6);
     __shared__ OctTable oct_lds;
     if (!LEAN) {
         for (uint32_t i = threadIdx.x; i < sizeof(OctTable) / 8u; i += blockDim.x)
@@ -1047,6 +1047,7 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
                         fault = kErrBadAs;
                         slot0 = slot1 = kNoSlot;
                     }
+                    if (!LEAN) tasks[rank] = Words4{slot0, slot1, lane, 0u};
                 }
                 const uint32_t ntri = 2u * (uint32_t)__popcll(tri_lanes);
                 uint32_t from = lane, slot = kNoSlot;
@@ -1064,7 +1065,6 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
                         from = whose;
                     }
                 } else {
-                    if (owner) tasks[rank] = Words4{slot0, slot1, lane, 0u};
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                     if (lane < ntri) {
                         const Words4 w = tasks[lane >> 1];
@@ -1132,7 +1132,7 @@ __device__ __forceinline__ void trace_body(const TraceArgs& args) {
                 }
                 const uint64_t hits = __builtin_amdgcn_ballot_w64(cand);
                 if (hits) {
-                    uint32_t t0 = 0, t1 = 0;  // the owner's two distances
+                    uint32_t t0, t1;  // the owner's two distances
                     if (LEAN) {
                         t0 = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(rank << 3), (int)__float_as_uint(th));
                         t1 = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(rank << 3) + 4, (int)__float_as_uint(th));

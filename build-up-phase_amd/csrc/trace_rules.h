@@ -17,7 +17,7 @@ RTX_RULE bool pops_entry(uint32_t sp, uint32_t entries) { return sp - 1u < entri
 
 // ---- launches ---------------------------------------------------------------------------------------------------
 
-// A CU's LDS, and the unit it is given out in (a block of 9,728 B takes 8 units of 16 blocks' 128).
+// A CU's LDS, and the unit it is given out in: 128 of them, so that 16 blocks of up to 10,240 B fit.
 constexpr uint32_t kCuLdsBytes = 160u * 1024u;
 constexpr uint32_t kLdsUnit = 1280u;
 constexpr uint32_t kCuSimds = 4;
